@@ -138,17 +138,15 @@ __device__ __forceinline__ void pair_f32_d(double sx, double sy, double sz, floa
 }
 
 // ---------------------------------------------------------------------------
-// FP64 pair (correctness mode): the reference's formula in double.
+// FP64 pairs (correctness mode, central bodies).
 // ---------------------------------------------------------------------------
-template <bool POT>
-__device__ __forceinline__ void pair_f64(double sx, double sy, double sz, double sm, double xi,
-                                         double yi, double zi, double h, double hinv, double hinv3,
-                                         double &ax, double &ay, double &az, double &aq) {
-    double dx = sx - xi, dy = sy - yi, dz = sz - zi;
-    double r2 = dx * dx + dy * dy + dz * dz;
+// The reference's formula in double, pair by pair: fac and q of a separation.
+__device__ __forceinline__ void terms_f64(double dx, double dy, double dz, double sm, double h, double hinv,
+                                          double hinv3, double &fac, double &q) {
+    const double r2 = dx * dx + dy * dy + dz * dz;
+    fac = q = 0.0;
     if (r2 == 0.0) return;  // self pair / coincident: 0 for h > 0 (NaN in the reference for h == 0)
-    double r = __builtin_sqrt(r2);
-    double fac, q;
+    const double r = __builtin_sqrt(r2);
     if (r >= h) {
         fac = sm / (r2 * r);
         q = sm / r;
@@ -165,10 +163,67 @@ __device__ __forceinline__ void pair_f64(double sx, double sy, double sz, double
                   (-NB_P5 + NB_C6 / u + u2 * (NB_C1 + u * (-NB_P6 + u * (NB_P4 - NB_P7 * u)))));
         }
     }
+}
+
+template <bool POT>
+__device__ __forceinline__ void pair_f64(double sx, double sy, double sz, double sm, double xi,
+                                         double yi, double zi, double h, double hinv, double hinv3,
+                                         double &ax, double &ay, double &az, double &aq) {
+    const double dx = sx - xi, dy = sy - yi, dz = sz - zi;
+    double fac, q;
+    terms_f64(dx, dy, dz, sm, h, hinv, hinv3, fac, q);
     ax += dx * fac;
     ay += dy * fac;
     az += dz * fac;
     if (POT) aq += q;
+}
+
+// The Newtonian terms of an FP64 pair without a square root or a divide:
+// y = v_rsq_f64(r2) (relative error up to about 2^-23), t = y^2 and e = 1 - r2 t
+// in one FMA give
+//   r^-3 = y t (1 - e)^(-3/2) = y t (1 + e (3/2 + 15/8 e)) + O(e^3),
+//   r^-1 = y (1 - e)^(-1/2)   = y (1 + e (1/2 + 3/8 e)) + O(e^3),
+// with e^3 below 2^-64.  The rounding of t enters e and y t with opposite
+// signs, so the factor carries the two or three half-ulp roundings that
+// sqrt, r2 r and the divide had.  r2_pair adds F64_TINY inside the FMA
+// chain (no operation of its own): a self pair then has a finite factor times
+// a zero separation, and any r2 above 2^54 F64_TINY is unchanged.
+// fast_f64 tells the pairs this holds for: r2 above h^2 (and above 1e-140) and
+// below about 1e300, decided on the high dword by one unsigned subtraction
+// and compare; all others (softened, self, overflowing, NaN) take terms_f64.
+#define NB_F64_TINY 1.0e-160
+#define NB_F64_MIN_R2 1.0e-140
+__device__ __forceinline__ double r2_pair(double dx, double dy, double dz) {
+    return __builtin_fma(dx, dx, __builtin_fma(dy, dy, __builtin_fma(dz, dz, NB_F64_TINY)));
+}
+
+__device__ __forceinline__ unsigned hi_dword(double v) {
+    return (unsigned)(__builtin_bit_cast(unsigned long long, v) >> 32);
+}
+
+// The window of high dwords of the fast pairs of a target with softening h.
+__device__ __forceinline__ void fast_f64_window(double h, unsigned &first, unsigned &count) {
+    const double h2 = h * h;
+    const unsigned b = hi_dword(!(h2 <= NB_F64_MIN_R2) ? h2 : NB_F64_MIN_R2);   // (a NaN h has no fast pairs)
+    const unsigned end = 0x7e300000u;                                           // about 1.5e300
+    first = b + 1u;
+    count = first < end ? end - first : 0u;
+}
+__device__ __forceinline__ bool fast_f64(double r2, unsigned first, unsigned count) {
+    return hi_dword(r2) - first < count;
+}
+
+template <bool POT>
+__device__ __forceinline__ void newton_f64(double r2, double sm, double &fac, double &q) {
+    const double y = __builtin_amdgcn_rsq(r2);
+    const double t = y * y;
+    const double e = __builtin_fma(-r2, t, 1.0);
+    const double s = sm * (y * t);
+    fac = __builtin_fma(s * e, __builtin_fma(e, 1.875, 1.5), s);
+    if (POT) {
+        const double w = sm * y;
+        q = __builtin_fma(w * e, __builtin_fma(e, 0.375, 0.5), w);
+    }
 }
 
 }  // namespace nb

@@ -271,27 +271,60 @@ __global__ __launch_bounds__(BS) void k_force_f64(ForceArgs<double> a, int split
     }
 }
 
-// Sum the per-segment partials in fixed segment order and apply G.
-__global__ void k_finalize(const double *__restrict__ part, int nseg, int64_t n, double G,
-                           double *__restrict__ ax, double *__restrict__ ay,
-                           double *__restrict__ az, double *__restrict__ pot, int with_pot,
-                           int with_acc) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double sx = 0.0, sy = 0.0, sz = 0.0, sq = 0.0;
-    for (int s = 0; s < nseg; ++s) {
-        const double *p = part + (int64_t)s * 4 * n;
-        sx += p[i];
-        sy += p[n + i];
-        sz += p[2 * n + i];
-        if (with_pot) sq += p[3 * n + i];
+// One target's per-segment partial sums, added by the 4 waves of a workgroup:
+// wave w takes the segments w, w + 4, ..., and lane l of wave 0 gets
+// ((w0 + w1) + (w2 + w3)) for target i (the same for all n and grids, so
+// results repeat).  Bound by the latency of the loads where n is small: one
+// thread per target walked up to 64 segments serially on n / 256 workgroups.
+template <bool ACC, bool POT>
+struct PartSums {
+    static constexpr int NV = (ACC ? 3 : 0) + (POT ? 1 : 0);
+    double v[NV];
+};
+template <bool ACC, bool POT>
+__device__ __forceinline__ bool sum_partials(const double *__restrict__ part, int nseg, int64_t n, int64_t i,
+                                             double (&red)[3][PartSums<ACC, POT>::NV][64],
+                                             PartSums<ACC, POT> &r) {
+    constexpr int NV = PartSums<ACC, POT>::NV;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int q = 0; q < NV; ++q) r.v[q] = 0.0;
+    if (i < n) {
+        const double *p = part + (ACC ? 0 : 3) * n + i;
+#pragma unroll 4
+        for (int s = w; s < nseg; s += NW) {
+#pragma unroll
+            for (int q = 0; q < NV; ++q) r.v[q] += p[((int64_t)s * 4 + q) * n];
+        }
     }
-    if (with_acc) {
-        ax[i] = G * sx;
-        ay[i] = G * sy;
-        az[i] = G * sz;
+    if (w > 0) {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) red[w - 1][q][lane] = r.v[q];
     }
-    if (with_pot) pot[i] = -G * sq;
+    __syncthreads();
+    if (w > 0 || i >= n) return false;
+#pragma unroll
+    for (int q = 0; q < NV; ++q) r.v[q] = (r.v[q] + red[0][q][lane]) + (red[1][q][lane] + red[2][q][lane]);
+    return true;
+}
+
+// Sum the per-segment partials in a fixed order and apply G (64 targets per
+// workgroup).  Measured: 59 segments x 30011 potentials 27 -> 5.4 us, 63
+// segments x 16001 forces 21 -> 6.7 us.
+template <bool ACC, bool POT>
+__global__ __launch_bounds__(BS) void k_finalize(const double *__restrict__ part, int nseg, int64_t n, double G,
+                                                 double *__restrict__ ax, double *__restrict__ ay,
+                                                 double *__restrict__ az, double *__restrict__ pot) {
+    __shared__ double red[3][PartSums<ACC, POT>::NV][64];
+    const int64_t i = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
+    PartSums<ACC, POT> r;
+    if (!sum_partials<ACC, POT>(part, nseg, n, i, red, r)) return;
+    if constexpr (ACC) {
+        ax[i] = G * r.v[0];
+        ay[i] = G * r.v[1];
+        az[i] = G * r.v[2];
+    }
+    if constexpr (POT) pot[i] = -G * r.v[PartSums<ACC, POT>::NV - 1];
 }
 
 // Bounding box of each BS-source tile (lo xyz, hi xyz) and, when sub is not
@@ -395,19 +428,15 @@ __global__ __launch_bounds__(BS) void k_drift_boxes(T *__restrict__ x, T *__rest
 // k_finalize followed by the step's kick (Vel += Acc * coef, the operations
 // of k_kick) on the accelerations it has just written.
 template <typename T>
-__global__ void k_finalize_kick(const double *__restrict__ part, int nseg, int64_t n, double G,
-                                double *__restrict__ ax, double *__restrict__ ay, double *__restrict__ az,
-                                T *__restrict__ vx, T *__restrict__ vy, T *__restrict__ vz, double coef) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double sx = 0.0, sy = 0.0, sz = 0.0;
-    for (int s = 0; s < nseg; ++s) {
-        const double *p = part + (int64_t)s * 4 * n;
-        sx += p[i];
-        sy += p[n + i];
-        sz += p[2 * n + i];
-    }
-    const double fx = G * sx, fy = G * sy, fz = G * sz;
+__global__ __launch_bounds__(BS) void k_finalize_kick(const double *__restrict__ part, int nseg, int64_t n,
+                                                      double G, double *__restrict__ ax, double *__restrict__ ay,
+                                                      double *__restrict__ az, T *__restrict__ vx,
+                                                      T *__restrict__ vy, T *__restrict__ vz, double coef) {
+    __shared__ double red[3][3][64];
+    const int64_t i = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
+    PartSums<true, false> r;
+    if (!sum_partials<true, false>(part, nseg, n, i, red, r)) return;
+    const double fx = G * r.v[0], fy = G * r.v[1], fz = G * r.v[2];
     ax[i] = fx;
     ay[i] = fy;
     az[i] = fz;
@@ -607,12 +636,12 @@ int launch_drift_boxes(void *x, void *y, void *z, const void *vx, const void *vy
 int launch_finalize_kick(const double *part, int nseg, int64_t n, double G, double *ax, double *ay, double *az,
                          void *vx, void *vy, void *vz, double coef, int is_double, hipStream_t s) {
     if (n <= 0) return NB_OK;
-    const unsigned nb = (unsigned)((n + 255) / 256);
+    const unsigned nb = (unsigned)((n + 63) / 64);
     if (is_double)
-        k_finalize_kick<double><<<nb, 256, 0, s>>>(part, nseg, n, G, ax, ay, az, (double *)vx, (double *)vy,
+        k_finalize_kick<double><<<nb, BS, 0, s>>>(part, nseg, n, G, ax, ay, az, (double *)vx, (double *)vy,
                                                    (double *)vz, coef);
     else
-        k_finalize_kick<float><<<nb, 256, 0, s>>>(part, nseg, n, G, ax, ay, az, (float *)vx, (float *)vy,
+        k_finalize_kick<float><<<nb, BS, 0, s>>>(part, nseg, n, G, ax, ay, az, (float *)vx, (float *)vy,
                                                   (float *)vz, coef);
     return check_launch("k_finalize_kick");
 }
@@ -620,9 +649,10 @@ int launch_finalize_kick(const double *part, int nseg, int64_t n, double G, doub
 int launch_finalize(const double *part, int nseg, int64_t n, double G, double *ax, double *ay,
                     double *az, double *pot, bool with_pot, hipStream_t s, bool with_acc) {
     if (n <= 0) return NB_OK;
-    const unsigned nb = (unsigned)((n + 255) / 256);
-    k_finalize<<<nb, 256, 0, s>>>(part, nseg, n, G, ax, ay, az, pot, with_pot ? 1 : 0,
-                                  with_acc ? 1 : 0);
+    const unsigned nb = (unsigned)((n + 63) / 64);
+    if (with_pot && with_acc) k_finalize<true, true><<<nb, BS, 0, s>>>(part, nseg, n, G, ax, ay, az, pot);
+    else if (with_pot) k_finalize<false, true><<<nb, BS, 0, s>>>(part, nseg, n, G, ax, ay, az, pot);
+    else if (with_acc) k_finalize<true, false><<<nb, BS, 0, s>>>(part, nseg, n, G, ax, ay, az, pot);
     return check_launch("k_finalize");
 }
 

@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <cmath>
 #include <string>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -542,7 +543,7 @@ int nb_destroy(nb_ctx *c) {
     dfree(c->m); dfree(c->h); dfree(c->coll);
     dfree(c->ax); dfree(c->ay); dfree(c->az); dfree(c->pot);
     dfree(c->perm);
-    dfree(c->tile_box); dfree(c->sub_box); dfree(c->tgeo); dfree(c->tbg); dfree(c->nflag); dfree(c->part); dfree(c->stage); dfree(c->red); dfree(c->wsrc);
+    dfree(c->tile_box); dfree(c->sub_box); dfree(c->tgeo); dfree(c->tbg); dfree(c->nflag); dfree(c->part); dfree(c->stage); dfree(c->red); dfree(c->wsrc); dfree(c->probe);
     dfree(c->time); dfree(c->flag); dfree(c->central);
     dfree(c->cx); dfree(c->cy); dfree(c->cz); dfree(c->cm); dfree(c->cidx);
     dfree(c->ti_end); dfree(c->ti_beg);
@@ -704,6 +705,28 @@ int nb_compute_potential(nb_ctx *c, int32_t add_self_term) {
     return NB_OK;
 }
 
+// Probe-point calls keep their workspace in the context up to this size (a
+// larger one is given back when the call ends).
+constexpr size_t PROBE_KEEP_BYTES = (size_t)64 << 20;
+
+// Source segments of a probe launch: few points are few target blocks (1009
+// points: four), so the sources are cut until the launch has about 4096
+// blocks.  One segment left 252 of the 256 CUs idle: 1009 points in 200003
+// particles took 12.2 ms a call, 0.19 ms in 782 segments.
+static int probe_segments(int64_t npts, int64_t n) {
+    const int64_t nblk = (npts + BS - 1) / BS;
+    return (int)std::min<int64_t>((4096 + nblk - 1) / nblk, std::max<int64_t>((n + BS - 1) / BS, 1));
+}
+
+static int ensure_probe(nb_ctx *c, size_t bytes) {
+    if (bytes <= c->probe_bytes) return NB_OK;
+    dfree(c->probe);
+    c->probe_bytes = 0;
+    NB_TRY(dalloc(&c->probe, bytes));
+    c->probe_bytes = bytes;
+    return NB_OK;
+}
+
 static int probe_points(nb_ctx *c, int64_t npts, const double *pts, double h, double *acc,
                         double *pot) {
     NB_TRY(check_ctx(c));
@@ -714,62 +737,64 @@ static int probe_points(nb_ctx *c, int64_t npts, const double *pts, double h, do
     if (npts == 0) return NB_OK;
     hipStream_t s = c->stream;
     const bool with_pot = pot != nullptr;
-    double *buf = nullptr;
-    // target xyz (double or float), outputs ax ay az pot, packed xyz staging
-    NB_TRY(dalloc(&buf, sizeof(double) * (size_t)npts * 10));
-    double *tx = buf, *ty = buf + npts, *tz = buf + 2 * npts;
-    double *oax = buf + 3 * npts, *oay = buf + 4 * npts, *oaz = buf + 5 * npts, *opot = buf + 6 * npts;
-    double *aos = buf + 7 * npts;
-    int rc = NB_OK;
-    do {
-        hipError_t e = hipMemcpyAsync(aos, pts, sizeof(double) * 3 * (size_t)npts,
-                                      hipMemcpyHostToDevice, s);
-        if (e != hipSuccess) { set_error("probe upload: %s", hipGetErrorString(e)); rc = NB_ERR_HIP; break; }
-        if ((rc = launch_tile_boxes(c->x, c->y, c->z, c->is_double, c->n, c->tile_box, c->sub_box, s))) break;
-        Geometry g = geometry(npts, c->n, 1, 1);
-        if (c->is_double) {
-            if ((rc = to_soa(aos, nullptr, npts, tx, ty, tz, true, s))) break;
-            ForceArgs<double> a{};
-            a.tx = tx; a.ty = ty; a.tz = tz; a.th = nullptr; a.th_const = h; a.nt = npts;
-            a.sx = (const double *)c->x; a.sy = (const double *)c->y; a.sz = (const double *)c->z;
-            a.sm = (const double *)c->m; a.ns = c->n;
-            a.tile_box = c->tile_box; a.sub_box = c->sub_box; a.use_origin = 1;
-            a.nseg = 1; a.seg_len = g.seg_len; a.nblk_i = g.nblk_i; a.G = c->G;
+    const Geometry g = geometry(npts, c->n, 1, probe_segments(npts, c->n));
+    // target xyz (double or float), outputs ax ay az pot, packed xyz staging,
+    // the target blocks' geometry and the segments' partial sums
+    const size_t np = (size_t)npts, geo = g.nseg > 1 ? (size_t)g.nblk_i * TG_STRIDE : 0;
+    NB_TRY(ensure_probe(c, sizeof(double) * (10 * np + geo + (g.nseg > 1 ? 4 * np * (size_t)g.nseg : 0))));
+    double *buf = c->probe;
+    double *tx = buf, *ty = buf + np, *tz = buf + 2 * np;
+    double *oax = buf + 3 * np, *oay = buf + 4 * np, *oaz = buf + 5 * np, *opot = buf + 6 * np;
+    double *aos = buf + 7 * np;
+    double *tgeo = g.nseg > 1 ? buf + 10 * np : nullptr, *part = g.nseg > 1 ? tgeo + geo : nullptr;
+    auto launch = [&]() -> int {
+        NB_HIP(hipMemcpyAsync(aos, pts, sizeof(double) * 3 * np, hipMemcpyHostToDevice, s));
+        if (c->mode != NB_MODE_FP64)   // (the FP64 kernel has no tile classes)
+            NB_TRY(launch_tile_boxes(c->x, c->y, c->z, c->is_double, c->n, c->tile_box, c->sub_box, s));
+        auto fill = [&](auto &a, auto *x, auto *y, auto *z) {
+            using T = std::remove_pointer_t<decltype(x)>;
+            a.tx = x; a.ty = y; a.tz = z; a.th = nullptr; a.th_const = h; a.nt = npts;
+            a.sx = (const T *)c->x; a.sy = (const T *)c->y; a.sz = (const T *)c->z; a.sm = (const T *)c->m;
+            a.ns = c->n;
+            a.tile_box = c->tile_box; a.sub_box = c->sub_box; a.use_origin = c->is_double ? 1 : 0;
+            a.tgeo = tgeo; a.part = part;
+            a.nseg = g.nseg; a.seg_len = g.seg_len; a.nblk_i = g.nblk_i; a.G = c->G;
             a.ax = oax; a.ay = oay; a.az = oaz; a.pot = opot; a.accumulate = 0;
-            rc = c->mode == NB_MODE_FP64 ? launch_force_f64(a, with_pot, s)
-                                         : launch_force_split(a, 1, with_pot, s);
-            if (rc) break;
+        };
+        if (c->is_double) {
+            NB_TRY(to_soa(aos, nullptr, npts, tx, ty, tz, true, s));
+            ForceArgs<double> a{};
+            fill(a, tx, ty, tz);
+            if (c->mode == NB_MODE_FP64) NB_TRY(launch_force_f64(a, with_pot, s));
+            else NB_TRY(launch_force_split(a, 1, with_pot, s, FAR_VALU, !with_pot));
         } else {
             // FP32 state: probe coordinates are rounded to FP32 like the particles.
             float *fx = (float *)tx, *fy = (float *)ty, *fz = (float *)tz;
-            if ((rc = to_soa(aos, nullptr, npts, fx, fy, fz, false, s))) break;
+            NB_TRY(to_soa(aos, nullptr, npts, fx, fy, fz, false, s));
             ForceArgs<float> a{};
-            a.tx = fx; a.ty = fy; a.tz = fz; a.th = nullptr; a.th_const = h; a.nt = npts;
-            a.sx = (const float *)c->x; a.sy = (const float *)c->y; a.sz = (const float *)c->z;
-            a.sm = (const float *)c->m; a.ns = c->n;
-            a.tile_box = c->tile_box; a.sub_box = c->sub_box; a.use_origin = 0;
-            a.nseg = 1; a.seg_len = g.seg_len; a.nblk_i = g.nblk_i; a.G = c->G;
-            a.ax = oax; a.ay = oay; a.az = oaz; a.pot = opot; a.accumulate = 0;
-            if ((rc = launch_force_f32(a, 1, with_pot, s))) break;
-            if ((rc = to_soa(aos, nullptr, npts, tx, ty, tz, true, s))) break;
+            fill(a, fx, fy, fz);
+            NB_TRY(launch_force_f32(a, 1, with_pot, s, !with_pot));
+            if (!c->bg.empty()) NB_TRY(to_soa(aos, nullptr, npts, tx, ty, tz, true, s));
         }
+        if (g.nseg > 1)
+            NB_TRY(launch_finalize(part, g.nseg, npts, c->G, oax, oay, oaz, opot, with_pot, s, !with_pot));
         for (const BgField &f : c->bg)
-            if ((rc = background(tx, ty, tz, npts, true, f, oax, oay, oaz, with_pot ? opot : nullptr, s))) break;
-        if (rc) break;
+            NB_TRY(background(tx, ty, tz, npts, true, f, with_pot ? nullptr : oax, oay, oaz,
+                              with_pot ? opot : nullptr, s));
         if (acc) {
-            if ((rc = to_aos(oax, oay, oaz, nullptr, npts, true, aos, s))) break;
-            e = hipMemcpyAsync(acc, aos, sizeof(double) * 3 * (size_t)npts, hipMemcpyDeviceToHost, s);
-            if (e != hipSuccess) { set_error("probe download: %s", hipGetErrorString(e)); rc = NB_ERR_HIP; break; }
+            NB_TRY(to_aos(oax, oay, oaz, nullptr, npts, true, aos, s));
+            NB_HIP(hipMemcpyAsync(acc, aos, sizeof(double) * 3 * np, hipMemcpyDeviceToHost, s));
         }
-        if (pot) {
-            e = hipMemcpyAsync(pot, opot, sizeof(double) * (size_t)npts, hipMemcpyDeviceToHost, s);
-            if (e != hipSuccess) { set_error("probe download: %s", hipGetErrorString(e)); rc = NB_ERR_HIP; break; }
-        }
-        e = hipStreamSynchronize(s);
-        if (e != hipSuccess) { set_error("probe sync: %s", hipGetErrorString(e)); rc = NB_ERR_HIP; break; }
-    } while (0);
-    (void)hipStreamSynchronize(s);
-    dfree(buf);
+        if (pot) NB_HIP(hipMemcpyAsync(pot, opot, sizeof(double) * np, hipMemcpyDeviceToHost, s));
+        NB_HIP(hipStreamSynchronize(s));
+        return NB_OK;
+    };
+    const int rc = launch();
+    if (rc) (void)hipStreamSynchronize(s);   // the caller's arrays are free again
+    if (c->probe_bytes > PROBE_KEEP_BYTES) {
+        dfree(c->probe);
+        c->probe_bytes = 0;
+    }
     return rc;
 }
 

@@ -80,6 +80,8 @@ struct nb_ctx {
     double *stage = nullptr;      // 3n doubles
     float *wsrc = nullptr;        // source weights m^(-2/3) (weighted far paths), n floats
     bool wsrc_valid = false;      // wsrc holds the weights of the current masses in the current order
+    double *probe = nullptr;      // workspace of the probe-point calls (grown on need, up to PROBE_KEEP_BYTES)
+    size_t probe_bytes = 0;
     double *red = nullptr;        // energy scratch
     double *time = nullptr;       // two FP64 time slots for device-side drift
     unsigned *flag = nullptr;

@@ -271,19 +271,23 @@ __global__ __launch_bounds__(BS) void k_force_f64(ForceArgs<double> a, int split
     }
 }
 
-// One target's per-segment partial sums, added by the 4 waves of a workgroup:
-// wave w takes the segments w, w + 4, ..., and lane l of wave 0 gets
-// ((w0 + w1) + (w2 + w3)) for target i (the same for all n and grids, so
-// results repeat).  Bound by the latency of the loads where n is small: one
-// thread per target walked up to 64 segments serially on n / 256 workgroups.
+// One target's per-segment partial sums, added by the W waves of a workgroup
+// (64 targets): wave w takes the segments w, w + W, ..., and lane l of wave 0
+// adds the waves' sums in order of w for target i, so results repeat.  Bound
+// by the latency of the loads where n is small: one thread per target walked
+// all the segments serially on n / 256 workgroups.  Four waves up to 64
+// segments; the hundreds that a few probe points take get sixteen (782
+// segments x 1009 points: 27 -> 20 us).
+constexpr int FIN_WAVES = 4, FIN_WAVES_MANY = 16, FIN_MANY = 64;
+
 template <bool ACC, bool POT>
 struct PartSums {
     static constexpr int NV = (ACC ? 3 : 0) + (POT ? 1 : 0);
     double v[NV];
 };
-template <bool ACC, bool POT>
+template <bool ACC, bool POT, int W>
 __device__ __forceinline__ bool sum_partials(const double *__restrict__ part, int nseg, int64_t n, int64_t i,
-                                             double (&red)[3][PartSums<ACC, POT>::NV][64],
+                                             double (&red)[W - 1][PartSums<ACC, POT>::NV][64],
                                              PartSums<ACC, POT> &r) {
     constexpr int NV = PartSums<ACC, POT>::NV;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -292,7 +296,7 @@ __device__ __forceinline__ bool sum_partials(const double *__restrict__ part, in
     if (i < n) {
         const double *p = part + (ACC ? 0 : 3) * n + i;
 #pragma unroll 4
-        for (int s = w; s < nseg; s += NW) {
+        for (int s = w; s < nseg; s += W) {
 #pragma unroll
             for (int q = 0; q < NV; ++q) r.v[q] += p[((int64_t)s * 4 + q) * n];
         }
@@ -304,21 +308,23 @@ __device__ __forceinline__ bool sum_partials(const double *__restrict__ part, in
     __syncthreads();
     if (w > 0 || i >= n) return false;
 #pragma unroll
-    for (int q = 0; q < NV; ++q) r.v[q] = (r.v[q] + red[0][q][lane]) + (red[1][q][lane] + red[2][q][lane]);
+    for (int u = 0; u < W - 1; ++u)
+#pragma unroll
+        for (int q = 0; q < NV; ++q) r.v[q] += red[u][q][lane];
     return true;
 }
 
 // Sum the per-segment partials in a fixed order and apply G (64 targets per
-// workgroup).  Measured: 59 segments x 30011 potentials 27 -> 5.4 us, 63
-// segments x 16001 forces 21 -> 6.7 us.
-template <bool ACC, bool POT>
-__global__ __launch_bounds__(BS) void k_finalize(const double *__restrict__ part, int nseg, int64_t n, double G,
-                                                 double *__restrict__ ax, double *__restrict__ ay,
-                                                 double *__restrict__ az, double *__restrict__ pot) {
-    __shared__ double red[3][PartSums<ACC, POT>::NV][64];
+// workgroup).  Measured with four waves: 59 segments x 30011 potentials
+// 27 -> 5.4 us, 63 segments x 16001 forces 21 -> 6.7 us.
+template <bool ACC, bool POT, int W>
+__global__ __launch_bounds__(64 * W) void k_finalize(const double *__restrict__ part, int nseg, int64_t n, double G,
+                                                     double *__restrict__ ax, double *__restrict__ ay,
+                                                     double *__restrict__ az, double *__restrict__ pot) {
+    __shared__ double red[W - 1][PartSums<ACC, POT>::NV][64];
     const int64_t i = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
     PartSums<ACC, POT> r;
-    if (!sum_partials<ACC, POT>(part, nseg, n, i, red, r)) return;
+    if (!sum_partials<ACC, POT, W>(part, nseg, n, i, red, r)) return;
     if constexpr (ACC) {
         ax[i] = G * r.v[0];
         ay[i] = G * r.v[1];
@@ -428,14 +434,14 @@ __global__ __launch_bounds__(BS) void k_drift_boxes(T *__restrict__ x, T *__rest
 // k_finalize followed by the step's kick (Vel += Acc * coef, the operations
 // of k_kick) on the accelerations it has just written.
 template <typename T>
-__global__ __launch_bounds__(BS) void k_finalize_kick(const double *__restrict__ part, int nseg, int64_t n,
+__global__ __launch_bounds__(64 * FIN_WAVES) void k_finalize_kick(const double *__restrict__ part, int nseg, int64_t n,
                                                       double G, double *__restrict__ ax, double *__restrict__ ay,
                                                       double *__restrict__ az, T *__restrict__ vx,
                                                       T *__restrict__ vy, T *__restrict__ vz, double coef) {
-    __shared__ double red[3][3][64];
+    __shared__ double red[FIN_WAVES - 1][3][64];
     const int64_t i = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
     PartSums<true, false> r;
-    if (!sum_partials<true, false>(part, nseg, n, i, red, r)) return;
+    if (!sum_partials<true, false, FIN_WAVES>(part, nseg, n, i, red, r)) return;
     const double fx = G * r.v[0], fy = G * r.v[1], fz = G * r.v[2];
     ax[i] = fx;
     ay[i] = fy;
@@ -638,10 +644,10 @@ int launch_finalize_kick(const double *part, int nseg, int64_t n, double G, doub
     if (n <= 0) return NB_OK;
     const unsigned nb = (unsigned)((n + 63) / 64);
     if (is_double)
-        k_finalize_kick<double><<<nb, BS, 0, s>>>(part, nseg, n, G, ax, ay, az, (double *)vx, (double *)vy,
+        k_finalize_kick<double><<<nb, 64 * FIN_WAVES, 0, s>>>(part, nseg, n, G, ax, ay, az, (double *)vx, (double *)vy,
                                                    (double *)vz, coef);
     else
-        k_finalize_kick<float><<<nb, BS, 0, s>>>(part, nseg, n, G, ax, ay, az, (float *)vx, (float *)vy,
+        k_finalize_kick<float><<<nb, 64 * FIN_WAVES, 0, s>>>(part, nseg, n, G, ax, ay, az, (float *)vx, (float *)vy,
                                                   (float *)vz, coef);
     return check_launch("k_finalize_kick");
 }
@@ -650,9 +656,17 @@ int launch_finalize(const double *part, int nseg, int64_t n, double G, double *a
                     double *az, double *pot, bool with_pot, hipStream_t s, bool with_acc) {
     if (n <= 0) return NB_OK;
     const unsigned nb = (unsigned)((n + 63) / 64);
-    if (with_pot && with_acc) k_finalize<true, true><<<nb, BS, 0, s>>>(part, nseg, n, G, ax, ay, az, pot);
-    else if (with_pot) k_finalize<false, true><<<nb, BS, 0, s>>>(part, nseg, n, G, ax, ay, az, pot);
-    else if (with_acc) k_finalize<true, false><<<nb, BS, 0, s>>>(part, nseg, n, G, ax, ay, az, pot);
+#define NB_FIN(A_, P_)                                                                                          \
+    do {                                                                                                        \
+        if (nseg > FIN_MANY)                                                                                    \
+            k_finalize<A_, P_, FIN_WAVES_MANY><<<nb, 64 * FIN_WAVES_MANY, 0, s>>>(part, nseg, n, G, ax, ay, az, pot); \
+        else                                                                                                    \
+            k_finalize<A_, P_, FIN_WAVES><<<nb, 64 * FIN_WAVES, 0, s>>>(part, nseg, n, G, ax, ay, az, pot);     \
+    } while (0)
+    if (with_pot && with_acc) NB_FIN(true, true);
+    else if (with_pot) NB_FIN(false, true);
+    else if (with_acc) NB_FIN(true, false);
+#undef NB_FIN
     return check_launch("k_finalize");
 }
 

@@ -421,7 +421,7 @@ int nb_adaptive_compute_force(nb_ctx *c, int64_t t_int, int64_t *nactive) {
     void *gx = gaz + n;
     void *gy = (char *)gx + (c->is_double ? 8 : 4) * (size_t)n;
     void *gz = (char *)gy + (c->is_double ? 8 : 4) * (size_t)n;
-    NB_TRY(launch_tile_boxes(c->x, c->y, c->z, c->is_double, n, c->tile_box, c->sub_box, s));
+    NB_TRY(launch_tile_boxes(c->x, c->y, c->z, c->is_double, n, c->h, 0.0, c->tile_box, c->sub_box, s));
     if (c->is_double)
         k_gather_targets<double><<<gridn(na), 256, 0, s>>>(
             (const double *)c->x, (const double *)c->y, (const double *)c->z, c->h, c->ad.idx,
@@ -433,12 +433,12 @@ int nb_adaptive_compute_force(nb_ctx *c, int64_t t_int, int64_t *nactive) {
     NB_TRY(launch_ok("k_gather_targets"));
     // Few active targets still fill the GPU: split the sources into segments
     // (partials reduced in a fixed order) for about 4096 blocks.
-    const int64_t ntiles = (n + BS - 1) / BS;
     const int64_t nblk = (na + BS - 1) / BS;
-    int64_t want = (4096 + nblk - 1) / nblk;
-    want = std::max<int64_t>(1, std::min<int64_t>(want, std::min<int64_t>(ntiles, 64)));
-    const int64_t tiles_per_seg = (ntiles + want - 1) / want;
-    const int nseg = (int)((ntiles + tiles_per_seg - 1) / tiles_per_seg);
+    const int64_t want = std::min<int64_t>((4096 + nblk - 1) / nblk, 64);
+    const int far = c->is_double || c->tun.far_path == FAR_MFMA_BF16 ? c->tun.far_path : FAR_VALU;
+    const Geometry g = c->mode != NB_MODE_FP64 && wave_path(far, 1, false, true)
+                           ? wave_launch_geometry(na, n, 1) : geometry(na, n, 1, want);
+    const int nseg = g.nseg;
     NB_TRY(ctx_ensure_part(c, nseg));
     if (c->is_double) {
         ForceArgs<double> a{};
@@ -447,7 +447,7 @@ int nb_adaptive_compute_force(nb_ctx *c, int64_t t_int, int64_t *nactive) {
         a.sx = (const double *)c->x; a.sy = (const double *)c->y; a.sz = (const double *)c->z;
         a.sm = (const double *)c->m; a.ns = n;
         a.tile_box = c->tile_box; a.sub_box = c->sub_box; a.use_origin = 1;
-        a.nseg = nseg; a.seg_len = tiles_per_seg * BS; a.nblk_i = (int)nblk; a.G = c->G;
+        a.nseg = nseg; a.seg_len = g.seg_len; a.nblk_i = g.nblk_i; a.G = c->G;
         a.ax = gax; a.ay = gay; a.az = gaz; a.pot = nullptr; a.part = c->part;
         a.skip_src = (c->mode == NB_MODE_SPLIT_CENTRAL && c->ncentral > 0) ? c->central : nullptr;
         if (c->mode == NB_MODE_FP64) {
@@ -455,12 +455,11 @@ int nb_adaptive_compute_force(nb_ctx *c, int64_t t_int, int64_t *nactive) {
         } else {
             // the context's far path (one target per lane here), with the
             // source weights that the weighted and matrix-core paths read
-            const int fp = c->tun.far_path;
-            if (far_path_weighted(fp)) {
+            if (far_path_weighted(far)) {
                 NB_TRY(launch_source_weights(c->m, true, n, c->wsrc, s));
                 a.sw = c->wsrc;
             }
-            NB_TRY(launch_force_split(a, 1, false, s, fp));
+            NB_TRY(launch_force_split(a, 1, false, s, far));
         }
         if (nseg > 1) NB_TRY(launch_finalize(c->part, nseg, na, c->G, gax, gay, gaz, nullptr, false, s));
         if (c->mode == NB_MODE_SPLIT_CENTRAL && c->ncentral > 0) {
@@ -480,14 +479,13 @@ int nb_adaptive_compute_force(nb_ctx *c, int64_t t_int, int64_t *nactive) {
         a.sx = (const float *)c->x; a.sy = (const float *)c->y; a.sz = (const float *)c->z;
         a.sm = (const float *)c->m; a.ns = n;
         a.tile_box = c->tile_box; a.sub_box = c->sub_box; a.use_origin = 0;
-        a.nseg = nseg; a.seg_len = tiles_per_seg * BS; a.nblk_i = (int)nblk; a.G = c->G;
+        a.nseg = nseg; a.seg_len = g.seg_len; a.nblk_i = g.nblk_i; a.G = c->G;
         a.ax = gax; a.ay = gay; a.az = gaz; a.pot = nullptr; a.part = c->part;
-        const int fp = c->tun.far_path == FAR_MFMA_BF16 ? FAR_MFMA_BF16 : FAR_VALU;
-        if (fp == FAR_MFMA_BF16) {
+        if (far == FAR_MFMA_BF16) {
             NB_TRY(launch_source_weights(c->m, false, n, c->wsrc, s));
             a.sw = c->wsrc;
         }
-        NB_TRY(launch_force_f32(a, 1, false, s, true, fp));
+        NB_TRY(launch_force_f32(a, 1, false, s, true, far));
         if (nseg > 1) NB_TRY(launch_finalize(c->part, nseg, na, c->G, gax, gay, gaz, nullptr, false, s));
     }
     // post-processing of the active targets, in the order of

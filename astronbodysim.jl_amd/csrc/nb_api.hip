@@ -105,11 +105,6 @@ int ensure_part(nb_ctx *c, int nseg) {
     return NB_OK;
 }
 
-struct Geometry {
-    int tpt, nseg, nblk_i;
-    int64_t seg_len;
-};
-
 // Workspaces of the matrix-core far path, allocated when a launch first needs
 // them: the flags of the split far/near passes (one byte per wave) and, with
 // several source segments, the bf16 B operands (16 dwords per target).
@@ -130,16 +125,12 @@ int ensure_tbg(nb_ctx *c, const Geometry &g) {
     return dalloc(&c->tbg, sizeof(unsigned) * 16 * (size_t)BS * (size_t)((c->n + BS - 1) / BS + 1));
 }
 
-Geometry geometry(int64_t nt, int64_t ns, int tpt, int want_seg) {
-    Geometry g;
-    g.tpt = tpt;
-    g.nblk_i = (int)((nt + (int64_t)BS * tpt - 1) / ((int64_t)BS * tpt));
-    const int64_t ntiles = std::max<int64_t>((ns + BS - 1) / BS, 1);
-    int64_t nseg = std::min<int64_t>(std::max(want_seg, 1), ntiles);
-    const int64_t tiles_per_seg = (ntiles + nseg - 1) / nseg;
-    g.seg_len = tiles_per_seg * BS;
-    g.nseg = (int)((ntiles + tiles_per_seg - 1) / tiles_per_seg);
-    return g;
+// The launch of the context's own forces or potentials.
+Geometry force_geometry(const nb_ctx *c, bool pot, bool acc) {
+    if (c->mode == NB_MODE_FP64) return geometry(c->n, c->n, 1, c->tun.j_segments);
+    if (wave_path(c->tun.far_path, c->tun.targets_per_thread, pot, acc))
+        return wave_launch_geometry(c->n, c->n, c->tun.j_segments);
+    return geometry(c->n, c->n, c->tun.targets_per_thread, c->tun.j_segments);
 }
 
 int record_start(nb_ctx *c, hipEvent_t *e0) {
@@ -271,10 +262,10 @@ int run_force(nb_ctx *c, bool with_pot, bool allow_timing, bool allow_sort = tru
     c->force_calls++;
     c->calls_since_sort++;
     if (!(fuse && fuse->boxes_ready && !resorted))
-        NB_TRY(launch_tile_boxes(c->x, c->y, c->z, c->is_double, n, c->tile_box, c->sub_box, s));
+        NB_TRY(launch_tile_boxes(c->x, c->y, c->z, c->is_double, n, c->h, 0.0, c->tile_box, c->sub_box, s));
     const bool f64 = c->mode == NB_MODE_FP64;
     const int tpt = f64 ? 1 : c->tun.targets_per_thread;
-    Geometry g = geometry(n, n, tpt, c->tun.j_segments);
+    const Geometry g = force_geometry(c, with_pot, !(with_pot && pot_only));
     NB_TRY(ensure_part(c, g.nseg));
     NB_TRY(ensure_tbg(c, g));
     hipEvent_t e0 = nullptr;
@@ -286,7 +277,7 @@ int run_force(nb_ctx *c, bool with_pot, bool allow_timing, bool allow_sort = tru
         a.sx = (const double *)c->x; a.sy = (const double *)c->y; a.sz = (const double *)c->z;
         a.sm = (const double *)c->m; a.ns = n;
         a.tile_box = c->tile_box;
-        a.sub_box = c->sub_box;
+        a.sub_box = a.tbox = c->sub_box;
         a.tgeo = c->tgeo;
         a.tbg = c->tbg;
         a.tgeo_ready = fuse && !resorted ? fuse->geo_ready : 0;
@@ -311,7 +302,7 @@ int run_force(nb_ctx *c, bool with_pot, bool allow_timing, bool allow_sort = tru
         a.sx = (const float *)c->x; a.sy = (const float *)c->y; a.sz = (const float *)c->z;
         a.sm = (const float *)c->m; a.ns = n;
         a.tile_box = c->tile_box;
-        a.sub_box = c->sub_box;
+        a.sub_box = a.tbox = c->sub_box;
         a.tgeo = c->tgeo;
         a.tbg = c->tbg;
         a.tgeo_ready = fuse && !resorted ? fuse->geo_ready : 0;
@@ -713,6 +704,8 @@ constexpr size_t PROBE_KEEP_BYTES = (size_t)64 << 20;
 // points: four), so the sources are cut until the launch has about 4096
 // blocks.  One segment left 252 of the 256 CUs idle: 1009 points in 200003
 // particles took 12.2 ms a call, 0.19 ms in 782 segments.
+// (The FP32-pair kernels: at most PROBE_SEGMENTS.)
+constexpr int PROBE_SEGMENTS = 1024;
 static int probe_segments(int64_t npts, int64_t n) {
     const int64_t nblk = (npts + BS - 1) / BS;
     return (int)std::min<int64_t>((4096 + nblk - 1) / nblk, std::max<int64_t>((n + BS - 1) / BS, 1));
@@ -737,27 +730,29 @@ static int probe_points(nb_ctx *c, int64_t npts, const double *pts, double h, do
     if (npts == 0) return NB_OK;
     hipStream_t s = c->stream;
     const bool with_pot = pot != nullptr;
-    const Geometry g = geometry(npts, c->n, 1, probe_segments(npts, c->n));
-    // target xyz (double or float), outputs ax ay az pot, packed xyz staging,
-    // the target blocks' geometry and the segments' partial sums
-    const size_t np = (size_t)npts, geo = g.nseg > 1 ? (size_t)g.nblk_i * TG_STRIDE : 0;
-    NB_TRY(ensure_probe(c, sizeof(double) * (10 * np + geo + (g.nseg > 1 ? 4 * np * (size_t)g.nseg : 0))));
+    const bool f64 = c->mode == NB_MODE_FP64;
+    const Geometry g = f64 ? geometry(npts, c->n, 1, probe_segments(npts, c->n))
+                           : wave_launch_geometry(npts, c->n, 1, PROBE_SEGMENTS);
+    // target xyz (double or float), outputs ax ay az pot, packed xyz staging and
+    // the segments' partial sums
+    const size_t np = (size_t)npts;
+    NB_TRY(ensure_probe(c, sizeof(double) * (10 * np + (g.nseg > 1 ? 4 * np * (size_t)g.nseg : 0))));
     double *buf = c->probe;
     double *tx = buf, *ty = buf + np, *tz = buf + 2 * np;
     double *oax = buf + 3 * np, *oay = buf + 4 * np, *oaz = buf + 5 * np, *opot = buf + 6 * np;
     double *aos = buf + 7 * np;
-    double *tgeo = g.nseg > 1 ? buf + 10 * np : nullptr, *part = g.nseg > 1 ? tgeo + geo : nullptr;
+    double *part = g.nseg > 1 ? buf + 10 * np : nullptr;
     auto launch = [&]() -> int {
         NB_HIP(hipMemcpyAsync(aos, pts, sizeof(double) * 3 * np, hipMemcpyHostToDevice, s));
-        if (c->mode != NB_MODE_FP64)   // (the FP64 kernel has no tile classes)
-            NB_TRY(launch_tile_boxes(c->x, c->y, c->z, c->is_double, c->n, c->tile_box, c->sub_box, s));
+        if (!f64)   // (the FP64 kernel has no tile classes)
+            NB_TRY(launch_tile_boxes(c->x, c->y, c->z, c->is_double, c->n, c->h, 0.0, c->tile_box, c->sub_box, s));
         auto fill = [&](auto &a, auto *x, auto *y, auto *z) {
             using T = std::remove_pointer_t<decltype(x)>;
             a.tx = x; a.ty = y; a.tz = z; a.th = nullptr; a.th_const = h; a.nt = npts;
             a.sx = (const T *)c->x; a.sy = (const T *)c->y; a.sz = (const T *)c->z; a.sm = (const T *)c->m;
             a.ns = c->n;
             a.tile_box = c->tile_box; a.sub_box = c->sub_box; a.use_origin = c->is_double ? 1 : 0;
-            a.tgeo = tgeo; a.part = part;
+            a.part = part;
             a.nseg = g.nseg; a.seg_len = g.seg_len; a.nblk_i = g.nblk_i; a.G = c->G;
             a.ax = oax; a.ay = oay; a.az = oaz; a.pot = opot; a.accumulate = 0;
         };
@@ -765,7 +760,7 @@ static int probe_points(nb_ctx *c, int64_t npts, const double *pts, double h, do
             NB_TRY(to_soa(aos, nullptr, npts, tx, ty, tz, true, s));
             ForceArgs<double> a{};
             fill(a, tx, ty, tz);
-            if (c->mode == NB_MODE_FP64) NB_TRY(launch_force_f64(a, with_pot, s));
+            if (f64) NB_TRY(launch_force_f64(a, with_pot, s));
             else NB_TRY(launch_force_split(a, 1, with_pot, s, FAR_VALU, !with_pot));
         } else {
             // FP32 state: probe coordinates are rounded to FP32 like the particles.
@@ -860,13 +855,13 @@ static int enqueue_step(nb_ctx *c, int64_t k, double dt, bool allow_timing, bool
         // call's launch would store it (origin mode, B operands of far path 4).
         StepGeometry sg{};
         const StepGeometry *gp = nullptr;
-        if (c->mode != NB_MODE_FP64 && c->tun.targets_per_thread == 1 && c->tgeo) {
-            Geometry g = geometry(c->n, c->n, 1, c->tun.j_segments);
+        if (c->mode != NB_MODE_FP64 && c->tun.targets_per_thread == 1 && c->tgeo &&
+            !wave_path(c->tun.far_path, 1, false, true)) {
+            const Geometry g = force_geometry(c, false, true);
             if (g.nseg > 1) {
                 NB_TRY(ensure_part(c, g.nseg));
                 NB_TRY(ensure_tbg(c, g));
                 const bool bf16 = c->tun.far_path == FAR_MFMA_BF16;
-                sg.h = c->h;
                 sg.tgeo = c->tgeo;
                 sg.tbg = bf16 ? c->tbg : nullptr;
                 sg.use_origin = (c->is_double || bf16) ? 1 : 0;
@@ -875,7 +870,7 @@ static int enqueue_step(nb_ctx *c, int64_t k, double dt, bool allow_timing, bool
             }
         }
         NB_TRY(launch_drift_boxes(c->x, c->y, c->z, c->vx, c->vy, c->vz, c->n, dt, c->time, rd, wr, c->is_double,
-                                  c->tile_box, c->sub_box, c->stream, gp));
+                                  c->h, c->tile_box, c->sub_box, c->stream, gp));
         fuse.boxes_ready = true;
     } else {
         NB_TRY(drift(c->x, c->y, c->z, c->vx, c->vy, c->vz, c->n, dt, c->time, rd, wr, c->is_double,
@@ -909,8 +904,7 @@ int nb_kdk_steps(nb_ctx *c, int64_t nsteps, double dt, double t_begin, int32_t u
         if (!reuse) {
             drop_graph(c);
             // Make sure partial buffers exist before capture (no allocation inside).
-            Geometry g = geometry(c->n, c->n, c->mode == NB_MODE_FP64 ? 1 : c->tun.targets_per_thread,
-                                  c->tun.j_segments);
+            const Geometry g = force_geometry(c, false, true);
             NB_TRY(ensure_part(c, g.nseg));
             NB_TRY(ensure_tbg(c, g));
             NB_TRY(ensure_source_weights(c));

@@ -16,6 +16,7 @@
 #include "nb_block.h"
 #include "nb_internal.h"
 #include "nb_pair.h"
+#include "nb_wave.h"
 
 namespace nb {
 
@@ -68,6 +69,60 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(MF == 4 ? 4 
             if (POT) p[3 * a.nt + i] = Aq[k];
         }
     }
+}
+
+// Far path 0 with one target per lane: wave w of workgroup ib owns the targets
+// 64 (NW ib + w).. and walks the segment's sources on its own (wave_force); the
+// waves of a workgroup share the scalar cache's lines of those sources, nothing
+// else.  Held to 6 waves per SIMD (two values spilled outside the pair loops;
+// 5 without): 60000 particles in FP32 986 -> 929 us a force, 30011 in split
+// precision 312 -> 308 us.  Against the block-wide kernel that it replaced (one
+// force call with its boxes and segment sums, split precision, Plummer): 1000
+// particles 32 -> 16 us, 4096 35 -> 25, 16384 130 -> 110, 30011 333 -> 308;
+// FP32 60000 1030 -> 929.
+template <typename T, bool ACC, bool POT>
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(ACC &&POT && sizeof(T) == 8 ? 5 : 6)))
+void k_force_wave(ForceArgs<T> a) {
+    __shared__ WaveStage<T> st[NW];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    const int seg = logical / a.nblk_i;
+    const int ib = logical - seg * a.nblk_i;
+    const int64_t i0 = (int64_t)ib * BS + wave * 64;
+    if (i0 >= a.nt) return;   // (no workgroup barrier follows)
+    const int64_t i = i0 + (threadIdx.x & 63);
+    const int64_t ic = i < a.nt ? i : a.nt - 1;
+    const int64_t j0 = (int64_t)seg * a.seg_len;
+    const int64_t j1 = (j0 + a.seg_len < a.ns) ? j0 + a.seg_len : a.ns;
+    double Ax, Ay, Az, Aq;
+    wave_force<T, ACC, POT>(st[wave], a.tx[ic], a.ty[ic], a.tz[ic], a.th ? a.th[ic] : a.th_const,
+                            a.tbox ? a.tbox + (i0 / 64) * 8 : nullptr, a.sx, a.sy, a.sz, a.sm, a.skip_src,
+                            a.sub_box ? a.sub_box + (j0 / SB) * 8 : nullptr,
+                            a.sub_box ? nullptr : a.tile_box + (j0 / BS) * 8, j0, j1, Ax, Ay, Az, Aq);
+    if (i >= a.nt) return;
+    if (a.nseg == 1) {
+        if (ACC) {
+            a.ax[i] = a.G * Ax;
+            a.ay[i] = a.G * Ay;
+            a.az[i] = a.G * Az;
+        }
+        if (POT) a.pot[i] = -a.G * Aq;
+    } else {
+        double *p = a.part + (int64_t)seg * 4 * a.nt;
+        if (ACC) {
+            p[i] = Ax;
+            p[a.nt + i] = Ay;
+            p[2 * a.nt + i] = Az;
+        }
+        if (POT) p[3 * a.nt + i] = Aq;
+    }
+}
+
+template <typename T>
+static void launch_wave(const ForceArgs<T> &a, int64_t nb, bool pot, bool acc, hipStream_t s) {
+    if (pot && acc) k_force_wave<T, true, true><<<(unsigned)nb, BS, 0, s>>>(a);
+    else if (pot) k_force_wave<T, false, true><<<(unsigned)nb, BS, 0, s>>>(a);
+    else k_force_wave<T, true, false><<<(unsigned)nb, BS, 0, s>>>(a);
 }
 
 // Near pass of a split bf16 launch (forces only): one wavefront per
@@ -335,9 +390,10 @@ __global__ __launch_bounds__(64 * W) void k_finalize(const double *__restrict__ 
 
 // Bounding box of each BS-source tile (lo xyz, hi xyz) and, when sub is not
 // null, of each of its NQ quarters (the sources of one wave; an empty quarter
-// gets lo = DBL_MAX, hi = -DBL_MAX).  One block per tile; thread t holds the
-// position of source BS * blockIdx.x + t (v: the source exists).
-__device__ __forceinline__ void tile_box_block(double px, double py, double pz, bool v,
+// gets lo = DBL_MAX, hi = -DBL_MAX) with the quarter's largest h in slot 6.
+// One block per tile; thread t holds the position of source BS * blockIdx.x + t
+// (v: the source exists).
+__device__ __forceinline__ void tile_box_block(double px, double py, double pz, double ph, bool v,
                                                double *__restrict__ box, double *__restrict__ sub,
                                                double (&red)[6][NW]) {
     double lo[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, hi[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
@@ -351,6 +407,7 @@ __device__ __forceinline__ void tile_box_block(double px, double py, double pz, 
         lo[d] = wave_min(lo[d]);
         hi[d] = wave_max(hi[d]);
     }
+    const double hm = sub ? wave_max(v ? ph : 0.0) : 0.0;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     if (lane == 0) {
 #pragma unroll
@@ -360,7 +417,9 @@ __device__ __forceinline__ void tile_box_block(double px, double py, double pz, 
         double *o = sub + ((int64_t)blockIdx.x * NQ + w) * 8;
 #pragma unroll
         for (int d = 0; d < 3; ++d) { o[d] = lo[d]; o[3 + d] = hi[d]; }
+        o[6] = hm;
     }
+    if (!box) return;   // (uniform over the launch)
     __syncthreads();
     if (threadIdx.x < 6) {
         const int q = threadIdx.x;
@@ -373,11 +432,13 @@ __device__ __forceinline__ void tile_box_block(double px, double py, double pz, 
 template <typename T>
 __global__ __launch_bounds__(BS) void k_tile_boxes(const T *__restrict__ x, const T *__restrict__ y,
                                                    const T *__restrict__ z, int64_t n,
+                                                   const double *__restrict__ h, double h_const,
                                                    double *__restrict__ box, double *__restrict__ sub) {
     __shared__ double red[6][NW];
     const int64_t j = (int64_t)blockIdx.x * BS + threadIdx.x;
     const bool v = j < n;
-    tile_box_block(v ? (double)x[j] : 0.0, v ? (double)y[j] : 0.0, v ? (double)z[j] : 0.0, v, box, sub, red);
+    tile_box_block(v ? (double)x[j] : 0.0, v ? (double)y[j] : 0.0, v ? (double)z[j] : 0.0,
+                   v && h ? h[j] : h_const, v, box, sub, red);
 }
 
 // A step's drift (Pos += Vel * (t_new - t_old), the operations of k_drift,
@@ -410,11 +471,12 @@ __global__ __launch_bounds__(BS) void k_drift_boxes(T *__restrict__ x, T *__rest
         pz += vz[j] * d;
         x[j] = px; y[j] = py; z[j] = pz;
     }
-    tile_box_block((double)px, (double)py, (double)pz, v, box, sub, red);
+    const double ph = v ? h[j] : 0.0;
+    tile_box_block((double)px, (double)py, (double)pz, ph, v, box, sub, red);
     if constexpr (GEO) {
         const int tid = threadIdx.x;
         double gx[1] = {v ? (double)px : 0.0}, gy[1] = {v ? (double)py : 0.0}, gz[1] = {v ? (double)pz : 0.0};
-        double gh[1] = {v ? h[j] : 0.0};
+        double gh[1] = {ph};
         bool gv[1] = {v};
         BlockStats st;
         block_stats<1>(gx, gy, gz, gh, gv, use_origin != 0, gred, st);
@@ -465,15 +527,15 @@ static int check_launch(const char *what) {
 }
 
 int launch_tile_boxes(const void *x, const void *y, const void *z, int is_double, int64_t n,
-                      double *box, double *sub_box, hipStream_t s) {
+                      const double *h, double h_const, double *box, double *sub_box, hipStream_t s) {
     if (n <= 0) return NB_OK;
     const int64_t ntiles = (n + BS - 1) / BS;
     if (is_double)
         k_tile_boxes<double><<<(unsigned)ntiles, BS, 0, s>>>((const double *)x, (const double *)y,
-                                                            (const double *)z, n, box, sub_box);
+                                                            (const double *)z, n, h, h_const, box, sub_box);
     else
         k_tile_boxes<float><<<(unsigned)ntiles, BS, 0, s>>>((const float *)x, (const float *)y,
-                                                           (const float *)z, n, box, sub_box);
+                                                           (const float *)z, n, h, h_const, box, sub_box);
     return check_launch("k_tile_boxes");
 }
 
@@ -516,12 +578,17 @@ static int launch_f32_impl(ForceArgs<T> a, int tpt, bool pot, hipStream_t s, boo
         set_error("force grid too large (%lld blocks)", (long long)nb);
         return NB_ERR_INVALID;
     }
+    if (wave_path(MF, tpt, pot, acc)) {
+        launch_wave<T>(a, nb, pot, acc, s);
+        return check_launch("k_force_wave");
+    }
     NB_TRY(prepare_target_geom(a, tpt, s));
     dim3 g((unsigned)nb), b(BS);
 #define NB_L(TPT_, POT_) k_force_f32<T, TPT_, POT_, (POT_ ? 0 : MF)><<<g, b, 0, s>>>(a)
 #define NB_LP(TPT_) k_force_f32<T, TPT_, true, 0, false><<<g, b, 0, s>>>(a)
-    if (tpt == 1) { if (pot && !acc) NB_LP(1); else if (pot) NB_L(1, true); else NB_L(1, false); }
-    else if (tpt == 2) { if (pot && !acc) NB_LP(2); else if (pot) NB_L(2, true); else NB_L(2, false); }
+    if (tpt == 1) {
+        if constexpr (MF != FAR_VALU) NB_L(1, false);   // (the others take k_force_wave)
+    } else if (tpt == 2) { if (pot && !acc) NB_LP(2); else if (pot) NB_L(2, true); else NB_L(2, false); }
     else if (tpt == 4) { if (pot && !acc) NB_LP(4); else if (pot) NB_L(4, true); else NB_L(4, false); }
     else {
         set_error("unsupported targets_per_thread %d", tpt);
@@ -613,12 +680,11 @@ int launch_force_f64(const ForceArgs<double> &a_in, bool pot, hipStream_t s) {
 }
 
 int launch_drift_boxes(void *x, void *y, void *z, const void *vx, const void *vy, const void *vz, int64_t n,
-                       double dt, double *time, int rd, int wr, int is_double, double *box, double *sub_box,
-                       hipStream_t s, const StepGeometry *geo) {
+                       double dt, double *time, int rd, int wr, int is_double, const double *h, double *box,
+                       double *sub_box, hipStream_t s, const StepGeometry *geo) {
     if (n <= 0) return NB_OK;
     const unsigned nt = (unsigned)((n + BS - 1) / BS);
     const bool g = geo && geo->tgeo, r = g && geo->tbg;
-    const double *h = g ? geo->h : nullptr;
     double *tg = g ? geo->tgeo : nullptr;
     unsigned *tb = r ? geo->tbg : nullptr;
     const int uo = g ? geo->use_origin : 0;

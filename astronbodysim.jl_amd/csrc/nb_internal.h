@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <algorithm>
 #include <string>
 #include <vector>
 
@@ -50,7 +51,10 @@ struct ForceArgs {
     const T *sx, *sy, *sz, *sm;  // sources
     int64_t ns;
     const double *tile_box;  // [ntiles][8]: lo xyz, hi xyz, (unused) of each BS-source tile
-    const double *sub_box;   // [ntiles][NQ][8]: the same for each tile's quarters, or nullptr
+    const double *sub_box;   // [ntiles][NQ][8]: the same for each tile's quarters (with the quarter's
+                             // largest softening length in slot 6), or nullptr
+    const double *tbox;      // the same record for every 64 targets (sub_box where targets are the
+                             // sources), or nullptr: reduced by the kernel (k_force_wave)
     double *tgeo;            // [nblk_i][TG_STRIDE] workspace for the target blocks' geometry, or nullptr
     int tgeo_ready;          // 1: tgeo holds this call's geometry (written by the step's drift), 2: tbg too
     unsigned *tbg;           // [nblk_i][BS][16] workspace for their bf16 B operands, or nullptr
@@ -74,14 +78,62 @@ constexpr int FAR_MFMA_R2 = 2;    // r^2 and sum on the matrix cores (farthest t
 constexpr int FAR_WEIGHTED = 3;   // weighted far tiles: 10 VALU + rsq per pair
 constexpr int FAR_MFMA_BF16 = 4;  // bf16-split r^2 on the matrix cores, sum on the VALU
 
+// Whether a launch of the FP32-pair kernels takes the wavefront kernel
+// (k_force_wave: far path 0, one target per lane; also forces and potentials
+// together where the far path has no such kernel), whose source segments may
+// be cut at any quarter (SB sources) instead of at tiles.
+inline bool wave_path(int far_path, int tpt, bool pot, bool acc) {
+    return tpt == 1 && (far_path == FAR_VALU || (pot && (acc || far_path != FAR_MFMA_BF16)));
+}
+
+// A launch over target blocks (BS targets per target of a lane) and source
+// segments.
+struct Geometry {
+    int tpt, nseg, nblk_i;
+    int64_t seg_len;
+};
+
+// Segments of whole tiles.
+inline Geometry geometry(int64_t nt, int64_t ns, int tpt, int64_t want_seg) {
+    Geometry g;
+    g.tpt = tpt;
+    g.nblk_i = (int)((nt + (int64_t)BS * tpt - 1) / ((int64_t)BS * tpt));
+    const int64_t ntiles = std::max<int64_t>((ns + BS - 1) / BS, 1);
+    const int64_t nseg = std::min<int64_t>(std::max<int64_t>(want_seg, 1), ntiles);
+    const int64_t tiles_per_seg = (ntiles + nseg - 1) / nseg;
+    g.seg_len = tiles_per_seg * BS;
+    g.nseg = (int)((ntiles + tiles_per_seg - 1) / tiles_per_seg);
+    return g;
+}
+
+// A k_force_wave launch: the segments are cut at quarters.  Few targets are
+// spread over more segments than asked for, up to max_seg (or one per quarter),
+// until the chip has 8 waves per SIMD (8192 waves): a wave alone on its SIMD
+// is bound by latency.
+constexpr int WAVE_SEGMENTS = 64;
+inline Geometry wave_launch_geometry(int64_t nt, int64_t ns, int64_t want_seg, int64_t max_seg = WAVE_SEGMENTS) {
+    Geometry g;
+    g.tpt = 1;
+    g.nblk_i = (int)((nt + BS - 1) / BS);
+    const int64_t nq = std::max<int64_t>((ns + SB - 1) / SB, 1), ntw = std::max<int64_t>((nt + 63) / 64, 1);
+    const int64_t fill = std::min<int64_t>((8192 + ntw - 1) / ntw, max_seg);
+    const int64_t nseg = std::min<int64_t>(std::max<int64_t>(std::max<int64_t>(want_seg, 1), fill), nq);
+    const int64_t qs = (nq + nseg - 1) / nseg;
+    g.seg_len = qs * SB;
+    g.nseg = (int)((nq + qs - 1) / qs);
+    return g;
+}
+
 // Passes of the force kernel (force_block): every tile, or the far tiles
 // only (the split bf16 matrix-core launch, whose near tiles k_force_near adds).
 constexpr int PASS_ALL = 0;
 constexpr int PASS_FAR = 1;
 
 // Launchers (nb_force.hip)
+// Tile boxes (box) and quarter boxes (sub_box, with the largest of h or h_const
+// in slot 6) of n particles; either output may be nullptr.
 int launch_tile_boxes(const void *x, const void *y, const void *z, int is_double, int64_t n,
-                      double *box, double *sub_box, hipStream_t s);
+                      const double *h, double h_const, double *box, double *sub_box, hipStream_t s);
 // acc = false (with pot) writes the potential alone.
 // far_path FAR_MFMA_BF16 (tpt 1, forces or potential alone) runs the FP32
 // state relative to a per-block FP64 origin; any other value is far path 0.
@@ -103,14 +155,13 @@ int launch_finalize(const double *part, int nseg, int64_t n, double G, double *a
 // blocks' geometry (tgeo non-null; one target per lane, several segments),
 // with the bf16 B operands when tbg is non-null.
 struct StepGeometry {
-    const double *h;     // target softening lengths
     double *tgeo;
     unsigned *tbg;
     int use_origin;
 };
 int launch_drift_boxes(void *x, void *y, void *z, const void *vx, const void *vy, const void *vz, int64_t n,
-                       double dt, double *time, int rd, int wr, int is_double, double *box, double *sub_box,
-                       hipStream_t s, const StepGeometry *geo = nullptr);
+                       double dt, double *time, int rd, int wr, int is_double, const double *h, double *box,
+                       double *sub_box, hipStream_t s, const StepGeometry *geo = nullptr);
 int launch_finalize_kick(const double *part, int nseg, int64_t n, double G, double *ax, double *ay, double *az,
                          void *vx, void *vy, void *vz, double coef, int is_double, hipStream_t s);
 

@@ -88,29 +88,31 @@ extern "C" int nb_compute_force_noalloc(int32_t precision_mode, int64_t n, const
     hipStream_t s = (hipStream_t)stream;
     const bool f64 = precision_mode == NB_MODE_FP64;
 
-    // scratch layout: tile boxes, then the per-segment partials
+    // scratch layout: the boxes, then the per-segment partials.  The boxes are
+    // those of the tile quarters (FP32-pair kernel) while these take a quarter
+    // of the scratch at most, else those of the tiles.
     const int64_t ntiles = (n + BS - 1) / BS;
-    const size_t box_bytes = align256(sizeof(double) * 8 * (size_t)ntiles);
+    const size_t sub_bytes = align256(sizeof(double) * 8 * NQ * (size_t)ntiles);
+    const bool quarters = !f64 && sub_bytes <= SCRATCH_BYTES / 4;
+    const size_t box_bytes = f64 ? 0 : quarters ? sub_bytes : align256(sizeof(double) * 8 * (size_t)ntiles);
     const size_t seg_bytes = sizeof(double) * 4 * (size_t)n;
     const int64_t nblk = (n + BS - 1) / BS;
     // about 8k blocks to fill the 256 CUs, as many segments as the scratch holds
-    int64_t want = std::min<int64_t>(std::max<int64_t>((8192 + nblk - 1) / nblk, 1), 64);
-    want = std::min<int64_t>(want, ntiles);
     const int64_t fit = (int64_t)((SCRATCH_BYTES - box_bytes) / seg_bytes);
-    if (want > fit) want = fit;
-    if (want < 2) want = 1;
-    const int64_t tiles_per_seg = (ntiles + want - 1) / want;
-    const int nseg = (int)((ntiles + tiles_per_seg - 1) / tiles_per_seg);
+    const int64_t want = std::min<int64_t>(std::min<int64_t>(std::max<int64_t>((8192 + nblk - 1) / nblk, 1), 64), fit);
+    const Geometry g = quarters ? wave_launch_geometry(n, n, 1, std::max<int64_t>(std::min<int64_t>(want, fit), 1))
+                                : geometry(n, n, 1, want);
     double *box = (double *)base;
-    double *part = nseg > 1 ? (double *)((unsigned char *)base + box_bytes) : nullptr;
+    double *part = g.nseg > 1 ? (double *)((unsigned char *)base + box_bytes) : nullptr;
 
     ForceArgs<double> a{};
     a.tx = x; a.ty = y; a.tz = z;
     a.th = h; a.th_const = h_const; a.nt = n;
     a.sx = x; a.sy = y; a.sz = z; a.sm = m; a.ns = n;
-    a.tile_box = box;
+    a.tile_box = quarters ? nullptr : box;
+    a.sub_box = a.tbox = quarters ? box : nullptr;
     a.use_origin = 1;
-    a.nseg = nseg; a.seg_len = tiles_per_seg * BS; a.nblk_i = (int)nblk;
+    a.nseg = g.nseg; a.seg_len = g.seg_len; a.nblk_i = g.nblk_i;
     a.G = G;
     a.ax = ax; a.ay = ay; a.az = az; a.pot = pot;
     a.part = part;
@@ -120,9 +122,9 @@ extern "C" int nb_compute_force_noalloc(int32_t precision_mode, int64_t n, const
     if (f64) {
         NB_TRY(launch_force_f64(a, with_pot, s));
     } else {
-        NB_TRY(launch_tile_boxes(x, y, z, 1, n, box, nullptr, s));
+        NB_TRY(launch_tile_boxes(x, y, z, 1, n, h, h_const, quarters ? nullptr : box, quarters ? box : nullptr, s));
         NB_TRY(launch_force_split(a, 1, with_pot, s, FAR_VALU, true));
     }
-    if (nseg > 1) NB_TRY(launch_finalize(part, nseg, n, G, ax, ay, az, pot, with_pot, s, true));
+    if (g.nseg > 1) NB_TRY(launch_finalize(part, g.nseg, n, G, ax, ay, az, pot, with_pot, s, true));
     return NB_OK;
 }

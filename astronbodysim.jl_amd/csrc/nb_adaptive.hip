@@ -20,9 +20,8 @@
 #include <algorithm>
 #include <cstring>
 #include <math.h>
-#include <rocprim/device/device_select.hpp>
-#include <rocprim/iterator/counting_iterator.hpp>
 
+#include "nb_block.h"
 #include "nb_ctx.h"
 
 namespace nb {
@@ -48,13 +47,13 @@ struct AdaptParams {
 
 // Error flags: 1 = dt < MinStep, 2 = integer step <= 0.
 __device__ __forceinline__ int64_t get_timestep_dev(double ax, double ay, double az, double h,
-                                                    const AdaptParams &p, unsigned *flag) {
+                                                    const AdaptParams &p, unsigned &flag) {
     const double ac = sqrt(ax * ax + ay * ay + az * az);
     double dt = sqrt(2.0 * p.err_tol * h / ac);
     if (dt > p.max_step) dt = p.max_step;
-    if (dt < p.min_step) atomicOr(flag, 1u);
+    if (dt < p.min_step) flag |= 1u;
     const double ti_step = dt / p.time_interval;
-    if (!(ti_step > 0.0)) atomicOr(flag, 2u);
+    if (!(ti_step > 0.0)) flag |= 2u;
     int64_t ti_min = p.time_base;
     while ((double)ti_min > ti_step && ti_min > 0) ti_min >>= 1;
     return ti_min;
@@ -67,8 +66,10 @@ __global__ void k_init_timesteps(const double *__restrict__ ax, const double *__
                                  int64_t *__restrict__ tb, unsigned *flag) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    te[i] = get_timestep_dev(ax[i], ay[i], az[i], h[i], p, flag);
+    unsigned f = 0;
+    te[i] = get_timestep_dev(ax[i], ay[i], az[i], h[i], p, f);
     tb[i] = 0;
+    if (f) atomicOr(flag, f);
 }
 
 template <typename T>
@@ -83,28 +84,6 @@ __global__ void k_adaptive_half_kick(T *__restrict__ vx, T *__restrict__ vy, T *
     vx[i] += (T)(ax[i] * c);
     vy[i] += (T)(ay[i] * c);
     vz[i] += (T)(az[i] * c);
-}
-
-template <typename T>
-__global__ void k_adaptive_advance(T *__restrict__ vx, T *__restrict__ vy, T *__restrict__ vz,
-                                   const double *__restrict__ ax, const double *__restrict__ ay,
-                                   const double *__restrict__ az, const double *__restrict__ h,
-                                   int64_t *__restrict__ te, int64_t *__restrict__ tb, int64_t n,
-                                   int64_t t_int, AdaptParams p, unsigned *flag) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || te[i] != t_int) return;
-    int64_t ti_step = get_timestep_dev(ax[i], ay[i], az[i], h[i], p, flag);
-    if (t_int == p.time_base) ti_step = 0;
-    if (p.time_base - t_int < ti_step) ti_step = p.time_base - t_int;
-    const double tstart = (double)(tb[i] + te[i]) / 2.0;
-    const double tend = (double)te[i] + 0.5 * (double)ti_step;
-    const double dt = (tend - tstart) * p.time_interval;
-    vx[i] += (T)(ax[i] * dt);
-    vy[i] += (T)(ay[i] * dt);
-    vz[i] += (T)(az[i] * dt);
-    const int64_t beg = te[i];
-    tb[i] = beg;
-    te[i] = beg + ti_step;
 }
 
 template <typename T>
@@ -124,74 +103,134 @@ __global__ void k_adaptive_drift(T *__restrict__ x, T *__restrict__ y, T *__rest
 // (time_base, 0), so an empty range leaves (time_base, 0).
 constexpr int MINRED_BLOCKS = 256;
 
-__device__ __forceinline__ void min_count_block(int64_t m, int64_t k, int64_t *sm, int64_t *sk) {
-    const int t = threadIdx.x;
-    sm[t] = m;
-    sk[t] = k;
+struct MinCount {
+    int64_t m, k;
+};
+__device__ __forceinline__ void add_step(MinCount &r, int64_t v) {
+    if (v < r.m) {
+        r.m = v;
+        r.k = 1;
+    } else if (v == r.m) {
+        ++r.k;
+    }
+}
+
+// A block's (min, count, error flags), written to its slot of the pinned host
+// array that the host combines after its one wait per block step.
+__device__ __forceinline__ void store_min_count(MinCount r, unsigned flags, int64_t *__restrict__ out) {
+    __shared__ int64_t sm[4], sk[4];
+    __shared__ unsigned sf[4];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const int64_t m2 = __shfl_xor(r.m, off, 64), k2 = __shfl_xor(r.k, off, 64);
+        const int64_t mm = m2 < r.m ? m2 : r.m;
+        r.k = (r.m == mm ? r.k : 0) + (m2 == mm ? k2 : 0);
+        r.m = mm;
+        flags |= (unsigned)__shfl_xor((int)flags, off, 64);
+    }
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) { sm[w] = r.m; sk[w] = r.k; sf[w] = flags; }
     __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if (t < off) {
-            const int64_t m1 = sm[t], m2 = sm[t + off];
-            const int64_t mm = m2 < m1 ? m2 : m1;
-            sk[t] = (m1 == mm ? sk[t] : 0) + (m2 == mm ? sk[t + off] : 0);
-            sm[t] = mm;
-        }
-        __syncthreads();
+    if (threadIdx.x != 0) return;
+    int64_t mm = sm[0], kk = 0;
+    unsigned f = 0;
+#pragma unroll
+    for (int q = 1; q < 4; ++q) mm = sm[q] < mm ? sm[q] : mm;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        kk += sm[q] == mm ? sk[q] : 0;
+        f |= sf[q];
     }
+    out[3 * blockIdx.x] = mm;
+    out[3 * blockIdx.x + 1] = kk;
+    out[3 * blockIdx.x + 2] = (int64_t)f;
 }
 
-__global__ __launch_bounds__(256) void k_min_count_part(const int64_t *__restrict__ te, int64_t n,
-                                                        int64_t base, int64_t *__restrict__ part) {
-    __shared__ int64_t sm[256], sk[256];
-    int64_t m = base, k = 0;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-        const int64_t v = te[i];
-        if (v < m) {
-            m = v;
-            k = 1;
-        } else if (v == m) {
-            ++k;
-        }
-    }
-    min_count_block(m, k, sm, sk);
-    if (threadIdx.x == 0) {
-        part[2 * blockIdx.x] = sm[0];
-        part[2 * blockIdx.x + 1] = sk[0];
-    }
+__global__ __launch_bounds__(256) void k_min_count(const int64_t *__restrict__ te, int64_t n, int64_t base,
+                                                   int64_t *__restrict__ out) {
+    MinCount r{base, 0};
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+        add_step(r, te[i]);
+    store_min_count(r, 0, out);
 }
 
-// out = (minimum, count, error flag of the last kernel that set it)
-__global__ __launch_bounds__(256) void k_min_count_final(const int64_t *__restrict__ part, int nb,
-                                                         int64_t base,
-                                                         const unsigned *__restrict__ flag,
-                                                         int64_t *__restrict__ out) {
-    __shared__ int64_t sm[256], sk[256];
-    const int t = threadIdx.x;
-    const bool in = t < nb;
-    min_count_block(in ? part[2 * t] : base, in ? part[2 * t + 1] : 0, sm, sk);
-    if (t == 0) {
-        out[0] = sm[0];
-        out[1] = sk[0];
-        out[2] = (int64_t)*flag;
-    }
-}
-
-__global__ void k_active_flags(const int64_t *__restrict__ te, int64_t n, int64_t t_int,
-                               uint8_t *__restrict__ flags) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    flags[i] = te[i] == t_int ? 1 : 0;
-}
-
+// The active particles' kick and new steps, and the minimum and count of the
+// timeline that results, in one pass.
 template <typename T>
-__global__ void k_gather_targets(const T *__restrict__ x, const T *__restrict__ y,
-                                 const T *__restrict__ z, const double *__restrict__ h,
-                                 const int64_t *__restrict__ idx, const int64_t *__restrict__ cnt,
-                                 T *__restrict__ gx, T *__restrict__ gy, T *__restrict__ gz,
-                                 double *__restrict__ gh) {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= *cnt) return;
-    const int64_t i = idx[k];
+__global__ __launch_bounds__(256) void k_adaptive_advance(
+    T *__restrict__ vx, T *__restrict__ vy, T *__restrict__ vz, const double *__restrict__ ax,
+    const double *__restrict__ ay, const double *__restrict__ az, const double *__restrict__ h,
+    int64_t *__restrict__ te, int64_t *__restrict__ tb, int64_t n, int64_t t_int, AdaptParams p,
+    int64_t *__restrict__ out) {
+    MinCount r{p.time_base, 0};
+    unsigned flags = 0;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        int64_t end = te[i];
+        if (end == t_int) {
+            int64_t ti_step = get_timestep_dev(ax[i], ay[i], az[i], h[i], p, flags);
+            if (t_int == p.time_base) ti_step = 0;
+            if (p.time_base - t_int < ti_step) ti_step = p.time_base - t_int;
+            const double tstart = (double)(tb[i] + end) / 2.0;
+            const double tend = (double)end + 0.5 * (double)ti_step;
+            const double dt = (tend - tstart) * p.time_interval;
+            vx[i] += (T)(ax[i] * dt);
+            vy[i] += (T)(ay[i] * dt);
+            vz[i] += (T)(az[i] * dt);
+            tb[i] = end;
+            end += ti_step;
+            te[i] = end;
+        }
+        add_step(r, end);
+    }
+    store_min_count(r, flags, out);
+}
+
+// Active particles of each 256 (Morton-ordered) ones: the ballots of their
+// waves and their count.
+__global__ __launch_bounds__(256) void k_active_masks(const int64_t *__restrict__ te, int64_t n, int64_t t_int,
+                                                      uint64_t *__restrict__ mask, int *__restrict__ count) {
+    __shared__ int c[4];
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const uint64_t b = __builtin_amdgcn_ballot_w64(i < n && te[i] == t_int);
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+        mask[(int64_t)blockIdx.x * 4 + w] = b;
+        c[w] = __popcll(b);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) count[blockIdx.x] = c[0] + c[1] + c[2] + c[3];
+}
+
+// The active particles in order, gathered as targets.  Every block adds up the
+// counts of the blocks before it (a few KB in L2 at the sizes in use), so the
+// ordered compaction takes this launch and k_active_masks: with a device-wide
+// select in between a block step had four more launches.
+template <typename T>
+__global__ __launch_bounds__(256) void k_gather_active(
+    const T *__restrict__ x, const T *__restrict__ y, const T *__restrict__ z, const double *__restrict__ h,
+    int64_t n, const uint64_t *__restrict__ mask, const int *__restrict__ count, int64_t *__restrict__ idx,
+    int64_t *__restrict__ total, T *__restrict__ gx, T *__restrict__ gy, T *__restrict__ gz,
+    double *__restrict__ gh) {
+    __shared__ int64_t part[4];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int64_t before = 0;
+    for (int b = threadIdx.x; b < (int)blockIdx.x; b += 256) before += count[b];
+    before = wave_sum(before);
+    if (lane == 0) part[w] = before;
+    __syncthreads();
+    int64_t k = part[0] + part[1] + part[2] + part[3];
+    const uint64_t *m = mask + (int64_t)blockIdx.x * 4;
+    uint64_t mine = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        if (q < w) k += __popcll(m[q]);
+        if (q == w) mine = m[q];
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 255) *total = k + __popcll(mine);
+    if (!((mine >> lane) & 1)) return;
+    k += __popcll(mine & ((1ull << lane) - 1));
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    idx[k] = i;
     gx[k] = x[i];
     gy[k] = y[i];
     gz[k] = z[i];
@@ -200,10 +239,10 @@ __global__ void k_gather_targets(const T *__restrict__ x, const T *__restrict__ 
 
 __global__ void k_scatter_acc(const double *__restrict__ gax, const double *__restrict__ gay,
                               const double *__restrict__ gaz, const int64_t *__restrict__ idx,
-                              const int64_t *__restrict__ cnt, double *__restrict__ ax,
+                              int64_t na, double *__restrict__ ax,
                               double *__restrict__ ay, double *__restrict__ az) {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= *cnt) return;
+    if (k >= na) return;
     const int64_t i = idx[k];
     ax[i] = gax[k];
     ay[i] = gay[k];
@@ -247,7 +286,7 @@ int check_adaptive(nb_ctx *c) {
         set_error("no particle data uploaded");
         return NB_ERR_STATE;
     }
-    if (!c->ti_end) {
+    if (!c->ad.red) {
         set_error("adaptive timesteps not initialised (call nb_adaptive_init)");
         return NB_ERR_STATE;
     }
@@ -271,18 +310,26 @@ int read_flag(nb_ctx *c) {
     return flag_error(c, f);
 }
 
-// (minimum end step, particles at it, error flag) of the current timeline, in
-// one copy and one wait.
-int reduce_steps(nb_ctx *c, int64_t (&r)[3]) {
-    hipStream_t s = c->stream;
-    const int nb = (int)std::min<int64_t>(MINRED_BLOCKS, std::max<int64_t>(1, (c->n + 255) / 256));
-    k_min_count_part<<<nb, 256, 0, s>>>(c->ti_end, c->n, c->ad.time_base, c->ad.red);
-    NB_TRY(launch_ok("k_min_count_part"));
-    k_min_count_final<<<1, 256, 0, s>>>(c->ad.red, nb, c->ad.time_base, c->flag,
-                                        c->ad.red + 2 * MINRED_BLOCKS);
-    NB_TRY(launch_ok("k_min_count_final"));
-    NB_HIP(hipMemcpyAsync(r, c->ad.red + 2 * MINRED_BLOCKS, sizeof r, hipMemcpyDeviceToHost, s));
-    NB_HIP(hipStreamSynchronize(s));
+int min_blocks(const nb_ctx *c) {
+    return (int)std::min<int64_t>(MINRED_BLOCKS, std::max<int64_t>(1, (c->n + 255) / 256));
+}
+
+// (minimum end step, particles at it, error flags) from the blocks' slots, once
+// the kernel that wrote them has run.
+int read_steps(nb_ctx *c, int64_t (&r)[3]) {
+    NB_HIP(hipStreamSynchronize(c->stream));
+    r[0] = c->ad.time_base;
+    r[1] = r[2] = 0;
+    for (int b = 0; b < min_blocks(c); ++b) {
+        const int64_t *p = c->ad.red + 3 * b;
+        if (p[0] < r[0]) {
+            r[0] = p[0];
+            r[1] = p[1];
+        } else if (p[0] == r[0]) {
+            r[1] += p[1];
+        }
+        r[2] |= p[2];
+    }
     return NB_OK;
 }
 
@@ -314,20 +361,18 @@ int nb_adaptive_init(nb_ctx *c, double time_interval, int64_t time_base, double 
     c->ad.min_step = min_step;
     c->ad.max_step = max_step;
     const size_t n = (size_t)std::max<int64_t>(c->n, 1);
-    if (!c->ti_end) {
+    if (!c->ad.red) {   // (the last of the allocations: a call that failed among them starts over)
+        dfree(c->ti_end); dfree(c->ti_beg);
+        dfree(c->ad.mask); dfree(c->ad.count); dfree(c->ad.idx); dfree(c->ad.cnt); dfree(c->ad.buf);
         NB_TRY(dalloc(&c->ti_end, sizeof(int64_t) * n));
         NB_TRY(dalloc(&c->ti_beg, sizeof(int64_t) * n));
-        NB_TRY(dalloc(&c->ad.flags, n));
+        const size_t nblk = (n + 255) / 256;
+        NB_TRY(dalloc(&c->ad.mask, sizeof(uint64_t) * 4 * nblk));
+        NB_TRY(dalloc(&c->ad.count, sizeof(int) * nblk));
         NB_TRY(dalloc(&c->ad.idx, sizeof(int64_t) * n));
         NB_TRY(dalloc(&c->ad.cnt, sizeof(int64_t) * 2));
-        NB_TRY(dalloc(&c->ad.red, sizeof(int64_t) * (2 * MINRED_BLOCKS + 3)));
         NB_TRY(dalloc(&c->ad.buf, sizeof(double) * 7 * n));
-        size_t bytes = 0;
-        rocprim::counting_iterator<int64_t> it(0);
-        NB_HIP(rocprim::select(nullptr, bytes, it, c->ad.flags, c->ad.idx, c->ad.cnt, (size_t)n,
-                               c->stream));
-        NB_TRY(dalloc(&c->ad.tmp, bytes));
-        c->ad.tmp_bytes = bytes;
+        NB_HIP(hipHostMalloc((void **)&c->ad.red, sizeof(int64_t) * 3 * MINRED_BLOCKS, hipHostMallocDefault));
     }
     NB_HIP(hipMemsetAsync(c->flag, 0, sizeof(unsigned), c->stream));
     if (c->n > 0) {
@@ -365,7 +410,9 @@ int nb_adaptive_min_endstep(nb_ctx *c, int64_t *min_endstep) {
     // after a kick the reduction has already been read back with its flag
     if (!c->ad.next_valid) {
         int64_t r[3];
-        NB_TRY(reduce_steps(c, r));
+        k_min_count<<<min_blocks(c), 256, 0, c->stream>>>(c->ti_end, c->n, c->ad.time_base, c->ad.red);
+        NB_TRY(launch_ok("k_min_count"));
+        NB_TRY(read_steps(c, r));
         c->ad.next_min = r[0];
         c->ad.next_count = r[1];
         c->ad.next_valid = true;
@@ -397,72 +444,88 @@ int nb_adaptive_compute_force(nb_ctx *c, int64_t t_int, int64_t *nactive) {
     }
     hipStream_t s = c->stream;
     const int64_t n = c->n;
-    // ordered compaction of the active particles (deterministic)
-    k_active_flags<<<gridn(n), 256, 0, s>>>(c->ti_end, n, t_int, c->ad.flags);
-    NB_TRY(launch_ok("k_active_flags"));
-    size_t bytes = c->ad.tmp_bytes;
-    rocprim::counting_iterator<int64_t> it(0);
-    NB_HIP(rocprim::select(c->ad.tmp, bytes, it, c->ad.flags, c->ad.idx, c->ad.cnt, (size_t)n, s));
     // The count is known without a wait when t_int is the minimum end step
     // reduced since Ti_endstep last changed (the usual block step); the
     // kernels below read the device count, which equals it.
-    int64_t na = 0;
-    if (c->ad.next_valid && t_int == c->ad.next_min) {
-        na = c->ad.next_count;
-    } else {
-        NB_HIP(hipMemcpyAsync(&na, c->ad.cnt, sizeof na, hipMemcpyDeviceToHost, s));
-        NB_HIP(hipStreamSynchronize(s));
+    int64_t na = -1;
+    if (c->ad.next_valid && t_int == c->ad.next_min) na = c->ad.next_count;
+    if (na == n) {   // everyone active: the plain path
+        if (nactive) *nactive = na;
+        return ctx_run_force(c, false, true);
     }
-    if (nactive) *nactive = na;
-    if (na == 0) return NB_OK;
-    if (na == n) return ctx_run_force(c, false, true);   // everyone active: the plain path
+    // ordered compaction of the active particles (deterministic)
+    const unsigned nblk_n = gridn(n);
+    k_active_masks<<<nblk_n, 256, 0, s>>>(c->ti_end, n, t_int, c->ad.mask, c->ad.count);
+    NB_TRY(launch_ok("k_active_masks"));
     double *gh = c->ad.buf;
     double *gax = gh + n, *gay = gax + n, *gaz = gay + n;
     void *gx = gaz + n;
     void *gy = (char *)gx + (c->is_double ? 8 : 4) * (size_t)n;
     void *gz = (char *)gy + (c->is_double ? 8 : 4) * (size_t)n;
-    NB_TRY(launch_tile_boxes(c->x, c->y, c->z, c->is_double, n, c->h, 0.0, c->tile_box, c->sub_box, s));
     if (c->is_double)
-        k_gather_targets<double><<<gridn(na), 256, 0, s>>>(
-            (const double *)c->x, (const double *)c->y, (const double *)c->z, c->h, c->ad.idx,
-            c->ad.cnt, (double *)gx, (double *)gy, (double *)gz, gh);
+        k_gather_active<double><<<nblk_n, 256, 0, s>>>(
+            (const double *)c->x, (const double *)c->y, (const double *)c->z, c->h, n, c->ad.mask, c->ad.count,
+            c->ad.idx, c->ad.cnt, (double *)gx, (double *)gy, (double *)gz, gh);
     else
-        k_gather_targets<float><<<gridn(na), 256, 0, s>>>(
-            (const float *)c->x, (const float *)c->y, (const float *)c->z, c->h, c->ad.idx,
-            c->ad.cnt, (float *)gx, (float *)gy, (float *)gz, gh);
-    NB_TRY(launch_ok("k_gather_targets"));
-    // Few active targets still fill the GPU: split the sources into segments
-    // (partials reduced in a fixed order) for about 4096 blocks.
+        k_gather_active<float><<<nblk_n, 256, 0, s>>>(
+            (const float *)c->x, (const float *)c->y, (const float *)c->z, c->h, n, c->ad.mask, c->ad.count,
+            c->ad.idx, c->ad.cnt, (float *)gx, (float *)gy, (float *)gz, gh);
+    NB_TRY(launch_ok("k_gather_active"));
+    if (na < 0) {
+        NB_HIP(hipMemcpyAsync(&na, c->ad.cnt, sizeof na, hipMemcpyDeviceToHost, s));
+        NB_HIP(hipStreamSynchronize(s));
+    }
+    if (nactive) *nactive = na;
+    if (na == 0) return NB_OK;
+    if (na == n) return ctx_run_force(c, false, true);
+    NB_TRY(launch_tile_boxes(c->x, c->y, c->z, c->is_double, n, c->h, 0.0, c->tile_box, c->sub_box, s));
+    // Few active targets still fill the GPU: the sources are split into segments
+    // (partials reduced in a fixed order).  Below 2^14 targets the matrix-core
+    // path gives way to the wavefront kernel, whose segments go down to one
+    // quarter: 20 targets among 60000 took 52 us in 59 blocks, 8.7 us here.
+    // Above, about 16384 blocks even out the last round (4180 blocks on the 1024
+    // that fit: five rounds for four), with the target geometry stored once.
     const int64_t nblk = (na + BS - 1) / BS;
-    const int64_t want = std::min<int64_t>((4096 + nblk - 1) / nblk, 64);
-    const int far = c->is_double || c->tun.far_path == FAR_MFMA_BF16 ? c->tun.far_path : FAR_VALU;
+    int far = c->is_double || c->tun.far_path == FAR_MFMA_BF16 ? c->tun.far_path : FAR_VALU;
+    if (far == FAR_MFMA_BF16 && na < (1 << 14)) far = FAR_VALU;
     const Geometry g = c->mode != NB_MODE_FP64 && wave_path(far, 1, false, true)
-                           ? wave_launch_geometry(na, n, 1) : geometry(na, n, 1, want);
+                           ? wave_launch_geometry(na, n, 1, 256)
+                           : geometry(na, n, 1, std::min<int64_t>((16384 + nblk - 1) / nblk, 64));
     const int nseg = g.nseg;
-    NB_TRY(ctx_ensure_part(c, nseg));
+    // (the buffer holds part_cap segments of n targets)
+    NB_TRY(ctx_ensure_part(c, (int)std::max<int64_t>((na * nseg + n - 1) / n, 2)));
+    const bool central = c->mode == NB_MODE_SPLIT_CENTRAL && c->ncentral > 0;
+    // the segments' sums go straight to the particles when nothing follows
+    const bool direct = nseg > 1 && !central && c->bg.empty() && !(c->mond_acc0 > 0.0);
+    auto common = [&](auto &a) {
+        a.th = gh; a.nt = na; a.ns = n;
+        a.tile_box = c->tile_box; a.sub_box = c->sub_box;
+        a.nseg = nseg; a.seg_len = g.seg_len; a.nblk_i = g.nblk_i; a.wave_split = g.wave_split; a.G = c->G;
+        a.ax = gax; a.ay = gay; a.az = gaz; a.pot = nullptr; a.part = c->part;
+        if (nblk * nseg >= 2048) {
+            a.tgeo = c->tgeo;
+            a.tbg = c->tbg;
+            a.nflag = c->nflag_cap >= (size_t)(nblk * nseg * NW) ? c->nflag : nullptr;
+        }
+    };
+    if (far_path_weighted(far) && c->mode != NB_MODE_FP64) NB_TRY(ctx_ensure_source_weights(c));
     if (c->is_double) {
         ForceArgs<double> a{};
+        common(a);
         a.tx = (const double *)gx; a.ty = (const double *)gy; a.tz = (const double *)gz;
-        a.th = gh; a.nt = na;
         a.sx = (const double *)c->x; a.sy = (const double *)c->y; a.sz = (const double *)c->z;
-        a.sm = (const double *)c->m; a.ns = n;
-        a.tile_box = c->tile_box; a.sub_box = c->sub_box; a.use_origin = 1;
-        a.nseg = nseg; a.seg_len = g.seg_len; a.nblk_i = g.nblk_i; a.G = c->G;
-        a.ax = gax; a.ay = gay; a.az = gaz; a.pot = nullptr; a.part = c->part;
-        a.skip_src = (c->mode == NB_MODE_SPLIT_CENTRAL && c->ncentral > 0) ? c->central : nullptr;
+        a.sm = (const double *)c->m;
+        a.use_origin = 1;
+        a.skip_src = central ? c->central : nullptr;
         if (c->mode == NB_MODE_FP64) {
             NB_TRY(launch_force_f64(a, false, s));
         } else {
-            // the context's far path (one target per lane here), with the
-            // source weights that the weighted and matrix-core paths read
-            if (far_path_weighted(far)) {
-                NB_TRY(launch_source_weights(c->m, true, n, c->wsrc, s));
-                a.sw = c->wsrc;
-            }
+            if (far_path_weighted(far)) a.sw = c->wsrc;
             NB_TRY(launch_force_split(a, 1, false, s, far));
         }
-        if (nseg > 1) NB_TRY(launch_finalize(c->part, nseg, na, c->G, gax, gay, gaz, nullptr, false, s));
-        if (c->mode == NB_MODE_SPLIT_CENTRAL && c->ncentral > 0) {
+        if (nseg > 1 && !direct)
+            NB_TRY(launch_finalize(c->part, nseg, na, c->G, gax, gay, gaz, nullptr, false, s));
+        if (central) {
             // FP64 central terms for the active targets
             ForceArgs<double> b = a;
             b.sx = c->cx; b.sy = c->cy; b.sz = c->cz; b.sm = c->cm; b.ns = c->ncentral;
@@ -474,26 +537,24 @@ int nb_adaptive_compute_force(nb_ctx *c, int64_t t_int, int64_t *nactive) {
         }
     } else {
         ForceArgs<float> a{};
+        common(a);
         a.tx = (const float *)gx; a.ty = (const float *)gy; a.tz = (const float *)gz;
-        a.th = gh; a.nt = na;
         a.sx = (const float *)c->x; a.sy = (const float *)c->y; a.sz = (const float *)c->z;
-        a.sm = (const float *)c->m; a.ns = n;
-        a.tile_box = c->tile_box; a.sub_box = c->sub_box; a.use_origin = 0;
-        a.nseg = nseg; a.seg_len = g.seg_len; a.nblk_i = g.nblk_i; a.G = c->G;
-        a.ax = gax; a.ay = gay; a.az = gaz; a.pot = nullptr; a.part = c->part;
-        if (far == FAR_MFMA_BF16) {
-            NB_TRY(launch_source_weights(c->m, false, n, c->wsrc, s));
-            a.sw = c->wsrc;
-        }
+        a.sm = (const float *)c->m;
+        a.use_origin = 0;
+        if (far == FAR_MFMA_BF16) a.sw = c->wsrc;
         NB_TRY(launch_force_f32(a, 1, false, s, true, far));
-        if (nseg > 1) NB_TRY(launch_finalize(c->part, nseg, na, c->G, gax, gay, gaz, nullptr, false, s));
+        if (nseg > 1 && !direct)
+            NB_TRY(launch_finalize(c->part, nseg, na, c->G, gax, gay, gaz, nullptr, false, s));
     }
+    if (direct)
+        return launch_finalize(c->part, nseg, na, c->G, c->ax, c->ay, c->az, nullptr, false, s, true, c->ad.idx);
     // post-processing of the active targets, in the order of
     // src/base/PostProcessing/Force.jl:33-46: background fields, then MOND
     for (const BgField &f : c->bg)
         NB_TRY(background(gx, gy, gz, na, c->is_double, f, gax, gay, gaz, nullptr, s));
     if (c->mond_acc0 > 0.0) NB_TRY(mond(gax, gay, gaz, na, c->mond_acc0, c->mond_index, s));
-    k_scatter_acc<<<gridn(na), 256, 0, s>>>(gax, gay, gaz, c->ad.idx, c->ad.cnt, c->ax, c->ay, c->az);
+    k_scatter_acc<<<gridn(na), 256, 0, s>>>(gax, gay, gaz, c->ad.idx, na, c->ax, c->ay, c->az);
     NB_TRY(launch_ok("k_scatter_acc"));
     return NB_OK;
 }
@@ -503,17 +564,17 @@ int nb_adaptive_kick(nb_ctx *c, int64_t t_int) {
     if (c->n == 0) return NB_OK;
     c->ad.next_valid = false;
     if (c->is_double)
-        k_adaptive_advance<double><<<gridn(c->n), 256, 0, c->stream>>>(
+        k_adaptive_advance<double><<<min_blocks(c), 256, 0, c->stream>>>(
             (double *)c->vx, (double *)c->vy, (double *)c->vz, c->ax, c->ay, c->az, c->h, c->ti_end,
-            c->ti_beg, c->n, t_int, params_of(c), c->flag);
+            c->ti_beg, c->n, t_int, params_of(c), c->ad.red);
     else
-        k_adaptive_advance<float><<<gridn(c->n), 256, 0, c->stream>>>(
+        k_adaptive_advance<float><<<min_blocks(c), 256, 0, c->stream>>>(
             (float *)c->vx, (float *)c->vy, (float *)c->vz, c->ax, c->ay, c->az, c->h, c->ti_end,
-            c->ti_beg, c->n, t_int, params_of(c), c->flag);
+            c->ti_beg, c->n, t_int, params_of(c), c->ad.red);
     NB_TRY(launch_ok("k_adaptive_advance"));
-    // the new timeline's next sync point comes back with the error flag
+    // the new timeline's next sync point comes back with the error flags
     int64_t r[3];
-    NB_TRY(reduce_steps(c, r));
+    NB_TRY(read_steps(c, r));
     NB_TRY(flag_error(c, (unsigned)r[2]));
     c->ad.next_min = r[0];
     c->ad.next_count = r[1];

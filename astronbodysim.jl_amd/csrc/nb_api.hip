@@ -284,6 +284,7 @@ int run_force(nb_ctx *c, bool with_pot, bool allow_timing, bool allow_sort = tru
         a.nflag = c->nflag_cap >= (size_t)g.nblk_i * (size_t)g.nseg * NW ? c->nflag : nullptr;
         a.use_origin = 1;
         a.nseg = g.nseg; a.seg_len = g.seg_len; a.nblk_i = g.nblk_i;
+        a.wave_split = g.wave_split;
         a.G = c->G;
         a.ax = c->ax; a.ay = c->ay; a.az = c->az; a.pot = c->pot;
         a.part = c->part;
@@ -309,6 +310,7 @@ int run_force(nb_ctx *c, bool with_pot, bool allow_timing, bool allow_sort = tru
         a.nflag = c->nflag_cap >= (size_t)g.nblk_i * (size_t)g.nseg * NW ? c->nflag : nullptr;
         a.use_origin = 0;
         a.nseg = g.nseg; a.seg_len = g.seg_len; a.nblk_i = g.nblk_i;
+        a.wave_split = g.wave_split;
         a.G = c->G;
         a.ax = c->ax; a.ay = c->ay; a.az = c->az; a.pot = c->pot;
         a.part = c->part;
@@ -397,6 +399,7 @@ int ctx_run_force(nb_ctx *c, bool with_pot, bool allow_timing) {
 int ctx_rebuild_central(nb_ctx *c) { return rebuild_central(c); }
 int ctx_gather_central(nb_ctx *c) { return gather_central(c); }
 void ctx_drop_graph(nb_ctx *c) { drop_graph(c); }
+int ctx_ensure_source_weights(nb_ctx *c) { return ensure_source_weights(c); }
 int ctx_ensure_part(nb_ctx *c, int nseg) { return ensure_part(c, nseg); }
 }  // namespace nb
 
@@ -538,8 +541,8 @@ int nb_destroy(nb_ctx *c) {
     dfree(c->time); dfree(c->flag); dfree(c->central);
     dfree(c->cx); dfree(c->cy); dfree(c->cz); dfree(c->cm); dfree(c->cidx);
     dfree(c->ti_end); dfree(c->ti_beg);
-    dfree(c->ad.flags); dfree(c->ad.idx); dfree(c->ad.cnt); dfree(c->ad.red); dfree(c->ad.buf);
-    dfree(c->ad.tmp);
+    dfree(c->ad.mask); dfree(c->ad.count); dfree(c->ad.idx); dfree(c->ad.cnt); dfree(c->ad.buf);
+    if (c->ad.red) (void)hipHostFree(c->ad.red);
     sort_free(c);
     snapshot_free(c);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -705,7 +708,7 @@ constexpr size_t PROBE_KEEP_BYTES = (size_t)64 << 20;
 // blocks.  One segment left 252 of the 256 CUs idle: 1009 points in 200003
 // particles took 12.2 ms a call, 0.19 ms in 782 segments.
 // (The FP32-pair kernels: at most PROBE_SEGMENTS.)
-constexpr int PROBE_SEGMENTS = 1024;
+constexpr int PROBE_SEGMENTS = 512;
 static int probe_segments(int64_t npts, int64_t n) {
     const int64_t nblk = (npts + BS - 1) / BS;
     return (int)std::min<int64_t>((4096 + nblk - 1) / nblk, std::max<int64_t>((n + BS - 1) / BS, 1));
@@ -732,7 +735,7 @@ static int probe_points(nb_ctx *c, int64_t npts, const double *pts, double h, do
     const bool with_pot = pot != nullptr;
     const bool f64 = c->mode == NB_MODE_FP64;
     const Geometry g = f64 ? geometry(npts, c->n, 1, probe_segments(npts, c->n))
-                           : wave_launch_geometry(npts, c->n, 1, PROBE_SEGMENTS);
+                           : wave_launch_geometry(npts, c->n, 1, PROBE_SEGMENTS, true);
     // target xyz (double or float), outputs ax ay az pot, packed xyz staging and
     // the segments' partial sums
     const size_t np = (size_t)npts;
@@ -753,7 +756,7 @@ static int probe_points(nb_ctx *c, int64_t npts, const double *pts, double h, do
             a.ns = c->n;
             a.tile_box = c->tile_box; a.sub_box = c->sub_box; a.use_origin = c->is_double ? 1 : 0;
             a.part = part;
-            a.nseg = g.nseg; a.seg_len = g.seg_len; a.nblk_i = g.nblk_i; a.G = c->G;
+            a.nseg = g.nseg; a.seg_len = g.seg_len; a.nblk_i = g.nblk_i; a.wave_split = g.wave_split; a.G = c->G;
             a.ax = oax; a.ay = oay; a.az = oaz; a.pot = opot; a.accumulate = 0;
         };
         if (c->is_double) {

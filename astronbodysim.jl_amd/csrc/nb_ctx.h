@@ -28,17 +28,16 @@ struct AdaptState {
     double time_interval = 0.0;
     int64_t time_base = 0;
     double err_tol = 0.0, min_step = 0.0, max_step = 0.0;
-    uint8_t *flags = nullptr;  // active flags
+    uint64_t *mask = nullptr;  // active particles: one ballot per 64
+    int *count = nullptr;      // and their number per 256
     int64_t *idx = nullptr;    // compacted active indices
     int64_t *cnt = nullptr;    // [0] active count
-    int64_t *red = nullptr;    // end-step reduction: block partials, then (min, count, flag)
+    int64_t *red = nullptr;    // pinned host: (min, count, error flags) of each reduction block
     // (minimum end step, particles at it) of the current Ti_endstep, when
     // next_valid; read back together with the error flag after each kick
     bool next_valid = false;
     int64_t next_min = 0, next_count = 0;
     double *buf = nullptr;     // gathered targets and their accelerations (7n doubles)
-    void *tmp = nullptr;       // rocPRIM select storage
-    size_t tmp_bytes = 0;
 };
 
 // One pinned host slot of the asynchronous snapshot download (nb_snapshot.hip).
@@ -144,6 +143,7 @@ int ctx_run_force(nb_ctx *c, bool with_pot, bool allow_timing);
 int ctx_rebuild_central(nb_ctx *c);
 int ctx_gather_central(nb_ctx *c);
 void ctx_drop_graph(nb_ctx *c);
+int ctx_ensure_source_weights(nb_ctx *c);
 int ctx_ensure_part(nb_ctx *c, int nseg);
 // nb_snapshot.hip
 void snapshot_free(nb_ctx *c);

@@ -71,58 +71,83 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(MF == 4 ? 4 
     }
 }
 
-// Far path 0 with one target per lane: wave w of workgroup ib owns the targets
-// 64 (NW ib + w).. and walks the segment's sources on its own (wave_force); the
-// waves of a workgroup share the scalar cache's lines of those sources, nothing
-// else.  Held to 6 waves per SIMD (two values spilled outside the pair loops;
+// Far path 0 with one target per lane (wave_force).
+// split = 0: wave w of workgroup ib owns the targets 64 (NW ib + w).. and walks
+// the whole segment; the waves share the scalar cache's lines of its sources,
+// nothing else.
+// split = 1 (few targets): the waves share the targets 64 ib.. and take a part
+// of the segment each, down to 16 sources, and their sums meet in LDS in a
+// fixed order: the same waves on a quarter of the segments, so a quarter of the
+// partial sums to write and to add up.
+// Held to 6 waves per SIMD (two values spilled outside the pair loops;
 // 5 without): 60000 particles in FP32 986 -> 929 us a force, 30011 in split
 // precision 312 -> 308 us.  Against the block-wide kernel that it replaced (one
 // force call with its boxes and segment sums, split precision, Plummer): 1000
-// particles 32 -> 16 us, 4096 35 -> 25, 16384 130 -> 110, 30011 333 -> 308;
+// particles 32 -> 12.5 us, 4096 35 -> 22, 16384 130 -> 106, 30011 333 -> 301;
 // FP32 60000 1030 -> 929.
 template <typename T, bool ACC, bool POT>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(ACC &&POT && sizeof(T) == 8 ? 5 : 6)))
-void k_force_wave(ForceArgs<T> a) {
+void k_force_wave(ForceArgs<T> a, int split) {
+    constexpr int NV = (ACC ? 3 : 0) + (POT ? 1 : 0);
     __shared__ WaveStage<T> st[NW];
+    __shared__ double red[NW - 1][NV][64];
+    const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int logical = xcd_remap(blockIdx.x, gridDim.x);
     const int seg = logical / a.nblk_i;
     const int ib = logical - seg * a.nblk_i;
-    const int64_t i0 = (int64_t)ib * BS + wave * 64;
-    if (i0 >= a.nt) return;   // (no workgroup barrier follows)
-    const int64_t i = i0 + (threadIdx.x & 63);
+    const int64_t i0 = split ? (int64_t)ib * 64 : (int64_t)ib * BS + wave * 64;
+    if (i0 >= a.nt) return;   // (split: never)
+    const int64_t i = i0 + lane;
     const int64_t ic = i < a.nt ? i : a.nt - 1;
-    const int64_t j0 = (int64_t)seg * a.seg_len;
-    const int64_t j1 = (j0 + a.seg_len < a.ns) ? j0 + a.seg_len : a.ns;
-    double Ax, Ay, Az, Aq;
+    int64_t j0 = (int64_t)seg * a.seg_len;
+    int64_t j1 = (j0 + a.seg_len < a.ns) ? j0 + a.seg_len : a.ns;
+    if (split) {   // (segments of 1, 2 or a multiple of 4 quarters: no part starts inside a quarter and leaves it)
+        const int64_t part = a.seg_len / NW;
+        j0 = j0 + part * wave < j1 ? j0 + part * wave : j1;
+        j1 = j0 + part < j1 ? j0 + part : j1;
+    }
+    double v[4];   // ax, ay, az, pot
     wave_force<T, ACC, POT>(st[wave], a.tx[ic], a.ty[ic], a.tz[ic], a.th ? a.th[ic] : a.th_const,
                             a.tbox ? a.tbox + (i0 / 64) * 8 : nullptr, a.sx, a.sy, a.sz, a.sm, a.skip_src,
                             a.sub_box ? a.sub_box + (j0 / SB) * 8 : nullptr,
-                            a.sub_box ? nullptr : a.tile_box + (j0 / BS) * 8, j0, j1, Ax, Ay, Az, Aq);
+                            a.sub_box ? nullptr : a.tile_box + (j0 / BS) * 8, j0, j1, v[0], v[1], v[2], v[3]);
+    constexpr int V0 = ACC ? 0 : 3;
+    if (split) {
+        if (wave > 0) {
+#pragma unroll
+            for (int q = 0; q < NV; ++q) red[wave - 1][q][lane] = v[V0 + q];
+        }
+        __syncthreads();
+        if (wave > 0) return;
+#pragma unroll
+        for (int w = 0; w < NW - 1; ++w)
+#pragma unroll
+            for (int q = 0; q < NV; ++q) v[V0 + q] += red[w][q][lane];
+    }
     if (i >= a.nt) return;
     if (a.nseg == 1) {
         if (ACC) {
-            a.ax[i] = a.G * Ax;
-            a.ay[i] = a.G * Ay;
-            a.az[i] = a.G * Az;
+            a.ax[i] = a.G * v[0];
+            a.ay[i] = a.G * v[1];
+            a.az[i] = a.G * v[2];
         }
-        if (POT) a.pot[i] = -a.G * Aq;
+        if (POT) a.pot[i] = -a.G * v[3];
     } else {
         double *p = a.part + (int64_t)seg * 4 * a.nt;
-        if (ACC) {
-            p[i] = Ax;
-            p[a.nt + i] = Ay;
-            p[2 * a.nt + i] = Az;
-        }
-        if (POT) p[3 * a.nt + i] = Aq;
+#pragma unroll
+        for (int q = 0; q < NV; ++q) p[(V0 + q) * a.nt + i] = v[V0 + q];
     }
 }
 
 template <typename T>
-static void launch_wave(const ForceArgs<T> &a, int64_t nb, bool pot, bool acc, hipStream_t s) {
-    if (pot && acc) k_force_wave<T, true, true><<<(unsigned)nb, BS, 0, s>>>(a);
-    else if (pot) k_force_wave<T, false, true><<<(unsigned)nb, BS, 0, s>>>(a);
-    else k_force_wave<T, true, false><<<(unsigned)nb, BS, 0, s>>>(a);
+static void launch_wave(ForceArgs<T> a, bool pot, bool acc, hipStream_t s) {
+    const int split = a.wave_split;
+    if (split) a.nblk_i = (int)((a.nt + 63) / 64);
+    const unsigned nb = (unsigned)((int64_t)a.nblk_i * a.nseg);
+    if (pot && acc) k_force_wave<T, true, true><<<nb, BS, 0, s>>>(a, split);
+    else if (pot) k_force_wave<T, false, true><<<nb, BS, 0, s>>>(a, split);
+    else k_force_wave<T, true, false><<<nb, BS, 0, s>>>(a, split);
 }
 
 // Near pass of a split bf16 launch (forces only): one wavefront per
@@ -350,10 +375,22 @@ __device__ __forceinline__ bool sum_partials(const double *__restrict__ part, in
     for (int q = 0; q < NV; ++q) r.v[q] = 0.0;
     if (i < n) {
         const double *p = part + (ACC ? 0 : 3) * n + i;
-#pragma unroll 4
-        for (int s = w; s < nseg; s += W) {
+        // (eight segments in flight; past the end: the last one's, not added)
+        constexpr int U = 8;
+        for (int s = w; s < nseg; s += U * W) {
+            double t[U][NV];
 #pragma unroll
-            for (int q = 0; q < NV; ++q) r.v[q] += p[((int64_t)s * 4 + q) * n];
+            for (int u = 0; u < U; ++u) {
+                const int su = s + u * W < nseg ? s + u * W : nseg - 1;
+#pragma unroll
+                for (int q = 0; q < NV; ++q) t[u][q] = p[((int64_t)su * 4 + q) * n];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (s + u * W < nseg) {
+#pragma unroll
+                    for (int q = 0; q < NV; ++q) r.v[q] += t[u][q];
+                }
         }
     }
     if (w > 0) {
@@ -375,11 +412,13 @@ __device__ __forceinline__ bool sum_partials(const double *__restrict__ part, in
 template <bool ACC, bool POT, int W>
 __global__ __launch_bounds__(64 * W) void k_finalize(const double *__restrict__ part, int nseg, int64_t n, double G,
                                                      double *__restrict__ ax, double *__restrict__ ay,
-                                                     double *__restrict__ az, double *__restrict__ pot) {
+                                                     double *__restrict__ az, double *__restrict__ pot,
+                                                     const int64_t *__restrict__ idx) {
     __shared__ double red[W - 1][PartSums<ACC, POT>::NV][64];
-    const int64_t i = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
+    const int64_t k = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
     PartSums<ACC, POT> r;
-    if (!sum_partials<ACC, POT, W>(part, nseg, n, i, red, r)) return;
+    if (!sum_partials<ACC, POT, W>(part, nseg, n, k, red, r)) return;
+    const int64_t i = idx ? idx[k] : k;
     if constexpr (ACC) {
         ax[i] = G * r.v[0];
         ay[i] = G * r.v[1];
@@ -579,7 +618,7 @@ static int launch_f32_impl(ForceArgs<T> a, int tpt, bool pot, hipStream_t s, boo
         return NB_ERR_INVALID;
     }
     if (wave_path(MF, tpt, pot, acc)) {
-        launch_wave<T>(a, nb, pot, acc, s);
+        launch_wave<T>(a, pot, acc, s);
         return check_launch("k_force_wave");
     }
     NB_TRY(prepare_target_geom(a, tpt, s));
@@ -719,15 +758,15 @@ int launch_finalize_kick(const double *part, int nseg, int64_t n, double G, doub
 }
 
 int launch_finalize(const double *part, int nseg, int64_t n, double G, double *ax, double *ay,
-                    double *az, double *pot, bool with_pot, hipStream_t s, bool with_acc) {
+                    double *az, double *pot, bool with_pot, hipStream_t s, bool with_acc, const int64_t *idx) {
     if (n <= 0) return NB_OK;
     const unsigned nb = (unsigned)((n + 63) / 64);
 #define NB_FIN(A_, P_)                                                                                          \
     do {                                                                                                        \
         if (nseg > FIN_MANY)                                                                                    \
-            k_finalize<A_, P_, FIN_WAVES_MANY><<<nb, 64 * FIN_WAVES_MANY, 0, s>>>(part, nseg, n, G, ax, ay, az, pot); \
+            k_finalize<A_, P_, FIN_WAVES_MANY><<<nb, 64 * FIN_WAVES_MANY, 0, s>>>(part, nseg, n, G, ax, ay, az, pot, idx); \
         else                                                                                                    \
-            k_finalize<A_, P_, FIN_WAVES><<<nb, 64 * FIN_WAVES, 0, s>>>(part, nseg, n, G, ax, ay, az, pot);     \
+            k_finalize<A_, P_, FIN_WAVES><<<nb, 64 * FIN_WAVES, 0, s>>>(part, nseg, n, G, ax, ay, az, pot, idx);     \
     } while (0)
     if (with_pot && with_acc) NB_FIN(true, true);
     else if (with_pot) NB_FIN(false, true);

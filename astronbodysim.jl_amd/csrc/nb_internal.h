@@ -63,6 +63,7 @@ struct ForceArgs {
     int nseg;                // source segments (grid = nblk_i * nseg)
     int64_t seg_len;         // sources per segment (multiple of BS)
     int nblk_i;              // target blocks
+    int wave_split;          // k_force_wave: the waves of a workgroup share 64 targets and split the segment
     double G;
     double *ax, *ay, *az, *pot;  // final outputs (nseg == 1)
     double *part;                // partials [nseg][4][nt] (nseg > 1)
@@ -91,6 +92,7 @@ inline bool wave_path(int far_path, int tpt, bool pot, bool acc) {
 struct Geometry {
     int tpt, nseg, nblk_i;
     int64_t seg_len;
+    int wave_split = 0;
 };
 
 // Segments of whole tiles.
@@ -108,17 +110,25 @@ inline Geometry geometry(int64_t nt, int64_t ns, int tpt, int64_t want_seg) {
 
 // A k_force_wave launch: the segments are cut at quarters.  Few targets are
 // spread over more segments than asked for, up to max_seg (or one per quarter),
-// until the chip has 8 waves per SIMD (8192 waves): a wave alone on its SIMD
-// is bound by latency.
+// until the chip has about WAVE_FILL workgroups: a wave alone on its SIMD is
+// bound by latency.  Below WAVE_SPLIT_BELOW targets the four waves of a
+// workgroup share 64 targets and split the segment's sources, by whole quarters
+// only where asked (the FP32 sums of a quarter then never depend on the split).
 constexpr int WAVE_SEGMENTS = 64;
-inline Geometry wave_launch_geometry(int64_t nt, int64_t ns, int64_t want_seg, int64_t max_seg = WAVE_SEGMENTS) {
+constexpr int64_t WAVE_FILL = 2048, WAVE_SPLIT_BELOW = 32768;
+inline Geometry wave_launch_geometry(int64_t nt, int64_t ns, int64_t want_seg, int64_t max_seg = WAVE_SEGMENTS,
+                                     bool whole_quarters = false) {
     Geometry g;
     g.tpt = 1;
     g.nblk_i = (int)((nt + BS - 1) / BS);
-    const int64_t nq = std::max<int64_t>((ns + SB - 1) / SB, 1), ntw = std::max<int64_t>((nt + 63) / 64, 1);
-    const int64_t fill = std::min<int64_t>((8192 + ntw - 1) / ntw, max_seg);
+    g.wave_split = nt < WAVE_SPLIT_BELOW;
+    const int64_t nq = std::max<int64_t>((ns + SB - 1) / SB, 1);
+    const int64_t groups = std::max<int64_t>(g.wave_split ? (nt + 63) / 64 : g.nblk_i, 1);
+    if (g.wave_split) want_seg = (want_seg + NW - 1) / NW;
+    const int64_t fill = std::min<int64_t>((WAVE_FILL + groups - 1) / groups, max_seg);
     const int64_t nseg = std::min<int64_t>(std::max<int64_t>(std::max<int64_t>(want_seg, 1), fill), nq);
-    const int64_t qs = (nq + nseg - 1) / nseg;
+    int64_t qs = (nq + nseg - 1) / nseg;
+    if (g.wave_split && (qs > 2 || whole_quarters)) qs = (qs + NW - 1) / NW * NW;
     g.seg_len = qs * SB;
     g.nseg = (int)((nq + qs - 1) / qs);
     return g;
@@ -145,9 +155,10 @@ int launch_force_f64(const ForceArgs<double> &a, bool pot, hipStream_t s);
 // w_i = m_i^(-2/3) (0 for massless particles) for the weighted far paths.
 int launch_source_weights(const void *m, bool is_double, int64_t n, float *w, hipStream_t s);
 inline bool far_path_weighted(int far_path) { return far_path == FAR_WEIGHTED || far_path == FAR_MFMA_BF16; }
+// idx, when not null: target k's sums go to element idx[k].
 int launch_finalize(const double *part, int nseg, int64_t n, double G, double *ax, double *ay,
                     double *az, double *pot, bool with_pot, hipStream_t s,
-                    bool with_acc = true);
+                    bool with_acc = true, const int64_t *idx = nullptr);
 // The KDK step's drift fused with the tile boxes of the drifted positions, and
 // its kick fused with the finalize of the accelerations (same arithmetic as
 // the separate kernels).

@@ -113,6 +113,7 @@ extern "C" int nb_compute_force_noalloc(int32_t precision_mode, int64_t n, const
     a.sub_box = a.tbox = quarters ? box : nullptr;
     a.use_origin = 1;
     a.nseg = g.nseg; a.seg_len = g.seg_len; a.nblk_i = g.nblk_i;
+    a.wave_split = g.wave_split;
     a.G = G;
     a.ax = ax; a.ay = ay; a.az = az; a.pot = pot;
     a.part = part;

@@ -171,7 +171,7 @@ int morton_reorder(nb_ctx *c) {
     for (void *a : {(void *)c->h, (void *)c->ax, (void *)c->ay, (void *)c->az, (void *)c->pot}) add_array(set, a, 8, n);
     if (c->coll) add_array(set, c->coll, 1, n);
     if (c->central) add_array(set, c->central, 1, n);
-    if (c->ti_end) {
+    if (c->ad.red) {
         add_array(set, c->ti_end, 8, n);
         add_array(set, c->ti_beg, 8, n);
     }

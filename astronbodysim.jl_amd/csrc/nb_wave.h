@@ -243,10 +243,14 @@ __device__ __forceinline__ void wave_force(WaveStage<T> &st, T xt, T yt, T zt, d
             near_sources<T, false, ACC, POT>(as_scalar(sx + base), as_scalar(sy + base), as_scalar(sz + base),
                                              st.m, cnt, xt, yt, zt, t, ax, ay, az, aq);
         } else if constexpr (D) {
-#pragma unroll 4
-            for (int j = 0; j < SB; ++j) {
-                const float4 v = st.hi[j];
-                pair_f32<false, POT>(v.x, v.y, v.z, v.w, xi, yi, zi, t.h2c, t.h2, t.hinv, t.hinv3, ax, ay, az, aq);
+#pragma unroll 1
+            for (int j = 0; j < cnt; j += 4) {   // (past cnt: padding)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const float4 v = st.hi[j + g];
+                    pair_f32<false, POT>(v.x, v.y, v.z, v.w, xi, yi, zi, t.h2c, t.h2, t.hinv, t.hinv3, ax, ay, az,
+                                         aq);
+                }
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");   // read before the next staging

@@ -240,14 +240,14 @@ static int ensure_source_weights(nb_ctx *c) {
     return NB_OK;
 }
 
-// Work of a KDK step that rides on run_force's kernels: the drift has written
-// the tile boxes already (boxes_ready), and the kick of `kick` (x dt) may be
-// done by the finalize (kicked reports whether it was).
+// A KDK step around run_force: the drift has written the tile boxes already
+// (boxes_ready), and the sums of the force's segments may be left to the step's
+// k_step (left reports whether they were, with nseg segments).
 struct StepFusion {
     bool boxes_ready = false;
     int geo_ready = 0;     // the drift stored the target geometry (1), with the B operands (2)
-    double kick = 0.0;
-    bool kicked = false;
+    bool left = false;
+    int nseg = 0;
 };
 
 // pot_only: the FP32-pair kernels write the potential alone (the caller keeps
@@ -324,14 +324,14 @@ int run_force(nb_ctx *c, bool with_pot, bool allow_timing, bool allow_sort = tru
         NB_TRY(launch_force_f32(a, tpt, with_pot, s, acc_out, c->tun.far_path));
     }
     if (allow_timing) NB_TRY(record_stop(c, e0));
-    // the kick rides on the finalize when nothing else adds to the accelerations
-    const bool kick_here = fuse && !with_pot && g.nseg > 1 && c->bg.empty() && !(c->mond_acc0 > 0.0) &&
-                           !(c->mode == NB_MODE_SPLIT_CENTRAL && c->ncentral > 0);
-    if (kick_here) {
-        NB_TRY(launch_finalize_kick(c->part, g.nseg, n, c->G, c->ax, c->ay, c->az, c->vx, c->vy, c->vz,
-                                    fuse->kick, c->is_double, s));
-        fuse->kicked = true;
-    } else if (g.nseg > 1) {
+    // the step's kick takes the segments' sums (and the central bodies' terms)
+    // when nothing else adds to the accelerations
+    if (fuse && !with_pot && g.nseg > 1 && c->bg.empty() && !(c->mond_acc0 > 0.0)) {
+        fuse->left = true;
+        fuse->nseg = g.nseg;
+        return NB_OK;
+    }
+    if (g.nseg > 1) {
         NB_TRY(launch_finalize(c->part, g.nseg, n, c->G, c->ax, c->ay, c->az, c->pot, with_pot, s,
                                !(with_pot && pot_only) || f64));
     }
@@ -539,7 +539,7 @@ int nb_destroy(nb_ctx *c) {
     dfree(c->perm);
     dfree(c->tile_box); dfree(c->sub_box); dfree(c->tgeo); dfree(c->tbg); dfree(c->nflag); dfree(c->part); dfree(c->stage); dfree(c->red); dfree(c->wsrc); dfree(c->probe);
     dfree(c->time); dfree(c->flag); dfree(c->central);
-    dfree(c->cx); dfree(c->cy); dfree(c->cz); dfree(c->cm); dfree(c->cidx);
+    dfree(c->cx); dfree(c->cy); dfree(c->cz); dfree(c->cm); dfree(c->cidx); dfree(c->cstep);
     dfree(c->ti_end); dfree(c->ti_beg);
     dfree(c->ad.mask); dfree(c->ad.count); dfree(c->ad.idx); dfree(c->ad.cnt); dfree(c->ad.buf);
     if (c->ad.red) (void)hipHostFree(c->ad.red);
@@ -847,42 +847,82 @@ int nb_kick(nb_ctx *c, double dt) {
     return NB_OK;
 }
 
-// Drift (with the tile boxes of the new positions), force, kick (with the
-// finalize of the accelerations where it can).
-static int enqueue_step(nb_ctx *c, int64_t k, double dt, bool allow_timing, bool allow_sort) {
-    const int rd = (int)(k & 1), wr = 1 - rd;
-    StepFusion fuse;
-    if (c->n > 0) {
-        // The target geometry of a force call with one target per lane and
-        // several source segments rides on the drift as well, stored as that
-        // call's launch would store it (origin mode, B operands of far path 4).
-        StepGeometry sg{};
-        const StepGeometry *gp = nullptr;
-        if (c->mode != NB_MODE_FP64 && c->tun.targets_per_thread == 1 && c->tgeo &&
-            !wave_path(c->tun.far_path, 1, false, true)) {
-            const Geometry g = force_geometry(c, false, true);
-            if (g.nseg > 1) {
-                NB_TRY(ensure_part(c, g.nseg));
-                NB_TRY(ensure_tbg(c, g));
-                const bool bf16 = c->tun.far_path == FAR_MFMA_BF16;
-                sg.tgeo = c->tgeo;
-                sg.tbg = bf16 ? c->tbg : nullptr;
-                sg.use_origin = (c->is_double || bf16) ? 1 : 0;
-                gp = &sg;
-                fuse.geo_ready = sg.tbg ? 2 : 1;
-            }
-        }
-        NB_TRY(launch_drift_boxes(c->x, c->y, c->z, c->vx, c->vy, c->vz, c->n, dt, c->time, rd, wr, c->is_double,
-                                  c->h, c->tile_box, c->sub_box, c->stream, gp));
-        fuse.boxes_ready = true;
-    } else {
-        NB_TRY(drift(c->x, c->y, c->z, c->vx, c->vy, c->vz, c->n, dt, c->time, rd, wr, c->is_double,
-                     c->stream));
+// The k_step arguments of step k: its kick, or the drift that begins it.
+static int step_args(nb_ctx *c, int64_t k, double dt, StepArgs &a, int *geo_ready) {
+    a = StepArgs{};
+    a.n = c->n; a.dt = dt; a.G = c->G;
+    a.x = c->x; a.y = c->y; a.z = c->z; a.vx = c->vx; a.vy = c->vy; a.vz = c->vz; a.m = c->m; a.h = c->h;
+    a.ax = c->ax; a.ay = c->ay; a.az = c->az;
+    a.time = c->time; a.box = c->tile_box; a.sub = c->sub_box;
+    if (c->mode == NB_MODE_SPLIT_CENTRAL && c->ncentral > 0) {
+        a.ncentral = c->ncentral; a.cidx = c->cidx; a.central = c->central;
+        a.c_in = c->cstep + (k & 1) * 4 * c->ncentral;
     }
-    fuse.kick = dt;
-    NB_TRY(run_force(c, false, allow_timing, allow_sort, false, &fuse));
-    if (!fuse.kicked)
-        NB_TRY(kick(c->vx, c->vy, c->vz, c->ax, c->ay, c->az, c->n, dt, c->is_double, c->stream));
+    // The target geometry of a force call with one target per lane and several
+    // source segments rides on the drift as well, stored as that call's launch
+    // would store it (origin mode, B operands of far path 4).
+    *geo_ready = 0;
+    if (c->mode != NB_MODE_FP64 && c->tun.targets_per_thread == 1 && c->tgeo &&
+        !wave_path(c->tun.far_path, 1, false, true)) {
+        const Geometry g = force_geometry(c, false, true);
+        if (g.nseg > 1) {
+            NB_TRY(ensure_part(c, g.nseg));
+            NB_TRY(ensure_tbg(c, g));
+            const bool bf16 = c->tun.far_path == FAR_MFMA_BF16;
+            a.tgeo = c->tgeo;
+            a.tbg = bf16 ? c->tbg : nullptr;
+            a.use_origin = (c->is_double || bf16) ? 1 : 0;
+            *geo_ready = a.tbg ? 2 : 1;
+        }
+    }
+    return NB_OK;
+}
+
+// The drift that begins step k, in the arguments of a k_step launch.
+static void add_drift(nb_ctx *c, int64_t k, StepArgs &a) {
+    a.drift = 1;
+    a.rd = (int)(k & 1);
+    a.wr = 1 - a.rd;
+    a.c_out = a.ncentral > 0 ? c->cstep + (k & 1) * 4 * c->ncentral : nullptr;
+}
+
+// Steps k .. k + count - 1: drift (with the tile boxes of the new positions),
+// force, kick; one launch takes a step's kick and the next one's drift.
+static int enqueue_steps(nb_ctx *c, int64_t k, int64_t count, double dt, bool allow_timing, bool allow_sort) {
+    StepArgs a;
+    int geo_ready = 0;
+    bool drifted = false;
+    for (int64_t q = 0; q < count; ++q) {
+        const int64_t st = k + q;
+        if (c->n <= 0) {
+            NB_TRY(drift(c->x, c->y, c->z, c->vx, c->vy, c->vz, c->n, dt, c->time, (int)(st & 1), 1 - (int)(st & 1),
+                         c->is_double, c->stream));
+            continue;
+        }
+        if (!drifted) {
+            NB_TRY(step_args(c, st, dt, a, &geo_ready));
+            add_drift(c, st, a);
+            NB_TRY(launch_step(a, c->is_double, c->stream));
+        }
+        StepFusion fuse;
+        fuse.boxes_ready = true;
+        fuse.geo_ready = geo_ready;
+        NB_TRY(run_force(c, false, allow_timing, allow_sort, false, &fuse));
+        drifted = false;
+        if (fuse.left) {
+            NB_TRY(step_args(c, st, dt, a, &geo_ready));
+            a.kick = 1;
+            a.part = c->part;
+            a.nseg = fuse.nseg;
+            if (q + 1 < count) {
+                add_drift(c, st + 1, a);
+                drifted = true;
+            }
+            NB_TRY(launch_step(a, c->is_double, c->stream));
+        } else {
+            NB_TRY(kick(c->vx, c->vy, c->vz, c->ax, c->ay, c->az, c->n, dt, c->is_double, c->stream));
+        }
+    }
     return NB_OK;
 }
 
@@ -897,6 +937,7 @@ int nb_kdk_steps(nb_ctx *c, int64_t nsteps, double dt, double t_begin, int32_t u
     // Graph replay needs a static schedule: re-sorting happens between
     // graph launches, never inside one.
     const bool graph_ok = use_graph && nsteps >= 2;
+    const bool weighted = c->mode != NB_MODE_FP64 && far_path_weighted(c->tun.far_path);
     int64_t k = 0;
     if (graph_ok) {
         const int64_t chunk = std::min<int64_t>(nsteps & ~(int64_t)1, 16);
@@ -910,11 +951,9 @@ int nb_kdk_steps(nb_ctx *c, int64_t nsteps, double dt, double t_begin, int32_t u
             const Geometry g = force_geometry(c, false, true);
             NB_TRY(ensure_part(c, g.nseg));
             NB_TRY(ensure_tbg(c, g));
-            NB_TRY(ensure_source_weights(c));
+            if (weighted) NB_TRY(ensure_source_weights(c));
             NB_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-            int rc = NB_OK;
-            for (int64_t q = 0; q < chunk && rc == NB_OK; ++q)
-                rc = enqueue_step(c, q, dt, false, false);
+            const int rc = enqueue_steps(c, 0, chunk, dt, false, false);
             hipGraph_t graph = nullptr;
             hipError_t e = hipStreamEndCapture(s, &graph);
             if (rc != NB_OK) {
@@ -943,14 +982,13 @@ int nb_kdk_steps(nb_ctx *c, int64_t nsteps, double dt, double t_begin, int32_t u
         }
         for (; k + c->g_steps <= nsteps; k += c->g_steps) {
             NB_TRY(maybe_sort(c, c->g_steps));
-            NB_TRY(ensure_source_weights(c));   // after a re-sort the graph's forces need them again
+            if (weighted) NB_TRY(ensure_source_weights(c));   // after a re-sort the graph's forces need them again
             NB_HIP(hipGraphLaunch(c->gexec, s));
             c->force_calls += c->g_steps;
             c->calls_since_sort += c->g_steps;
         }
     }
-    for (; k < nsteps; ++k) NB_TRY(enqueue_step(c, k, dt, true, true));
-    return NB_OK;
+    return enqueue_steps(c, k, nsteps - k, dt, true, true);
 }
 
 int nb_energy(nb_ctx *c, double *K, double *W, double P[3], double L[3]) {
@@ -994,7 +1032,7 @@ int nb_set_central(nb_ctx *c, int64_t count) {
         return NB_ERR_STATE;
     }
     drop_graph(c);
-    dfree(c->cx); dfree(c->cy); dfree(c->cz); dfree(c->cm); dfree(c->cidx);
+    dfree(c->cx); dfree(c->cy); dfree(c->cz); dfree(c->cm); dfree(c->cidx); dfree(c->cstep);
     c->ncentral = count;
     if (count > 0) {
         NB_TRY(dalloc(&c->cx, sizeof(double) * count));
@@ -1002,6 +1040,7 @@ int nb_set_central(nb_ctx *c, int64_t count) {
         NB_TRY(dalloc(&c->cz, sizeof(double) * count));
         NB_TRY(dalloc(&c->cm, sizeof(double) * count));
         NB_TRY(dalloc(&c->cidx, sizeof(int64_t) * count));
+        NB_TRY(dalloc(&c->cstep, sizeof(double) * 8 * count));
     }
     NB_HIP(hipMemsetAsync(c->central, 0, (size_t)c->n, c->stream));
     NB_TRY(rebuild_central(c));

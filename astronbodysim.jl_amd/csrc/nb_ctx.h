@@ -88,6 +88,7 @@ struct nb_ctx {
     int64_t ncentral = 0;
     double *cx = nullptr, *cy = nullptr, *cz = nullptr, *cm = nullptr;  // compacted central sources
     int64_t *cidx = nullptr;      // internal indices of the central sources
+    double *cstep = nullptr;      // [2][4][ncentral]: their x, y, z, m from step to step (k_step)
     nb::SortState sort;
     int64_t *ti_end = nullptr, *ti_beg = nullptr;   // adaptive integer timeline (internal order)
     nb::AdaptState ad;

@@ -480,77 +480,131 @@ __global__ __launch_bounds__(BS) void k_tile_boxes(const T *__restrict__ x, cons
                    v && h ? h[j] : h_const, v, box, sub, red);
 }
 
-// A step's drift (Pos += Vel * (t_new - t_old), the operations of k_drift,
-// with block 0 publishing t_new = time[rd] + dt to time[wr]) fused with the
-// tile boxes of the drifted positions, which the next force needs.
-// GEO: the block's target geometry as k_target_geom<T, 1, ROWS> stores it
-// (the force call that follows has one target per lane and several source
-// segments), from the drifted positions.
+// The per-particle part of a KDK step, between one force launch and the next
+// (one workgroup per 256 particles): the sums of the force's segments, the
+// central bodies' FP64 terms and the kick (a.kick), then the next step's drift
+// (a.drift) with the tile boxes of the drifted positions and, with GEO, the
+// block's target geometry as k_target_geom<T, 1, ROWS> stores it.
+// Bound by launch and load latency up to 10^5 particles, hence one launch for
+// all of it: 64 steps of 1000 particles 1047 us with a launch each for the
+// sums and kick and for the drift and boxes, 968 us in one; a disc of 16001
+// with a central star (six launches a step) 1007 and 937 us per 8 steps.
+// The segments' sums are split over four groups of 256 threads and meet in
+// LDS in a fixed order; the first group does the rest.
+//   kick:  Acc = G sum (+ central terms), Vel += Acc dt
+//   drift: Pos += Vel (t_new - t_old), block 0 publishing t_new = time[rd] + dt
+//          to time[wr] (rd != wr)
+// The central bodies' terms read their positions from c_in, and the drift
+// leaves the new ones in c_out: other workgroups still read the old ones.
+constexpr int STEP_GROUPS = 4;
 template <typename T, bool GEO, bool ROWS>
-__global__ __launch_bounds__(BS) void k_drift_boxes(T *__restrict__ x, T *__restrict__ y, T *__restrict__ z,
-                                                    const T *__restrict__ vx, const T *__restrict__ vy,
-                                                    const T *__restrict__ vz, int64_t n, double dt,
-                                                    double *time, int rd, int wr, double *__restrict__ box,
-                                                    double *__restrict__ sub, const double *__restrict__ h,
-                                                    double *__restrict__ tgeo, unsigned *__restrict__ tbg,
-                                                    int use_origin, bool hilo) {
+__global__ __launch_bounds__(BS * STEP_GROUPS) void k_step(StepArgs a) {
+    __shared__ double sums[STEP_GROUPS - 1][3][BS];
     __shared__ double red[6][NW];
     __shared__ double gred[GEO ? 11 : 1][NW];
-    const int64_t j = (int64_t)blockIdx.x * BS + threadIdx.x;
-    const double t_old = time[rd];
-    const double t_new = t_old + dt;
-    if (j == 0) time[wr] = t_new;
-    const bool v = j < n;
-    T px = 0, py = 0, pz = 0;
+    const int tid = threadIdx.x & (BS - 1), grp = threadIdx.x / BS;
+    const int64_t j = (int64_t)blockIdx.x * BS + tid;
+    const bool v = j < a.n;
+    T *x = (T *)a.x, *y = (T *)a.y, *z = (T *)a.z, *vx = (T *)a.vx, *vy = (T *)a.vy, *vz = (T *)a.vz;
+    T px = 0, py = 0, pz = 0, ux = 0, uy = 0, uz = 0;
+    double ph = 0.0;
+    if (grp == 0 && v) {
+        px = x[j]; py = y[j]; pz = z[j];
+        ux = vx[j]; uy = vy[j]; uz = vz[j];
+        ph = a.h[j];
+    }
+    if (a.kick) {
+        double s[3] = {0.0, 0.0, 0.0};
+        if (v) {
+            const double *p = a.part + j;
+            constexpr int U = 4;   // segments in flight; past the end: the last one's, not added
+            for (int g = grp; g < a.nseg; g += U * STEP_GROUPS) {
+                double t[U][3];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int gu = g + u * STEP_GROUPS < a.nseg ? g + u * STEP_GROUPS : a.nseg - 1;
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) t[u][q] = p[((int64_t)gu * 4 + q) * a.n];
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (g + u * STEP_GROUPS < a.nseg) {
+#pragma unroll
+                        for (int q = 0; q < 3; ++q) s[q] += t[u][q];
+                    }
+            }
+        }
+        if (grp > 0) {
+#pragma unroll
+            for (int q = 0; q < 3; ++q) sums[grp - 1][q][tid] = s[q];
+        }
+        __syncthreads();
+        if (grp == 0 && v) {
+#pragma unroll
+            for (int g = 0; g < STEP_GROUPS - 1; ++g)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) s[q] += sums[g][q][tid];
+            double fx = a.G * s[0], fy = a.G * s[1], fz = a.G * s[2];
+            if (a.ncentral > 0) {
+                const double hinv = 1.0 / ph, hinv3 = hinv * hinv * hinv;
+                double bx = 0.0, by = 0.0, bz = 0.0, bq = 0.0;
+                const double *c = a.c_in;
+                const int64_t k = a.ncentral;
+                for (int64_t u = 0; u < k; ++u)
+                    pair_f64<false>(c[u], c[k + u], c[2 * k + u], c[3 * k + u], (double)px, (double)py, (double)pz,
+                                    ph, hinv, hinv3, bx, by, bz, bq);
+                fx += bx * a.G;
+                fy += by * a.G;
+                fz += bz * a.G;
+            }
+            a.ax[j] = fx;
+            a.ay[j] = fy;
+            a.az[j] = fz;
+            const T c = (T)a.dt;
+            ux += (T)fx * c;
+            uy += (T)fy * c;
+            uz += (T)fz * c;
+            vx[j] = ux; vy[j] = uy; vz[j] = uz;
+        }
+    }
+    if (!a.drift || grp > 0) return;   // (a barrier waits for the waves that remain)
+    const double t_old = a.time[a.rd];
+    const double t_new = t_old + a.dt;
+    if (j == 0) a.time[a.wr] = t_new;
     if (v) {
         const T d = (T)(t_new - t_old);
-        px = x[j]; py = y[j]; pz = z[j];
-        px += vx[j] * d;
-        py += vy[j] * d;
-        pz += vz[j] * d;
+        px += ux * d;
+        py += uy * d;
+        pz += uz * d;
         x[j] = px; y[j] = py; z[j] = pz;
+        if (a.ncentral > 0 && a.central[j]) {
+            for (int64_t u = 0; u < a.ncentral; ++u)
+                if (a.cidx[u] == j) {
+                    a.c_out[u] = (double)px;
+                    a.c_out[a.ncentral + u] = (double)py;
+                    a.c_out[2 * a.ncentral + u] = (double)pz;
+                    a.c_out[3 * a.ncentral + u] = (double)((const T *)a.m)[j];
+                }
+        }
     }
-    const double ph = v ? h[j] : 0.0;
-    tile_box_block((double)px, (double)py, (double)pz, ph, v, box, sub, red);
+    tile_box_block((double)px, (double)py, (double)pz, ph, v, a.box, a.sub, red);
     if constexpr (GEO) {
-        const int tid = threadIdx.x;
-        double gx[1] = {v ? (double)px : 0.0}, gy[1] = {v ? (double)py : 0.0}, gz[1] = {v ? (double)pz : 0.0};
+        double gx[1] = {(double)px}, gy[1] = {(double)py}, gz[1] = {(double)pz};
         double gh[1] = {ph};
         bool gv[1] = {v};
         BlockStats st;
-        block_stats<1>(gx, gy, gz, gh, gv, use_origin != 0, gred, st);
+        block_stats<1>(gx, gy, gz, gh, gv, a.use_origin != 0, gred, st);
         const double ox = uniform_f64(st.ox), oy = uniform_f64(st.oy), oz = uniform_f64(st.oz);
-        const WaveGeom wg = wave_geometry<1>(gx, gy, gz, gh, gv, ox, oy, oz, hilo);
-        store_target_geom(tgeo + (int64_t)blockIdx.x * TG_STRIDE, ox, oy, oz, wg, tid >> 6, tid & 63);
+        const WaveGeom wg = wave_geometry<1>(gx, gy, gz, gh, gv, ox, oy, oz, sizeof(T) == 8);
+        store_target_geom(a.tgeo + (int64_t)blockIdx.x * TG_STRIDE, ox, oy, oz, wg, tid >> 6, tid & 63);
         if constexpr (ROWS) {
             nb_bf8 Bg[4];
             target_b_operands(gx[0] - ox, gy[0] - oy, gz[0] - oz, tid & 63, Bg);
-            nb_u4v *b = reinterpret_cast<nb_u4v *>(tbg + ((int64_t)blockIdx.x * BS + tid) * 16);
+            nb_u4v *b = reinterpret_cast<nb_u4v *>(a.tbg + ((int64_t)blockIdx.x * BS + tid) * 16);
 #pragma unroll
             for (int g = 0; g < 4; ++g) b[g] = __builtin_bit_cast(nb_u4v, Bg[g]);
         }
     }
-}
-
-// k_finalize followed by the step's kick (Vel += Acc * coef, the operations
-// of k_kick) on the accelerations it has just written.
-template <typename T>
-__global__ __launch_bounds__(64 * FIN_WAVES) void k_finalize_kick(const double *__restrict__ part, int nseg, int64_t n,
-                                                      double G, double *__restrict__ ax, double *__restrict__ ay,
-                                                      double *__restrict__ az, T *__restrict__ vx,
-                                                      T *__restrict__ vy, T *__restrict__ vz, double coef) {
-    __shared__ double red[FIN_WAVES - 1][3][64];
-    const int64_t i = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
-    PartSums<true, false> r;
-    if (!sum_partials<true, false, FIN_WAVES>(part, nseg, n, i, red, r)) return;
-    const double fx = G * r.v[0], fy = G * r.v[1], fz = G * r.v[2];
-    ax[i] = fx;
-    ay[i] = fy;
-    az[i] = fz;
-    const T c = (T)coef;
-    vx[i] += (T)fx * c;
-    vy[i] += (T)fy * c;
-    vz[i] += (T)fz * c;
 }
 
 // ---------------------------------------------------------------------------
@@ -718,43 +772,20 @@ int launch_force_f64(const ForceArgs<double> &a_in, bool pot, hipStream_t s) {
     return check_launch("k_force_f64");
 }
 
-int launch_drift_boxes(void *x, void *y, void *z, const void *vx, const void *vy, const void *vz, int64_t n,
-                       double dt, double *time, int rd, int wr, int is_double, const double *h, double *box,
-                       double *sub_box, hipStream_t s, const StepGeometry *geo) {
-    if (n <= 0) return NB_OK;
-    const unsigned nt = (unsigned)((n + BS - 1) / BS);
-    const bool g = geo && geo->tgeo, r = g && geo->tbg;
-    double *tg = g ? geo->tgeo : nullptr;
-    unsigned *tb = r ? geo->tbg : nullptr;
-    const int uo = g ? geo->use_origin : 0;
-#define NB_DB(T_, G_, R_)                                                                                       \
-    k_drift_boxes<T_, G_, R_><<<nt, BS, 0, s>>>((T_ *)x, (T_ *)y, (T_ *)z, (const T_ *)vx, (const T_ *)vy,     \
-                                                (const T_ *)vz, n, dt, time, rd, wr, box, sub_box, h, tg, tb, uo, \
-                                                sizeof(T_) == 8)
-    if (is_double) {
-        if (r) NB_DB(double, true, true);
-        else if (g) NB_DB(double, true, false);
-        else NB_DB(double, false, false);
-    } else {
-        if (r) NB_DB(float, true, true);
-        else if (g) NB_DB(float, true, false);
-        else NB_DB(float, false, false);
-    }
-#undef NB_DB
-    return check_launch("k_drift_boxes");
-}
-
-int launch_finalize_kick(const double *part, int nseg, int64_t n, double G, double *ax, double *ay, double *az,
-                         void *vx, void *vy, void *vz, double coef, int is_double, hipStream_t s) {
-    if (n <= 0) return NB_OK;
-    const unsigned nb = (unsigned)((n + 63) / 64);
-    if (is_double)
-        k_finalize_kick<double><<<nb, 64 * FIN_WAVES, 0, s>>>(part, nseg, n, G, ax, ay, az, (double *)vx, (double *)vy,
-                                                   (double *)vz, coef);
-    else
-        k_finalize_kick<float><<<nb, 64 * FIN_WAVES, 0, s>>>(part, nseg, n, G, ax, ay, az, (float *)vx, (float *)vy,
-                                                  (float *)vz, coef);
-    return check_launch("k_finalize_kick");
+int launch_step(const StepArgs &a, bool is_double, hipStream_t s) {
+    if (a.n <= 0) return NB_OK;
+    const unsigned nt = (unsigned)((a.n + BS - 1) / BS), bs = BS * STEP_GROUPS;
+    const bool g = a.drift && a.tgeo, r = g && a.tbg;
+#define NB_ST(T_)                                                       \
+    do {                                                                \
+        if (r) k_step<T_, true, true><<<nt, bs, 0, s>>>(a);             \
+        else if (g) k_step<T_, true, false><<<nt, bs, 0, s>>>(a);       \
+        else k_step<T_, false, false><<<nt, bs, 0, s>>>(a);             \
+    } while (0)
+    if (is_double) NB_ST(double);
+    else NB_ST(float);
+#undef NB_ST
+    return check_launch("k_step");
 }
 
 int launch_finalize(const double *part, int nseg, int64_t n, double G, double *ax, double *ay,

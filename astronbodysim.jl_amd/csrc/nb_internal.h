@@ -159,21 +159,32 @@ inline bool far_path_weighted(int far_path) { return far_path == FAR_WEIGHTED ||
 int launch_finalize(const double *part, int nseg, int64_t n, double G, double *ax, double *ay,
                     double *az, double *pot, bool with_pot, hipStream_t s,
                     bool with_acc = true, const int64_t *idx = nullptr);
-// The KDK step's drift fused with the tile boxes of the drifted positions, and
-// its kick fused with the finalize of the accelerations (same arithmetic as
-// the separate kernels).
-// What the drift may also store for the force call that follows: the target
-// blocks' geometry (tgeo non-null; one target per lane, several segments),
-// with the bf16 B operands when tbg is non-null.
-struct StepGeometry {
-    double *tgeo;
+// The per-particle part of a KDK step (k_step): the kick of the force launch
+// before it (from its segments' partial sums) and/or the next step's drift,
+// which stores the tile boxes of the drifted positions and what else the force
+// call that follows takes from it: with tgeo the target blocks' geometry
+// (one target per lane, several segments), with tbg their bf16 B operands.
+struct StepArgs {
+    int64_t n;
+    double dt, G;
+    int kick, drift;
+    void *x, *y, *z, *vx, *vy, *vz;
+    const void *m;
+    const double *h;             // target softening lengths
+    const double *part;          // kick: [nseg][4][n]
+    int nseg;
+    double *ax, *ay, *az;
+    int64_t ncentral;            // central bodies, with FP64 terms in the kick
+    const int64_t *cidx;
+    const uint8_t *central;
+    const double *c_in;          // their x, y, z, m [4][ncentral] at the force's positions
+    double *c_out;               // and where the drift stores the new ones
+    double *time;
+    int rd, wr;
+    double *box, *sub, *tgeo;
     unsigned *tbg;
     int use_origin;
 };
-int launch_drift_boxes(void *x, void *y, void *z, const void *vx, const void *vy, const void *vz, int64_t n,
-                       double dt, double *time, int rd, int wr, int is_double, const double *h, double *box,
-                       double *sub_box, hipStream_t s, const StepGeometry *geo = nullptr);
-int launch_finalize_kick(const double *part, int nseg, int64_t n, double G, double *ax, double *ay, double *az,
-                         void *vx, void *vy, void *vz, double coef, int is_double, hipStream_t s);
+int launch_step(const StepArgs &a, bool is_double, hipStream_t s);
 
 }  // namespace nb

@@ -50,6 +50,7 @@ struct nb_batch {
     int32_t *tile_sys = nullptr;  // [ntiles]
     double *tile_box = nullptr;   // [ntiles][8]
     double *sub_box = nullptr;    // [ntiles][NQ][8] boxes of the tile quarters
+    double *tgeo = nullptr;       // [ntiles][TG_STRIDE] geometry of each tile as a target block
     // work items of the ragged kernel: (system << 32) | target tile, by cost
     int64_t nitems = 0;
     int64_t *items = nullptr;
@@ -78,3 +79,27 @@ struct nb_batch {
     int64_t tcount = 0;
     double tms = 0.0;
 };
+
+namespace nb {
+
+struct BatchArgs {
+    const int64_t *off;
+    const int64_t *tile_base;
+    const double *tile_box;
+    const double *sub_box;        // [ntiles][NQ][8]: boxes of the tile quarters
+    const double *tgeo;           // [ntiles][TG_STRIDE]: geometry of each tile as a target block
+    const double *Gs;
+    const double *x, *y, *z, *m, *h;
+    const float *w;               // source weights (weighted far paths) or nullptr
+    const uint8_t *skip_src;
+    double *ax, *ay, *az, *pot;
+    const int64_t *items;
+    int64_t nitems;
+    unsigned *counter;
+};
+
+// nb_batch_wave.hip: the FP32-pair sums of every item on far path 0 with one
+// target per lane.
+int launch_batch_wave(const BatchArgs &a, bool pot, bool acc, hipStream_t s);
+
+}  // namespace nb

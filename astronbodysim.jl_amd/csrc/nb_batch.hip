@@ -4,12 +4,14 @@
 // (src/directsum/gravity.jl:8-28 pair law with the system's softening and G;
 // constant-dt KDK as src/directsumgpu/timestep.jl:156-224):
 //
-//  * ragged path: one persistent launch of the all-pairs kernel serves every
-//    system.  The work items are (system, tile of 256*TPT targets), ordered by
-//    cost (largest systems first) and pulled from an atomic queue; each item
-//    is the same block routine as the one-system kernel (force_block), with
-//    the system's own source range, per-system Morton order, FP64 origin and
-//    hi/lo near tiles.  KDK steps are captured in HIP graphs.
+//  * ragged path: one launch of the all-pairs kernel serves every system.  The
+//    work items are (system, tile of 256*TPT targets), ordered by cost (largest
+//    systems first).  With one target per lane on far path 0 each item is four
+//    workgroups of the one-system wavefront routine (nb_batch_wave.hip); else
+//    a persistent launch pulls the items from an atomic queue and runs the
+//    one-system block routine (force_block).  Either way an item has its
+//    system's own source range, per-system Morton order and FP64 origins.
+//    KDK steps are captured in HIP graphs.
 //  * resident path (small systems): the particles stay in registers and many
 //    KDK steps run in a single launch, the sources broadcast through LDS;
 //    central bodies use FP64 pair terms, the other massive bodies FP32 pair
@@ -49,14 +51,18 @@ static inline unsigned blocks_for(int64_t n, int bs = 256) {
 // ---------------------------------------------------------------------------
 // Kernels
 // ---------------------------------------------------------------------------
+// The boxes of each source tile and of its quarters, and, with tgeo, the tile's
+// geometry as a block of targets (k_batch_wave).
 __global__ __launch_bounds__(BS) void k_batch_tile_boxes(const double *__restrict__ x,
                                                         const double *__restrict__ y,
                                                         const double *__restrict__ z,
+                                                        const double *__restrict__ h,
                                                         const int64_t *__restrict__ off,
                                                         const int64_t *__restrict__ tile_base,
                                                         const int32_t *__restrict__ tile_sys,
-                                                        double *__restrict__ box, double *__restrict__ sub) {
-    __shared__ double red[6][NW];
+                                                        double *__restrict__ box, double *__restrict__ sub,
+                                                        double *__restrict__ tgeo) {
+    __shared__ double red[11][NW];
     const int64_t t = blockIdx.x;
     const int s = tile_sys[t];
     const int64_t start = off[s] + (t - tile_base[s]) * BS;
@@ -89,22 +95,17 @@ __global__ __launch_bounds__(BS) void k_batch_tile_boxes(const double *__restric
         for (int ww = 1; ww < NW; ++ww) r = q < 3 ? fmin(r, red[q][ww]) : fmax(r, red[q][ww]);
         box[t * 8 + q] = r;
     }
+    if (!tgeo) return;   // (uniform over the launch)
+    __syncthreads();
+    const bool valid[1] = {j < end};
+    const double px[1] = {valid[0] ? x[j] : 0.0}, py[1] = {valid[0] ? y[j] : 0.0}, pz[1] = {valid[0] ? z[j] : 0.0};
+    const double ph[1] = {valid[0] ? h[j] : 0.0};
+    BlockStats st;
+    block_stats<1>(px, py, pz, ph, valid, true, red, st);
+    const double ox = uniform_f64(st.ox), oy = uniform_f64(st.oy), oz = uniform_f64(st.oz);
+    const WaveGeom wg = wave_geometry<1>(px, py, pz, ph, valid, ox, oy, oz, true);
+    store_target_geom(tgeo + t * TG_STRIDE, ox, oy, oz, wg, w, lane);
 }
-
-struct BatchArgs {
-    const int64_t *off;
-    const int64_t *tile_base;
-    const double *tile_box;
-    const double *sub_box;        // [ntiles][NQ][8]: boxes of the tile quarters
-    const double *Gs;
-    const double *x, *y, *z, *m, *h;
-    const float *w;               // source weights (weighted far paths) or nullptr
-    const uint8_t *skip_src;
-    double *ax, *ay, *az, *pot;
-    const int64_t *items;
-    int64_t nitems;
-    unsigned *counter;
-};
 
 // Persistent ragged all-pairs kernel: blocks pull (system, target tile) items
 // from an atomic queue until it is empty; the last block to finish resets the
@@ -1104,9 +1105,11 @@ static int bforce(nb_batch *b, bool with_pot, bool allow_timing, bool pot_only =
         else k_batch_force_f64<false><<<(unsigned)b->nitems, BS, 0, s>>>(a);
         NB_TRY(launch_ok("k_batch_force_f64"));
     } else {
-        k_batch_tile_boxes<<<(unsigned)b->ntiles, BS, 0, s>>>(b->x, b->y, b->z, b->off,
+        const bool wave = wave_path(b->tun.far_path, tpt, with_pot, !(with_pot && pot_only));
+        a.tgeo = wave ? b->tgeo : nullptr;
+        k_batch_tile_boxes<<<(unsigned)b->ntiles, BS, 0, s>>>(b->x, b->y, b->z, b->h, b->off,
                                                               b->tile_base, b->tile_sys, b->tile_box,
-                                                              b->sub_box);
+                                                              b->sub_box, wave ? b->tgeo : nullptr);
         NB_TRY(launch_ok("k_batch_tile_boxes"));
         pot_only = pot_only && with_pot;
         // potential alone on far path 4: m/r = rsq(w r^2) m^(2/3)
@@ -1115,25 +1118,27 @@ static int bforce(nb_batch *b, bool with_pot, bool allow_timing, bool pot_only =
             NB_TRY(launch_source_weights(b->m, true, b->n, b->wsrc, s));
             a.w = b->wsrc;
         }
-        int nblk = b->tun.blocks > 0 ? b->tun.blocks : 8 * b->cu_count;
-        nblk = (int)std::max<int64_t>(1, std::min<int64_t>(nblk, b->nitems));
+        if (wave) {
+            NB_TRY(launch_batch_wave(a, with_pot, !pot_only, s));
+        } else {
+            int nblk = b->tun.blocks > 0 ? b->tun.blocks : 8 * b->cu_count;
+            nblk = (int)std::max<int64_t>(1, std::min<int64_t>(nblk, b->nitems));
 #define NB_BL(T_, P_) k_batch_force<T_, P_><<<nblk, BS, 0, s>>>(a)
-        const int fp = with_pot ? FAR_VALU : b->tun.far_path;
-        if (pot_mf4) k_batch_force<1, true, FAR_MFMA_BF16, false><<<nblk, BS, 0, s>>>(a);
-        else if (pot_only && tpt == 1) k_batch_force<1, true, FAR_VALU, false><<<nblk, BS, 0, s>>>(a);
-        else if (pot_only && tpt == 2) k_batch_force<2, true, FAR_VALU, false><<<nblk, BS, 0, s>>>(a);
-        else if (pot_only) k_batch_force<4, true, FAR_VALU, false><<<nblk, BS, 0, s>>>(a);
-        else if (tpt == 1 && fp == FAR_MFMA_R2) k_batch_force<1, false, FAR_MFMA_R2><<<nblk, BS, 0, s>>>(a);
-        else if (tpt == 1 && fp == FAR_MFMA_SUM) k_batch_force<1, false, FAR_MFMA_SUM><<<nblk, BS, 0, s>>>(a);
-        else if (tpt == 1 && fp == FAR_MFMA_BF16) k_batch_force<1, false, FAR_MFMA_BF16><<<nblk, BS, 0, s>>>(a);
-        else if (fp == FAR_WEIGHTED && tpt == 1) k_batch_force<1, false, FAR_WEIGHTED><<<nblk, BS, 0, s>>>(a);
-        else if (fp == FAR_WEIGHTED && tpt == 2) k_batch_force<2, false, FAR_WEIGHTED><<<nblk, BS, 0, s>>>(a);
-        else if (fp == FAR_WEIGHTED && tpt == 4) k_batch_force<4, false, FAR_WEIGHTED><<<nblk, BS, 0, s>>>(a);
-        else if (tpt == 1) { if (with_pot) NB_BL(1, true); else NB_BL(1, false); }
-        else if (tpt == 2) { if (with_pot) NB_BL(2, true); else NB_BL(2, false); }
-        else { if (with_pot) NB_BL(4, true); else NB_BL(4, false); }
+            const int fp = with_pot ? FAR_VALU : b->tun.far_path;
+            if (pot_mf4) k_batch_force<1, true, FAR_MFMA_BF16, false><<<nblk, BS, 0, s>>>(a);
+            else if (pot_only && tpt == 2) k_batch_force<2, true, FAR_VALU, false><<<nblk, BS, 0, s>>>(a);
+            else if (pot_only) k_batch_force<4, true, FAR_VALU, false><<<nblk, BS, 0, s>>>(a);
+            else if (tpt == 1 && fp == FAR_MFMA_R2) k_batch_force<1, false, FAR_MFMA_R2><<<nblk, BS, 0, s>>>(a);
+            else if (tpt == 1 && fp == FAR_MFMA_SUM) k_batch_force<1, false, FAR_MFMA_SUM><<<nblk, BS, 0, s>>>(a);
+            else if (tpt == 1 && fp == FAR_MFMA_BF16) k_batch_force<1, false, FAR_MFMA_BF16><<<nblk, BS, 0, s>>>(a);
+            else if (fp == FAR_WEIGHTED && tpt == 1) k_batch_force<1, false, FAR_WEIGHTED><<<nblk, BS, 0, s>>>(a);
+            else if (fp == FAR_WEIGHTED && tpt == 2) k_batch_force<2, false, FAR_WEIGHTED><<<nblk, BS, 0, s>>>(a);
+            else if (fp == FAR_WEIGHTED && tpt == 4) k_batch_force<4, false, FAR_WEIGHTED><<<nblk, BS, 0, s>>>(a);
+            else if (tpt == 2) { if (with_pot) NB_BL(2, true); else NB_BL(2, false); }
+            else { if (with_pot) NB_BL(4, true); else NB_BL(4, false); }
 #undef NB_BL
-        NB_TRY(launch_ok("k_batch_force"));
+            NB_TRY(launch_ok("k_batch_force"));
+        }
     }
     if (e0) {
         hipEvent_t e1;
@@ -1627,6 +1632,7 @@ int nb_batch_create(nb_batch **out, int32_t nsys, const int64_t *offsets, int32_
             (rc = dalloc(&b->tile_sys, sizeof(int32_t) * (size_t)std::max<int64_t>(b->ntiles, 1))) ||
             (rc = dalloc(&b->tile_box, sizeof(double) * 8 * (size_t)std::max<int64_t>(b->ntiles, 1))) ||
             (rc = dalloc(&b->sub_box, sizeof(double) * 8 * NQ * (size_t)std::max<int64_t>(b->ntiles, 1))) ||
+            (rc = dalloc(&b->tgeo, sizeof(double) * TG_STRIDE * (size_t)std::max<int64_t>(b->ntiles, 1))) ||
             (rc = dalloc(&b->counter, sizeof(unsigned) * 2)) ||
             (rc = dalloc(&b->stage, sizeof(double) * 3 * n)) ||
             (rc = dalloc(&b->wsrc, sizeof(float) * std::max<int64_t>(n, 1))) ||
@@ -1673,7 +1679,7 @@ int nb_batch_destroy(nb_batch *b) {
     dfree(b->x); dfree(b->y); dfree(b->z); dfree(b->vx); dfree(b->vy); dfree(b->vz);
     dfree(b->m); dfree(b->h); dfree(b->ax); dfree(b->ay); dfree(b->az); dfree(b->pot);
     dfree(b->perm); dfree(b->central); dfree(b->cidx);
-    dfree(b->tile_base); dfree(b->tile_sys); dfree(b->tile_box); dfree(b->sub_box);
+    dfree(b->tile_base); dfree(b->tile_sys); dfree(b->tile_box); dfree(b->sub_box); dfree(b->tgeo);
     dfree(b->items); dfree(b->counter); dfree(b->stage); dfree(b->red); dfree(b->wsrc);
     dfree(b->sort_tmp); dfree(b->keys); dfree(b->idx); dfree(b->sysbox); dfree(b->spare);
     dfree(b->pk_lane); dfree(b->pk_meta); dfree(b->pk_blk); dfree(b->pk_tiny);

@@ -1,0 +1,113 @@
+// nb_batch_wave.hip -- the ensemble's all-pairs kernel of far path 0 with one
+// target per lane.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "nb_batch.h"
+#include "nb_wave.h"
+
+namespace nb {
+
+// Far path 0 with one target per lane (wave_force): one workgroup per quarter
+// (64 targets) of an item, whose W waves take a part of the system's sources
+// each, by whole tiles; their sums meet in LDS in a fixed order.  The origins,
+// classes and FP32 sums of a tile are force_block's, so the results are too (but
+// for the order of the FP64 sums).  Bound by FP32 VALU issue on large
+// ensembles (2.85e12 pairs/s on the 512 clusters below); the block-wide
+// persistent kernel that it replaced held a workgroup at its barriers for the
+// slowest of four waves, and a small ensemble gave it few waves with long
+// source loops: an item of 16384 sources took about 0.9 ms alone.
+//
+// The items come in order of cost, so the last workgroups are the shortest, and
+// ITEM_RUN consecutive ones (quarters of one system, or of a few) run on the
+// same XCD, whose L2 then holds their sources.  Runs of 8, 16 and 32 are alike
+// (512 clusters 5.75 / 5.76 / 5.79 ms a force); 256 leave the XCDs unequal work
+// (5 % slower).
+//
+// Measured per force with its tile boxes (clusters of 256 to 16384 bodies,
+// log-uniform): 512 clusters 6.05 -> 5.76 ms, 200 2.16 -> 1.85, 64 1.21 -> 0.74,
+// 32 1.05 -> 0.48, 8 0.98 -> 0.30, one of 3271 0.223 -> 0.055 ms.
+constexpr unsigned ITEM_RUN = 16, XCDS = 8;
+template <bool ACC, bool POT, int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(ACC &&POT ? 5 : 6)))
+void k_batch_wave(BatchArgs a) {
+    constexpr int NV = (ACC ? 3 : 0) + (POT ? 1 : 0);
+    constexpr int V0 = ACC ? 0 : 3;
+    __shared__ WaveStage<double> st[W];
+    __shared__ double red[W - 1][NV][64];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    unsigned b = blockIdx.x;
+    if (b < gridDim.x / (ITEM_RUN * XCDS) * (ITEM_RUN * XCDS)) {
+        const unsigned slot = b / XCDS;
+        b = (slot / ITEM_RUN * XCDS + b % XCDS) * ITEM_RUN + slot % ITEM_RUN;
+    }
+    const int64_t item = a.items[b / NQ];
+    const int s = (int)(item >> 32);
+    const int64_t o0 = a.off[s], o1 = a.off[s + 1];
+    const int64_t qt = (item & 0xffffffffll) * NQ + b % NQ;   // the targets' quarter of the system
+    const int64_t i0 = o0 + qt * SB;
+    if (i0 >= o1) return;   // (the whole workgroup)
+    const int64_t i = i0 + lane;
+    const int64_t ic = i < o1 ? i : o1 - 1;
+    const int64_t part = ((o1 - o0 + BS - 1) / BS + W - 1) / W * BS;
+    const int64_t j0 = o0 + part * wave < o1 ? o0 + part * wave : o1;
+    const int64_t j1 = j0 + part < o1 ? j0 + part : o1;
+    const int64_t tb = a.tile_base[s];
+    double v[4];   // ax, ay, az, pot
+    wave_force<double, ACC, POT, true>(st[wave], a.x[ic], a.y[ic], a.z[ic], a.h[ic], nullptr, a.x, a.y, a.z, a.m,
+                                       a.skip_src, a.sub_box + (tb * NQ + (j0 - o0) / SB) * 8, a.tile_box, j0, j1,
+                                       v[0], v[1], v[2], v[3], a.tgeo + (tb + qt / NQ) * TG_STRIDE,
+                                       (int)(qt % NQ));
+    if (wave > 0) {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) red[wave - 1][q][lane] = v[V0 + q];
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int w = 0; w < W - 1; ++w)
+#pragma unroll
+        for (int q = 0; q < NV; ++q) v[V0 + q] += red[w][q][lane];
+    if (i >= o1) return;
+    const double G = a.Gs[s];
+    if (ACC) {
+        a.ax[i] = G * v[0];
+        a.ay[i] = G * v[1];
+        a.az[i] = G * v[2];
+    }
+    if (POT) a.pot[i] = -G * v[3];
+}
+
+template <int W>
+static void launch(const BatchArgs &a, bool pot, bool acc, hipStream_t s) {
+    const unsigned nb = (unsigned)(a.nitems * NQ), bs = 64 * W;
+    if (pot && acc) k_batch_wave<true, true, W><<<nb, bs, 0, s>>>(a);
+    else if (pot) k_batch_wave<false, true, W><<<nb, bs, 0, s>>>(a);
+    else k_batch_wave<true, false, W><<<nb, bs, 0, s>>>(a);
+}
+
+// Four waves per 64 targets, or eight while the launch has fewer workgroups
+// than this: eight / four waves took 48 / 62 us a force at 52 workgroups, 273 /
+// 302 at 776 and 459 / 479 at 2100, but 713 / 710 at 3600 and 5.66 / 5.57 ms at
+// 33000; sixteen were slower from 776 on (timed with the sources split by
+// quarters instead of tiles).
+constexpr int64_t EIGHT_WAVES_BELOW = 3072;
+
+int launch_batch_wave(const BatchArgs &a, bool pot, bool acc, hipStream_t s) {
+    if (a.nitems <= 0) return NB_OK;
+    if (a.nitems * NQ > INT32_MAX) {
+        set_error("ensemble force grid too large (%lld items)", (long long)a.nitems);
+        return NB_ERR_INVALID;
+    }
+    if (a.nitems * NQ < EIGHT_WAVES_BELOW) launch<2 * NW>(a, pot, acc, s);
+    else launch<NW>(a, pot, acc, s);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+        set_error("launch of k_batch_wave failed: %s", hipGetErrorString(e));
+        return NB_ERR_HIP;
+    }
+    return NB_OK;
+}
+
+}  // namespace nb

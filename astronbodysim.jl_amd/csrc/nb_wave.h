@@ -142,19 +142,27 @@ __device__ __forceinline__ void near_sources(scalar_ptr<T> sx, scalar_ptr<T> sy,
 // tbox, when not null: the box and largest h of the wave's targets (lo xyz,
 // hi xyz, h); else reduced here.  sub_box: the boxes of the quarters from j0
 // on, or, when null, tile_box: the boxes of the BS-source tiles from j0 on.
+// TILES: the origin, box and classes are those of the targets' block (tgeo, its
+// stored record, and the wave's place gw in it) and the FP32 sums run over a
+// whole tile (j0 starts one), as in force_block, whose sums these then are.
 // Returns FP64 sums without G.
-template <typename T, bool ACC, bool POT>
+template <typename T, bool ACC, bool POT, bool TILES = false>
 __device__ __forceinline__ void wave_force(WaveStage<T> &st, T xt, T yt, T zt, double h,
                                            const double *__restrict__ tbox, const T *__restrict__ sx,
                                            const T *__restrict__ sy, const T *__restrict__ sz,
                                            const T *__restrict__ sm, const uint8_t *__restrict__ skip_src,
                                            const double *__restrict__ sub_box,
                                            const double *__restrict__ tile_box, int64_t j0, int64_t j1,
-                                           double &Ax, double &Ay, double &Az, double &Aq) {
+                                           double &Ax, double &Ay, double &Az, double &Aq,
+                                           const double *__restrict__ tgeo = nullptr, int gw = 0) {
     constexpr bool D = WaveStage<T>::D;
     const int lane = threadIdx.x & 63;
     double o[3];
-    {
+    if constexpr (TILES) {
+        if (lane < 8) st.geo[lane] = tgeo[3 + 9 * gw + lane];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) o[d] = uniform_f64(tgeo[d]);
+    } else {
         double lo[3], hi[3], hmax, rb = 0.0;
         if (tbox) {
 #pragma unroll
@@ -204,6 +212,7 @@ __device__ __forceinline__ void wave_force(WaveStage<T> &st, T xt, T yt, T zt, d
     uint64_t m_soft = 0, m_close = 0;
     if (j0 < j1) fetch(j0 + lane);
     int q = 0;
+    float ax = 0.0f, ay = 0.0f, az = 0.0f, aq = 0.0f;
     for (int64_t base = j0; base < j1; base += SB, ++q) {
         {
             const bool rv = base + lane < j1;
@@ -235,7 +244,6 @@ __device__ __forceinline__ void wave_force(WaveStage<T> &st, T xt, T yt, T zt, d
         }
         const uint64_t bit = 1ull << (q & 63);
         const int cnt = j1 - base < SB ? (int)(j1 - base) : SB;
-        float ax = 0.0f, ay = 0.0f, az = 0.0f, aq = 0.0f;
         if (m_soft & bit) {
             near_sources<T, true, ACC, POT>(as_scalar(sx + base), as_scalar(sy + base), as_scalar(sz + base), st.m,
                                             cnt, xt, yt, zt, t, ax, ay, az, aq);
@@ -254,8 +262,10 @@ __device__ __forceinline__ void wave_force(WaveStage<T> &st, T xt, T yt, T zt, d
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");   // read before the next staging
+        if (TILES && (q & (NQ - 1)) != NQ - 1 && base + SB < j1) continue;
         if (ACC) { Ax += (double)ax; Ay += (double)ay; Az += (double)az; }
         if (POT) Aq += (double)aq;
+        ax = ay = az = aq = 0.0f;
     }
 }
 

@@ -647,27 +647,16 @@ int nb_download(nb_ctx *c, double *pos, double *vel, double *acc, double *pot) {
     if (n == 0) return NB_OK;
     hipStream_t s = c->stream;
     const size_t nn = (size_t)n;
-    if (pos) {
-        NB_TRY(to_aos(c->x, c->y, c->z, c->perm, n, c->is_double, c->stage, s));
-        NB_HIP(hipMemcpyAsync(pos, c->stage, sizeof(double) * 3 * nn, hipMemcpyDeviceToHost, s));
-        NB_HIP(hipStreamSynchronize(s));
-    }
-    if (vel) {
-        NB_TRY(to_aos(c->vx, c->vy, c->vz, c->perm, n, c->is_double, c->stage, s));
-        NB_HIP(hipMemcpyAsync(vel, c->stage, sizeof(double) * 3 * nn, hipMemcpyDeviceToHost, s));
-        NB_HIP(hipStreamSynchronize(s));
-    }
-    if (acc) {
-        NB_TRY(to_aos(c->ax, c->ay, c->az, c->perm, n, true, c->stage, s));
-        NB_HIP(hipMemcpyAsync(acc, c->stage, sizeof(double) * 3 * nn, hipMemcpyDeviceToHost, s));
-        NB_HIP(hipStreamSynchronize(s));
-    }
-    if (pot) {
-        NB_TRY(scalar_out(c->pot, c->perm, n, c->stage, s));
-        NB_HIP(hipMemcpyAsync(pot, c->stage, sizeof(double) * nn, hipMemcpyDeviceToHost, s));
-        NB_HIP(hipStreamSynchronize(s));
-    }
-    return NB_OK;
+    auto aos = [&](const void *x, const void *y, const void *z, bool is_double) {
+        return to_aos(x, y, z, c->perm, n, is_double, c->stage, s);
+    };
+    auto fpos = [&] { return aos(c->x, c->y, c->z, c->is_double); };
+    auto fvel = [&] { return aos(c->vx, c->vy, c->vz, c->is_double); };
+    auto facc = [&] { return aos(c->ax, c->ay, c->az, true); };
+    auto fpot = [&] { return scalar_out(c->pot, c->perm, n, c->stage, s); };
+    const DownField f[4] = {{pos, c->stage, 3 * nn, fpos}, {vel, c->stage, 3 * nn, fvel},
+                            {acc, c->stage, 3 * nn, facc}, {pot, c->stage, nn, fpot}};
+    return download_fields(f, 4, c->dev, s);
 }
 
 int nb_compute_force(nb_ctx *c) {
@@ -779,13 +768,10 @@ static int probe_points(nb_ctx *c, int64_t npts, const double *pts, double h, do
         for (const BgField &f : c->bg)
             NB_TRY(background(tx, ty, tz, npts, true, f, with_pot ? nullptr : oax, oay, oaz,
                               with_pot ? opot : nullptr, s));
-        if (acc) {
-            NB_TRY(to_aos(oax, oay, oaz, nullptr, npts, true, aos, s));
-            NB_HIP(hipMemcpyAsync(acc, aos, sizeof(double) * 3 * np, hipMemcpyDeviceToHost, s));
-        }
-        if (pot) NB_HIP(hipMemcpyAsync(pot, opot, sizeof(double) * np, hipMemcpyDeviceToHost, s));
-        NB_HIP(hipStreamSynchronize(s));
-        return NB_OK;
+        auto facc = [&] { return to_aos(oax, oay, oaz, nullptr, npts, true, aos, s); };
+        auto fpot = [] { return (int)NB_OK; };
+        const DownField f[2] = {{acc, aos, 3 * np, facc}, {pot, opot, np, fpot}};
+        return download_fields(f, 2, c->dev, s);
     };
     const int rc = launch();
     if (rc) (void)hipStreamSynchronize(s);   // the caller's arrays are free again

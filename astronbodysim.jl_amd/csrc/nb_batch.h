@@ -9,6 +9,7 @@
 #include "nb_ctx.h"
 
 struct nb_batch {
+    nb::DownloadUse download;
     int dev = 0;
     int mode = NB_MODE_SPLIT;
     hipStream_t stream = nullptr;

@@ -1774,28 +1774,17 @@ int nb_batch_download(nb_batch *b, double *pos, double *vel, double *acc, double
     const int64_t n = b->n;
     if (n == 0) return NB_OK;
     hipStream_t s = b->stream;
-    const size_t b3 = sizeof(double) * 3 * (size_t)n;
-    if (pos) {
-        NB_TRY(to_aos(b->x, b->y, b->z, b->perm, n, true, b->stage, s));
-        NB_HIP(hipMemcpyAsync(pos, b->stage, b3, hipMemcpyDeviceToHost, s));
-        NB_HIP(hipStreamSynchronize(s));
-    }
-    if (vel) {
-        NB_TRY(to_aos(b->vx, b->vy, b->vz, b->perm, n, true, b->stage, s));
-        NB_HIP(hipMemcpyAsync(vel, b->stage, b3, hipMemcpyDeviceToHost, s));
-        NB_HIP(hipStreamSynchronize(s));
-    }
-    if (acc) {
-        NB_TRY(to_aos(b->ax, b->ay, b->az, b->perm, n, true, b->stage, s));
-        NB_HIP(hipMemcpyAsync(acc, b->stage, b3, hipMemcpyDeviceToHost, s));
-        NB_HIP(hipStreamSynchronize(s));
-    }
-    if (pot) {
-        NB_TRY(scalar_out(b->pot, b->perm, n, b->stage, s));
-        NB_HIP(hipMemcpyAsync(pot, b->stage, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, s));
-        NB_HIP(hipStreamSynchronize(s));
-    }
-    return NB_OK;
+    const size_t nn = (size_t)n;
+    auto aos = [&](const double *x, const double *y, const double *z) {
+        return to_aos(x, y, z, b->perm, n, true, b->stage, s);
+    };
+    auto fpos = [&] { return aos(b->x, b->y, b->z); };
+    auto fvel = [&] { return aos(b->vx, b->vy, b->vz); };
+    auto facc = [&] { return aos(b->ax, b->ay, b->az); };
+    auto fpot = [&] { return scalar_out(b->pot, b->perm, n, b->stage, s); };
+    const DownField f[4] = {{pos, b->stage, 3 * nn, fpos}, {vel, b->stage, 3 * nn, fvel},
+                            {acc, b->stage, 3 * nn, facc}, {pot, b->stage, nn, fpot}};
+    return download_fields(f, 4, b->dev, s);
 }
 
 int nb_batch_set_central(nb_batch *b, int32_t count) {

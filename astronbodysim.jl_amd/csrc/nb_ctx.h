@@ -6,6 +6,7 @@
 #include <utility>
 #include <vector>
 
+#include "nb_download.h"
 #include "nb_integrate.h"
 #include "nb_internal.h"
 
@@ -54,6 +55,7 @@ struct SnapSlot {
 }  // namespace nb
 
 struct nb_ctx {
+    nb::DownloadUse download;
     int dev = 0;
     int mode = NB_MODE_SPLIT;
     int64_t n = 0;

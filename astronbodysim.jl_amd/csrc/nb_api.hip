@@ -667,18 +667,21 @@ int nb_compute_force(nb_ctx *c) {
 
 int nb_compute_potential(nb_ctx *c, int32_t add_self_term) {
     NB_TRY(check_ctx(c));
-    // The potential is produced together with the acceleration by the same
-    // kernel; keep the caller's accelerations by saving them around it.
+    // The FP32-pair kernels write the potential alone.  The FP64 kernel, the
+    // central bodies' pass and background fields add to the accelerations too:
+    // the caller's are kept around them (30011 particles in split precision:
+    // the six copies were about 30 of 300 us).
+    const bool keep = c->n > 0 && (c->mode == NB_MODE_FP64 || c->ncentral > 0 || !c->bg.empty() || c->mond_acc0 > 0.0);
     hipStream_t s = c->stream;
     const size_t nb3 = sizeof(double) * (size_t)c->n;
     NB_TRY(maybe_sort(c, 1));   // reorder first, so the saved accelerations stay aligned
-    if (c->n > 0) {
+    if (keep) {
         NB_HIP(hipMemcpyAsync(c->stage, c->ax, nb3, hipMemcpyDeviceToDevice, s));
         NB_HIP(hipMemcpyAsync(c->stage + c->n, c->ay, nb3, hipMemcpyDeviceToDevice, s));
         NB_HIP(hipMemcpyAsync(c->stage + 2 * c->n, c->az, nb3, hipMemcpyDeviceToDevice, s));
     }
     NB_TRY(run_force(c, true, false, false, true));
-    if (c->n > 0) {
+    if (keep) {
         NB_HIP(hipMemcpyAsync(c->ax, c->stage, nb3, hipMemcpyDeviceToDevice, s));
         NB_HIP(hipMemcpyAsync(c->ay, c->stage + c->n, nb3, hipMemcpyDeviceToDevice, s));
         NB_HIP(hipMemcpyAsync(c->az, c->stage + 2 * c->n, nb3, hipMemcpyDeviceToDevice, s));

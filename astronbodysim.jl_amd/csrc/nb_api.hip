@@ -125,11 +125,18 @@ int ensure_tbg(nb_ctx *c, const Geometry &g) {
     return dalloc(&c->tbg, sizeof(unsigned) * 16 * (size_t)BS * (size_t)((c->n + BS - 1) / BS + 1));
 }
 
+// At most STEP_SEGMENTS source segments for the forces of few targets: in
+// k_force_step each is one more arrival before the last one's sums (2000
+// particles in 32 / 16 segments 17.4 / 15.3 us a step, 4096 in FP32 23.5 / 19.1,
+// from 8000 on alike), and every other launch of the same forces cuts the
+// sources alike, so that its sums have the same bits.
+constexpr int STEP_SEGMENTS = 16;
+
 // The launch of the context's own forces or potentials.
 Geometry force_geometry(const nb_ctx *c, bool pot, bool acc) {
     if (c->mode == NB_MODE_FP64) return geometry(c->n, c->n, 1, c->tun.j_segments);
     if (wave_path(c->tun.far_path, c->tun.targets_per_thread, pot, acc))
-        return wave_launch_geometry(c->n, c->n, c->tun.j_segments);
+        return wave_launch_geometry(c->n, c->n, c->tun.j_segments, pot ? WAVE_SEGMENTS : STEP_SEGMENTS);
     return geometry(c->n, c->n, c->tun.targets_per_thread, c->tun.j_segments);
 }
 
@@ -537,7 +544,7 @@ int nb_destroy(nb_ctx *c) {
     dfree(c->m); dfree(c->h); dfree(c->coll);
     dfree(c->ax); dfree(c->ay); dfree(c->az); dfree(c->pot);
     dfree(c->perm);
-    dfree(c->tile_box); dfree(c->sub_box); dfree(c->tgeo); dfree(c->tbg); dfree(c->nflag); dfree(c->part); dfree(c->stage); dfree(c->red); dfree(c->wsrc); dfree(c->probe);
+    dfree(c->tile_box); dfree(c->sub_box); dfree(c->tgeo); dfree(c->tbg); dfree(c->nflag); dfree(c->part); dfree(c->xyz2); dfree(c->sub2); dfree(c->arrived); dfree(c->stage); dfree(c->red); dfree(c->wsrc); dfree(c->probe);
     dfree(c->time); dfree(c->flag); dfree(c->central);
     dfree(c->cx); dfree(c->cy); dfree(c->cz); dfree(c->cm); dfree(c->cidx); dfree(c->cstep);
     dfree(c->ti_end); dfree(c->ti_beg);
@@ -840,7 +847,8 @@ int nb_kick(nb_ctx *c, double dt) {
 static int step_args(nb_ctx *c, int64_t k, double dt, StepArgs &a, int *geo_ready) {
     a = StepArgs{};
     a.n = c->n; a.dt = dt; a.G = c->G;
-    a.x = c->x; a.y = c->y; a.z = c->z; a.vx = c->vx; a.vy = c->vy; a.vz = c->vz; a.m = c->m; a.h = c->h;
+    a.x = a.xn = c->x; a.y = a.yn = c->y; a.z = a.zn = c->z;
+    a.vx = c->vx; a.vy = c->vy; a.vz = c->vz; a.m = c->m; a.h = c->h;
     a.ax = c->ax; a.ay = c->ay; a.az = c->az;
     a.time = c->time; a.box = c->tile_box; a.sub = c->sub_box;
     if (c->mode == NB_MODE_SPLIT_CENTRAL && c->ncentral > 0) {
@@ -915,6 +923,82 @@ static int enqueue_steps(nb_ctx *c, int64_t k, int64_t count, double dt, bool al
     return NB_OK;
 }
 
+// Whole steps in one launch each (k_force_step): far path 0 on targets that share
+// waves (below WAVE_SPLIT_BELOW; there the gain is the same few microseconds of
+// a launch gap at every size), with nothing else that adds to the accelerations.
+static bool one_launch_steps(const nb_ctx *c) {
+    if (c->n <= 0 || c->mode == NB_MODE_FP64 || !wave_path(c->tun.far_path, c->tun.targets_per_thread, false, true) ||
+        !c->bg.empty() || c->mond_acc0 > 0.0)
+        return false;
+    // (with one segment the uncaptured steps take the central bodies' terms from
+    // the FP64 force kernel, whose last bits differ from the kick's)
+    const Geometry g = force_geometry(c, false, true);
+    return g.wave_split && (g.nseg > 1 || c->ncentral == 0);
+}
+
+// Their second set of positions and boxes, and the counters (zeros between
+// launches); before any capture.
+static int ensure_step2(nb_ctx *c) {
+    if (c->arrived) return NB_OK;
+    const size_t nn = (size_t)c->n, groups = (nn + 63) / 64;
+    dfree(c->xyz2); dfree(c->sub2);
+    NB_TRY(dalloc(&c->xyz2, (c->is_double ? sizeof(double) : sizeof(float)) * 3 * nn));
+    NB_TRY(dalloc(&c->sub2, sizeof(double) * 8 * NQ * ((nn + BS - 1) / BS)));
+    unsigned *arrived = nullptr;
+    NB_TRY(dalloc(&arrived, sizeof(unsigned) * groups));
+    const hipError_t e = hipMemsetAsync(arrived, 0, sizeof(unsigned) * groups, c->stream);
+    if (e != hipSuccess) {
+        dfree(arrived);
+        set_error("hipMemsetAsync failed: %s", hipGetErrorString(e));
+        return NB_ERR_HIP;
+    }
+    c->arrived = arrived;
+    return NB_OK;
+}
+
+// Steps 0 .. count - 1 (count even) of a captured run, one launch each after the
+// first drift.  The drifts alternate between the two sets of positions; the
+// first one goes to the second set, so the last one ends in the context's own.
+extern "C++" template <typename T>
+static int enqueue_one_launch_steps(nb_ctx *c, int64_t count, double dt) {
+    const int64_t n = c->n;
+    T *own[3] = {(T *)c->x, (T *)c->y, (T *)c->z};
+    T *two[3] = {(T *)c->xyz2, (T *)c->xyz2 + n, (T *)c->xyz2 + 2 * n};
+    const Geometry g = force_geometry(c, false, true);
+    ForceArgs<T> f{};
+    f.th = c->h; f.nt = n; f.sm = (const T *)c->m; f.ns = n;
+    f.use_origin = c->is_double ? 1 : 0;
+    f.nseg = g.nseg; f.seg_len = g.seg_len; f.nblk_i = g.nblk_i; f.wave_split = 1; f.G = c->G;
+    f.part = c->part;
+    f.tile_box = c->tile_box;
+    f.skip_src = (c->mode == NB_MODE_SPLIT_CENTRAL && c->ncentral > 0) ? c->central : nullptr;
+    StepArgs a;
+    int geo_ready = 0;
+    auto drift_to = [&](int64_t k, bool second) {
+        add_drift(c, k, a);
+        T **to = second ? two : own;
+        a.xn = to[0]; a.yn = to[1]; a.zn = to[2];
+        a.sub = second ? c->sub2 : c->sub_box;
+    };
+    NB_TRY(step_args(c, 0, dt, a, &geo_ready));
+    drift_to(0, true);
+    a.box = nullptr;
+    NB_TRY(launch_step(a, c->is_double, c->stream));
+    for (int64_t k = 0; k < count; ++k) {
+        T **at = k % 2 == 0 ? two : own;
+        f.tx = f.sx = at[0]; f.ty = f.sy = at[1]; f.tz = f.sz = at[2];
+        f.sub_box = f.tbox = k % 2 == 0 ? c->sub2 : c->sub_box;
+        NB_TRY(step_args(c, k, dt, a, &geo_ready));
+        a.kick = 1;
+        a.arrived = c->arrived;
+        if (k + 1 < count) drift_to(k + 1, k % 2 == 1);
+        NB_TRY(launch_force_step(f, a, c->stream));
+        c->force_calls++;
+        c->calls_since_sort++;
+    }
+    return NB_OK;
+}
+
 int nb_kdk_steps(nb_ctx *c, int64_t nsteps, double dt, double t_begin, int32_t use_graph) {
     NB_TRY(check_ctx(c));
     if (nsteps < 0 || !isfinite(dt) || !isfinite(t_begin)) {
@@ -941,8 +1025,12 @@ int nb_kdk_steps(nb_ctx *c, int64_t nsteps, double dt, double t_begin, int32_t u
             NB_TRY(ensure_part(c, g.nseg));
             NB_TRY(ensure_tbg(c, g));
             if (weighted) NB_TRY(ensure_source_weights(c));
+            const bool one = one_launch_steps(c);
+            if (one) NB_TRY(ensure_step2(c));
             NB_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-            const int rc = enqueue_steps(c, 0, chunk, dt, false, false);
+            const int rc = !one ? enqueue_steps(c, 0, chunk, dt, false, false)
+                           : c->is_double ? enqueue_one_launch_steps<double>(c, chunk, dt)
+                                          : enqueue_one_launch_steps<float>(c, chunk, dt);
             hipGraph_t graph = nullptr;
             hipError_t e = hipStreamEndCapture(s, &graph);
             if (rc != NB_OK) {

@@ -76,6 +76,9 @@ struct nb_ctx {
     unsigned *tbg = nullptr;      // [target blocks][BS][16] bf16 B operands (far path 4), on first need
     uint8_t *nflag = nullptr;     // one byte per force wave: near tiles left to the near pass
     size_t nflag_cap = 0;
+    void *xyz2 = nullptr;         // 3n: the other positions of a run of k_force_step launches
+    double *sub2 = nullptr;       // their quarter boxes
+    unsigned *arrived = nullptr;  // [64-target groups] workgroups counted in (k_force_step)
     double *part = nullptr;
     int part_cap = 0;             // segments the partial buffer holds
     double *stage = nullptr;      // 3n doubles

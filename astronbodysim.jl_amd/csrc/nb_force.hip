@@ -480,6 +480,91 @@ __global__ __launch_bounds__(BS) void k_tile_boxes(const T *__restrict__ x, cons
                    v && h ? h[j] : h_const, v, box, sub, red);
 }
 
+// Kick of particle j from the FP64 sums of its force (without G): the central
+// bodies' FP64 terms, Acc = G sum, Vel += Acc dt.
+template <typename T>
+__device__ __forceinline__ void kick_particle(const StepArgs &a, int64_t j, const double (&s)[3], T px, T py, T pz,
+                                              double ph, T &ux, T &uy, T &uz) {
+    double fx = a.G * s[0], fy = a.G * s[1], fz = a.G * s[2];
+    if (a.ncentral > 0) {
+        const double hinv = 1.0 / ph, hinv3 = hinv * hinv * hinv;
+        double bx = 0.0, by = 0.0, bz = 0.0, bq = 0.0;
+        const double *c = a.c_in;
+        const int64_t k = a.ncentral;
+        for (int64_t u = 0; u < k; ++u)
+            pair_f64<false>(c[u], c[k + u], c[2 * k + u], c[3 * k + u], (double)px, (double)py, (double)pz, ph, hinv,
+                            hinv3, bx, by, bz, bq);
+        fx += bx * a.G;
+        fy += by * a.G;
+        fz += bz * a.G;
+    }
+    a.ax[j] = fx;
+    a.ay[j] = fy;
+    a.az[j] = fz;
+    const T c = (T)a.dt;
+    ux += (T)fx * c;
+    uy += (T)fy * c;
+    uz += (T)fz * c;
+    ((T *)a.vx)[j] = ux;
+    ((T *)a.vy)[j] = uy;
+    ((T *)a.vz)[j] = uz;
+}
+
+// Drift of particle j (v: it exists): Pos += Vel (t_new - t_old), stored to
+// xn.., particle 0 publishing t_new; a central body's new position goes to c_out.
+template <typename T>
+__device__ __forceinline__ void drift_particle(const StepArgs &a, int64_t j, bool v, T ux, T uy, T uz, T &px, T &py,
+                                               T &pz) {
+    const double t_old = a.time[a.rd];
+    const double t_new = t_old + a.dt;
+    if (j == 0) a.time[a.wr] = t_new;
+    if (!v) return;
+    const T d = (T)(t_new - t_old);
+    px += ux * d;
+    py += uy * d;
+    pz += uz * d;
+    ((T *)a.xn)[j] = px;
+    ((T *)a.yn)[j] = py;
+    ((T *)a.zn)[j] = pz;
+    if (a.ncentral > 0 && a.central[j]) {
+        for (int64_t u = 0; u < a.ncentral; ++u)
+            if (a.cidx[u] == j) {
+                a.c_out[u] = (double)px;
+                a.c_out[a.ncentral + u] = (double)py;
+                a.c_out[2 * a.ncentral + u] = (double)pz;
+                a.c_out[3 * a.ncentral + u] = (double)((const T *)a.m)[j];
+            }
+    }
+}
+
+// Segments g, g + STEP_GROUPS, ... of target i's partial sums, in order.
+// SHARED: other workgroups of this launch wrote them.
+constexpr int STEP_GROUPS = 4;
+template <bool SHARED>
+__device__ __forceinline__ void group_sums(const double *part, int64_t n, int nseg, int64_t i, int grp,
+                                           double (&s)[3]) {
+    const double *p = part + i;
+    constexpr int U = 4;   // segments in flight; past the end: the last one's, not added
+    for (int g = grp; g < nseg; g += U * STEP_GROUPS) {
+        double t[U][3];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int gu = g + u * STEP_GROUPS < nseg ? g + u * STEP_GROUPS : nseg - 1;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                const double *e = p + ((int64_t)gu * 4 + q) * n;
+                t[u][q] = SHARED ? __hip_atomic_load(e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *e;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (g + u * STEP_GROUPS < nseg) {
+#pragma unroll
+                for (int q = 0; q < 3; ++q) s[q] += t[u][q];
+            }
+    }
+}
+
 // The per-particle part of a KDK step, between one force launch and the next
 // (one workgroup per 256 particles): the sums of the force's segments, the
 // central bodies' FP64 terms and the kick (a.kick), then the next step's drift
@@ -496,7 +581,6 @@ __global__ __launch_bounds__(BS) void k_tile_boxes(const T *__restrict__ x, cons
 //          to time[wr] (rd != wr)
 // The central bodies' terms read their positions from c_in, and the drift
 // leaves the new ones in c_out: other workgroups still read the old ones.
-constexpr int STEP_GROUPS = 4;
 template <typename T, bool GEO, bool ROWS>
 __global__ __launch_bounds__(BS * STEP_GROUPS) void k_step(StepArgs a) {
     __shared__ double sums[STEP_GROUPS - 1][3][BS];
@@ -505,7 +589,7 @@ __global__ __launch_bounds__(BS * STEP_GROUPS) void k_step(StepArgs a) {
     const int tid = threadIdx.x & (BS - 1), grp = threadIdx.x / BS;
     const int64_t j = (int64_t)blockIdx.x * BS + tid;
     const bool v = j < a.n;
-    T *x = (T *)a.x, *y = (T *)a.y, *z = (T *)a.z, *vx = (T *)a.vx, *vy = (T *)a.vy, *vz = (T *)a.vz;
+    const T *x = (T *)a.x, *y = (T *)a.y, *z = (T *)a.z, *vx = (T *)a.vx, *vy = (T *)a.vy, *vz = (T *)a.vz;
     T px = 0, py = 0, pz = 0, ux = 0, uy = 0, uz = 0;
     double ph = 0.0;
     if (grp == 0 && v) {
@@ -515,25 +599,7 @@ __global__ __launch_bounds__(BS * STEP_GROUPS) void k_step(StepArgs a) {
     }
     if (a.kick) {
         double s[3] = {0.0, 0.0, 0.0};
-        if (v) {
-            const double *p = a.part + j;
-            constexpr int U = 4;   // segments in flight; past the end: the last one's, not added
-            for (int g = grp; g < a.nseg; g += U * STEP_GROUPS) {
-                double t[U][3];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int gu = g + u * STEP_GROUPS < a.nseg ? g + u * STEP_GROUPS : a.nseg - 1;
-#pragma unroll
-                    for (int q = 0; q < 3; ++q) t[u][q] = p[((int64_t)gu * 4 + q) * a.n];
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-                    if (g + u * STEP_GROUPS < a.nseg) {
-#pragma unroll
-                        for (int q = 0; q < 3; ++q) s[q] += t[u][q];
-                    }
-            }
-        }
+        if (v) group_sums<false>(a.part, a.n, a.nseg, j, grp, s);
         if (grp > 0) {
 #pragma unroll
             for (int q = 0; q < 3; ++q) sums[grp - 1][q][tid] = s[q];
@@ -544,49 +610,11 @@ __global__ __launch_bounds__(BS * STEP_GROUPS) void k_step(StepArgs a) {
             for (int g = 0; g < STEP_GROUPS - 1; ++g)
 #pragma unroll
                 for (int q = 0; q < 3; ++q) s[q] += sums[g][q][tid];
-            double fx = a.G * s[0], fy = a.G * s[1], fz = a.G * s[2];
-            if (a.ncentral > 0) {
-                const double hinv = 1.0 / ph, hinv3 = hinv * hinv * hinv;
-                double bx = 0.0, by = 0.0, bz = 0.0, bq = 0.0;
-                const double *c = a.c_in;
-                const int64_t k = a.ncentral;
-                for (int64_t u = 0; u < k; ++u)
-                    pair_f64<false>(c[u], c[k + u], c[2 * k + u], c[3 * k + u], (double)px, (double)py, (double)pz,
-                                    ph, hinv, hinv3, bx, by, bz, bq);
-                fx += bx * a.G;
-                fy += by * a.G;
-                fz += bz * a.G;
-            }
-            a.ax[j] = fx;
-            a.ay[j] = fy;
-            a.az[j] = fz;
-            const T c = (T)a.dt;
-            ux += (T)fx * c;
-            uy += (T)fy * c;
-            uz += (T)fz * c;
-            vx[j] = ux; vy[j] = uy; vz[j] = uz;
+            kick_particle<T>(a, j, s, px, py, pz, ph, ux, uy, uz);
         }
     }
     if (!a.drift || grp > 0) return;   // (a barrier waits for the waves that remain)
-    const double t_old = a.time[a.rd];
-    const double t_new = t_old + a.dt;
-    if (j == 0) a.time[a.wr] = t_new;
-    if (v) {
-        const T d = (T)(t_new - t_old);
-        px += ux * d;
-        py += uy * d;
-        pz += uz * d;
-        x[j] = px; y[j] = py; z[j] = pz;
-        if (a.ncentral > 0 && a.central[j]) {
-            for (int64_t u = 0; u < a.ncentral; ++u)
-                if (a.cidx[u] == j) {
-                    a.c_out[u] = (double)px;
-                    a.c_out[a.ncentral + u] = (double)py;
-                    a.c_out[2 * a.ncentral + u] = (double)pz;
-                    a.c_out[3 * a.ncentral + u] = (double)((const T *)a.m)[j];
-                }
-        }
-    }
+    drift_particle<T>(a, j, v, ux, uy, uz, px, py, pz);
     tile_box_block((double)px, (double)py, (double)pz, ph, v, a.box, a.sub, red);
     if constexpr (GEO) {
         double gx[1] = {(double)px}, gy[1] = {(double)py}, gz[1] = {(double)pz};
@@ -605,6 +633,100 @@ __global__ __launch_bounds__(BS * STEP_GROUPS) void k_step(StepArgs a) {
             for (int g = 0; g < 4; ++g) b[g] = __builtin_bit_cast(nb_u4v, Bg[g]);
         }
     }
+}
+
+// A whole step of a small system in one launch: k_force_wave's forces on targets
+// that share waves, then, in the workgroup that is the last of its 64 targets'
+// segments to arrive, k_step's sums, kick and drift of those targets.
+// The segments' sums cross XCDs: they are written and read as agent-scope
+// atomics, which pass the XCDs' L2s by, and a workgroup counts itself in
+// (arrived) once its own are written; the last one leaves the count at zero.
+// (Plain stores between agent-scope fences write back and invalidate an L2 per
+// workgroup: 4096 particles 175 us a step.)  Small systems are bound by the
+// chain of memory latencies from the targets' load to the new boxes.
+// A step in split precision, two launches -> one: 300 particles 13.8 -> 12.3 us,
+// 1000 14.4 -> 13.3, 2000 18.5 -> 15.5, 4096 26.5 -> 23.9, 8000 44.8 -> 43.0,
+// 30000 308 -> 304; FP32: 1000 13.3 -> 12.8, 4096 22.7 -> 19.4, 16001 87.1 ->
+// 86.5.  Five waves per SIMD: nothing spills.  Positions are double-buffered: other workgroups
+// still read the old ones.
+template <typename T>
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(5))) void k_force_step(ForceArgs<T> a,
+                                                                                           StepArgs st) {
+    __shared__ WaveStage<T> stage[NW];
+    __shared__ double red[NW - 1][3][64];
+    __shared__ int last;
+    static_assert(NW == STEP_GROUPS, "one wave per group of segments");
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    const int seg = logical / a.nblk_i;
+    const int ib = logical - seg * a.nblk_i;
+    const int64_t i0 = (int64_t)ib * 64, i = i0 + lane, ic = i < a.nt ? i : a.nt - 1;
+    int64_t j0 = (int64_t)seg * a.seg_len;
+    int64_t j1 = (j0 + a.seg_len < a.ns) ? j0 + a.seg_len : a.ns;
+    const int64_t part = a.seg_len / NW;
+    j0 = j0 + part * wave < j1 ? j0 + part * wave : j1;
+    j1 = j0 + part < j1 ? j0 + part : j1;
+    const T xt = a.tx[ic], yt = a.ty[ic], zt = a.tz[ic];
+    const double ph = a.th[ic];
+    double s[3], q;
+    wave_force<T, true, false, false, true>(stage[wave], xt, yt, zt, ph, a.tbox + (i0 / 64) * 8, a.sx, a.sy, a.sz, a.sm,
+                               a.skip_src, a.sub_box + (j0 / SB) * 8, a.tile_box, j0, j1, s[0], s[1], s[2], q);
+    auto add_waves = [&]() {   // the waves' sums, in order, in wave 0
+        if (wave > 0) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d) red[wave - 1][d][lane] = s[d];
+        }
+        __syncthreads();
+        if (wave > 0) return;
+#pragma unroll
+        for (int w = 0; w < NW - 1; ++w)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) s[d] += red[w][d][lane];
+    };
+    add_waves();
+    const bool v = i < a.nt;
+    T ux = 0, uy = 0, uz = 0;
+    if (wave == 0 && v) {   // (requested before the wait for the sums' stores)
+        ux = ((const T *)st.vx)[i];
+        uy = ((const T *)st.vy)[i];
+        uz = ((const T *)st.vz)[i];
+    }
+    if (a.nseg > 1) {
+        if (wave == 0 && v) {
+            double *p = a.part + (int64_t)seg * 4 * a.nt + i;
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+                __hip_atomic_store(p + d * a.nt, s[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (wave == 0) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's sums are written
+            if (lane == 0) {
+                last = __hip_atomic_fetch_add(st.arrived + ib, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                       (unsigned)a.nseg - 1;
+                if (last) st.arrived[ib] = 0;
+            }
+        }
+        __syncthreads();
+        if (!last) return;
+        s[0] = s[1] = s[2] = 0.0;
+        if (i < a.nt) group_sums<true>(a.part, a.nt, a.nseg, i, wave, s);
+        add_waves();
+    }
+    if (wave > 0) return;
+    T px = xt, py = yt, pz = zt;
+    if (v) kick_particle<T>(st, i, s, px, py, pz, ph, ux, uy, uz);
+    if (!st.drift) return;
+    drift_particle<T>(st, i, v, ux, uy, uz, px, py, pz);
+    const double p[3] = {(double)px, (double)py, (double)pz};
+    double *o = st.sub + (i0 / 64) * 8;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {   // the new box of these 64 (lanes without a particle: none)
+        const double lo = wave_min(v ? p[d] : DBL_MAX), hi = wave_max(v ? p[d] : -DBL_MAX);
+        if (lane == 0) { o[d] = lo; o[3 + d] = hi; }
+    }
+    const double hm = wave_max(v ? ph : 0.0);
+    if (lane == 0) o[6] = hm;
 }
 
 // ---------------------------------------------------------------------------
@@ -787,6 +909,16 @@ int launch_step(const StepArgs &a, bool is_double, hipStream_t s) {
 #undef NB_ST
     return check_launch("k_step");
 }
+
+template <typename T>
+static int force_step(ForceArgs<T> f, const StepArgs &st, hipStream_t s) {
+    if (f.nt <= 0) return NB_OK;
+    f.nblk_i = (int)((f.nt + 63) / 64);
+    k_force_step<T><<<(unsigned)((int64_t)f.nblk_i * f.nseg), BS, 0, s>>>(f, st);
+    return check_launch("k_force_step");
+}
+int launch_force_step(const ForceArgs<float> &f, const StepArgs &st, hipStream_t s) { return force_step(f, st, s); }
+int launch_force_step(const ForceArgs<double> &f, const StepArgs &st, hipStream_t s) { return force_step(f, st, s); }
 
 int launch_finalize(const double *part, int nseg, int64_t n, double G, double *ax, double *ay,
                     double *az, double *pot, bool with_pot, hipStream_t s, bool with_acc, const int64_t *idx) {

@@ -181,10 +181,17 @@ struct StepArgs {
     double *c_out;               // and where the drift stores the new ones
     double *time;
     int rd, wr;
-    double *box, *sub, *tgeo;
+    void *xn, *yn, *zn;          // where the drift puts the new positions (k_step: may be x, y, z)
+    double *box, *sub, *tgeo;    // box may be nullptr
     unsigned *tbg;
     int use_origin;
+    unsigned *arrived;           // k_force_step: [target groups], zeros between launches
 };
 int launch_step(const StepArgs &a, bool is_double, hipStream_t s);
+// The forces of far path 0 on targets that share waves (wave_split) and the
+// step of their particles in one launch (k_force_step); positions are read from
+// f and the drifted ones written to st.xn.. and st.sub, which no workgroup reads.
+int launch_force_step(const ForceArgs<float> &f, const StepArgs &st, hipStream_t s);
+int launch_force_step(const ForceArgs<double> &f, const StepArgs &st, hipStream_t s);
 
 }  // namespace nb

@@ -4,9 +4,11 @@ and save what the autotuner measured.
 
     python astronbodysim.jl_amd/tuning/make_table.py [out.json] [--modes=split,fp32,fp64]
 
-(the package directory's name has a dot, so it does not run with -m).  Sizes 2^12 .. 2^20 in the split mode on
-two-Plummer collisions (the benchmark's geometry), 2^12 .. 2^18 in the fp32
-mode and 2^12 .. 2^15 in the fp64 mode on Plummer spheres.  With --modes= only those modes are
+(the package directory's name has a dot, so it does not run with -m).  Entry k serves the sizes above
+2^(k-1) up to 2^k and is measured in their middle, 2^(k-1/2) (at 2^16 itself the
+far paths of the split mode tie, at 40000 path 0 is 15 % faster): k = 12 .. 20
+in the split mode on two-Plummer collisions (the benchmark's geometry),
+12 .. 18 in the fp32 mode and 12 .. 15 in the fp64 mode on Plummer spheres.  With --modes= only those modes are
 measured again and the table's other entries are kept.  Needs the GPU; a
 few minutes.
 """
@@ -36,7 +38,7 @@ def main(out=None, modes=None):
            [("fp64", k) for k in range(12, 16)]
     plan = [(m, k) for m, k in plan if not modes or m in modes]
     for mode, k in plan:
-        n = 1 << k
+        n = 2 * round(2 ** (k - 1.5))
         if mode == "split":
             pos, vel, mass = pkg.ics.collision(n // 2)
             h = 0.002
@@ -48,7 +50,7 @@ def main(out=None, modes=None):
         ctx.upload(pos, vel, mass)
         t0 = time.time()
         ctx.autotune()
-        print(f"{mode} N=2^{k}: {ctx.get_tuning()} ({time.time() - t0:.1f} s)", flush=True)
+        print(f"{mode} N={n}: {ctx.get_tuning()} ({time.time() - t0:.1f} s)", flush=True)
         ctx.close()
     nat.tuner_save(out)
     print("saved", out, flush=True)

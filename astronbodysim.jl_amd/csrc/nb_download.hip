@@ -6,8 +6,10 @@
 // about 10 GB/s.  Here the arrays go through DL_SLOTS pinned pieces of DL_PIECE
 // bytes: a kernel writes a piece over PCIe (27 us less than a copy command for
 // two small arrays) while the host empties those before it, and results of
-// 2 DL_SLOTS pieces or more are emptied by several threads, which is where the
-// page faults of a new array cost most.
+// DL_SLOTS pieces or more are emptied by several threads, which is where the
+// page faults of a new array cost most (two arrays of 3.6 MB, eight pieces: by
+// one thread 1.49 ms into new memory and 0.29 into used, by four 0.88 and 0.25;
+// six pieces 0.22 and 0.23).
 // Positions and velocities into new arrays, before -> after: 1000 particles
 // 69 -> 29 us, 4096 130 -> 33, 16001 82 -> 50, 65536 213 -> 135, 2^20
 // 5.2 -> 1.8 ms, 2.1e6 10.3 -> 3.5 ms (one thread 8.7, two 5.2, eight 3.4).
@@ -136,7 +138,7 @@ int copy_direct(const DownField *f, int nf, hipStream_t s) {
 int copy_pieces(const DownField *f, int nf, Block *b, size_t npieces, hipStream_t s) {
     // worker t empties the pieces t, t + T, ... once `ready` has passed them
     // (T = 1: the calling thread does)
-    const int T = npieces >= 2 * DL_SLOTS ? DL_THREADS : 1;
+    const int T = npieces >= DL_SLOTS ? DL_THREADS : 1;
     std::atomic<size_t> ready{0};
     std::atomic<size_t> emptied[DL_SLOTS];   // pieces emptied from each slot
     for (auto &e : emptied) e.store(0, std::memory_order_relaxed);

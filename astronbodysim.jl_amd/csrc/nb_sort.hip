@@ -109,12 +109,12 @@ __device__ __forceinline__ void gather_one(const GatherSet &g, int a, int64_t k,
     else ((uint8_t *)dst)[i] = ((const uint8_t *)g.arr[a])[k];
 }
 
+// (blockIdx.y: the array.  A loop over the arrays in each thread waited for one
+// array's loads after the other: the copy back of 1000 particles took 6.5 us.)
 __global__ void k_gather_set(GatherSet g, const int64_t *__restrict__ idx, int64_t n,
                              char *__restrict__ spare) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int64_t k = idx[i];
-    for (int a = 0; a < g.count; ++a) gather_one(g, a, k, i, spare);
+    if (i < n) gather_one(g, blockIdx.y, idx[i], i, spare);
 }
 
 // The whole order of a small system in one launch, up to the copy back: every
@@ -125,7 +125,8 @@ __global__ void k_gather_set(GatherSet g, const int64_t *__restrict__ idx, int64
 // with the box, key, sort, gather, permutation and copy kernels launched one by
 // one a re-sort was eight to ten of them, about 36 us; a step with one re-sort in
 // sixteen took 12.3 us at 300 particles, 13.3 at 1000, 24.0 at 4096 and 43.0 at
-// 8000 with them, 10.9, 11.9, 22.4 and 42.0 with this one and the copy back.
+// 8000 with them, 10.5, 11.6, 21.8 and 41.0 with this one (13 us at 1000, 22 at 4096) and the copy
+// back.
 // Every workgroup reads all positions, so the gain falls with n (and the keys
 // have to fit the LDS): RANK_UPTO.
 constexpr int RANK_WAVES = 16;
@@ -137,15 +138,26 @@ __global__ __launch_bounds__(64 * RANK_WAVES) void k_rank_gather(GatherSet g, co
     __shared__ uint64_t key[RANK_UPTO];
     __shared__ double red[RANK_WAVES][6];
     __shared__ int below[RANK_WAVES][64];
-    constexpr int TH = 64 * RANK_WAVES;
+    constexpr int TH = 64 * RANK_WAVES, PER = RANK_UPTO / TH;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    // the positions: all loads in flight at once (past the end: the last one's)
+    T p[PER][3];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        if (u * TH >= n) break;
+        const int i = u * TH + threadIdx.x < n ? u * TH + threadIdx.x : n - 1;
+        p[u][0] = x[i];
+        p[u][1] = y[i];
+        p[u][2] = z[i];
+    }
     double v[6] = {1e300, 1e300, 1e300, -1e300, -1e300, -1e300};
-    for (int i = threadIdx.x; i < n; i += TH) {
-        const double p[3] = {(double)x[i], (double)y[i], (double)z[i]};
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        if (u * TH >= n) break;
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            v[d] = fmin(v[d], p[d]);
-            v[3 + d] = fmax(v[3 + d], p[d]);
+            v[d] = fmin(v[d], (double)p[u][d]);
+            v[3 + d] = fmax(v[3 + d], (double)p[u][d]);
         }
     }
 #pragma unroll
@@ -158,6 +170,7 @@ __global__ __launch_bounds__(64 * RANK_WAVES) void k_rank_gather(GatherSet g, co
         for (int d = 0; d < 6; ++d) red[w][d] = v[d];
     }
     __syncthreads();
+#pragma unroll
     for (int u = 0; u < RANK_WAVES; ++u) {
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
@@ -165,9 +178,11 @@ __global__ __launch_bounds__(64 * RANK_WAVES) void k_rank_gather(GatherSet g, co
             v[3 + d] = fmax(v[3 + d], red[u][3 + d]);
         }
     }
-    for (int i = threadIdx.x; i < n; i += TH) {
-        const double p[3] = {(double)x[i], (double)y[i], (double)z[i]};
-        key[i] = morton_key(p, v);
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        if (u * TH >= n) break;
+        const double q[3] = {(double)p[u][0], (double)p[u][1], (double)p[u][2]};
+        if (u * TH + (int)threadIdx.x < n) key[u * TH + threadIdx.x] = morton_key(q, v);
     }
     __syncthreads();
     const int i0 = blockIdx.x * 64, i = i0 + lane;
@@ -175,11 +190,15 @@ __global__ __launch_bounds__(64 * RANK_WAVES) void k_rank_gather(GatherSet g, co
     const int per = (n + RANK_WAVES - 1) / RANK_WAVES;
     const int j0 = per * w < n ? per * w : n, j1 = j0 + per < n ? j0 + per : n;
     int count = 0;
-    // before these 64, among them, and after them
+    // before these 64, among them, and after them (one broadcast LDS read per key
+    // and wave; ballots over 64 keys at a time took twice as long)
     const int a1 = j1 < i0 ? j1 : i0;
+#pragma unroll 16
     for (int j = j0; j < a1; ++j) count += key[j] <= mine;
     const int b0 = j0 > i0 ? j0 : i0, b1 = j1 < i0 + 64 ? j1 : i0 + 64;
+#pragma unroll 4
     for (int j = b0; j < b1; ++j) count += key[j] < mine || (key[j] == mine && j < i);
+#pragma unroll 16
     for (int j = j0 > i0 + 64 ? j0 : i0 + 64; j < j1; ++j) count += key[j] < mine;
     below[w][lane] = count;
     __syncthreads();
@@ -193,12 +212,11 @@ __global__ __launch_bounds__(64 * RANK_WAVES) void k_rank_gather(GatherSet g, co
 __global__ void k_copy_back_set(GatherSet g, int64_t n, const char *__restrict__ spare) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    for (int a = 0; a < g.count; ++a) {
-        const char *src = spare + g.off[a];
-        if (g.size[a] == 8) ((uint64_t *)g.arr[a])[i] = ((const uint64_t *)src)[i];
-        else if (g.size[a] == 4) ((uint32_t *)g.arr[a])[i] = ((const uint32_t *)src)[i];
-        else ((uint8_t *)g.arr[a])[i] = ((const uint8_t *)src)[i];
-    }
+    const int a = blockIdx.y;
+    const char *src = spare + g.off[a];
+    if (g.size[a] == 8) ((uint64_t *)g.arr[a])[i] = ((const uint64_t *)src)[i];
+    else if (g.size[a] == 4) ((uint32_t *)g.arr[a])[i] = ((const uint32_t *)src)[i];
+    else ((uint8_t *)g.arr[a])[i] = ((const uint8_t *)src)[i];
 }
 
 // Bytes of spare buffer for the largest set, of 8-byte elements.
@@ -281,12 +299,12 @@ int morton_reorder(nb_ctx *c) {
             return check_launch("k_rank_gather");
         }
         NB_TRY(sort_keys(c));
-        k_gather_set<<<g, 256, 0, s>>>(set, S.idx + n, n, (char *)S.spare);
+        k_gather_set<<<dim3(g, set.count), 256, 0, s>>>(set, S.idx + n, n, (char *)S.spare);
         return check_launch("k_gather_set");
     };
     auto move = [&]() -> int {
         NB_TRY(gather());
-        k_copy_back_set<<<g, 256, 0, s>>>(set, n, (const char *)S.spare);
+        k_copy_back_set<<<dim3(g, set.count), 256, 0, s>>>(set, n, (const char *)S.spare);
         return check_launch("k_copy_back_set");
     };
     const int rc = move();

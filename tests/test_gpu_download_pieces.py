@@ -1,5 +1,5 @@
 """Results that reach the host in pinned pieces of 2^17 doubles, eight in flight,
-by several threads from sixteen on (needs an MI355X): whole arrays, on the edges
+by several threads from eight on (needs an MI355X): whole arrays, on the edges
 of a piece and of the slots, several downloads at a time.
 """
 import threading

@@ -132,6 +132,29 @@ int ensure_tbg(nb_ctx *c, const Geometry &g) {
 // sources alike, so that its sums have the same bits.
 constexpr int STEP_SEGMENTS = 16;
 
+// Up to this many particles a launch adds its segments' sums itself instead of
+// leaving them to k_finalize: force calls with their download 27.9 -> 26.3 us at
+// 300 particles, 41.0 -> 38.5 at 3000, 91.3 -> 89.4 at 10007 (split precision),
+// 44.2 -> 43.1 at 3000 and alike at 10007 in FP64; alike or slower from 20000 on.
+constexpr int64_t OWN_SUMS_UPTO = 16384;
+
+// The counters of launches that add their segments' sums themselves (zeros
+// between launches); before any capture.
+int ensure_arrived(nb_ctx *c) {
+    if (c->arrived || c->n <= 0) return NB_OK;
+    const size_t bytes = sizeof(unsigned) * (((size_t)c->n + 63) / 64);
+    unsigned *p = nullptr;
+    NB_TRY(dalloc(&p, bytes));
+    const hipError_t e = hipMemsetAsync(p, 0, bytes, c->stream);
+    if (e != hipSuccess) {
+        dfree(p);
+        set_error("hipMemsetAsync failed: %s", hipGetErrorString(e));
+        return NB_ERR_HIP;
+    }
+    c->arrived = p;
+    return NB_OK;
+}
+
 // The launch of the context's own forces or potentials.
 Geometry force_geometry(const nb_ctx *c, bool pot, bool acc) {
     if (c->mode == NB_MODE_FP64) return geometry(c->n, c->n, 1, c->tun.j_segments);
@@ -275,6 +298,13 @@ int run_force(nb_ctx *c, bool with_pot, bool allow_timing, bool allow_sort = tru
     const Geometry g = force_geometry(c, with_pot, !(with_pot && pot_only));
     NB_TRY(ensure_part(c, g.nseg));
     NB_TRY(ensure_tbg(c, g));
+    const bool acc_out = !(with_pot && pot_only) || f64;
+    // the step's kick takes the segments' sums (and the central bodies' terms)
+    // when nothing else adds to the accelerations
+    const bool leave = fuse && !with_pot && g.nseg > 1 && c->bg.empty() && !(c->mond_acc0 > 0.0);
+    // few targets: the launch adds its segments' sums itself
+    const bool fin = !leave && n <= OWN_SUMS_UPTO && g.nseg > 1 && (f64 ? f64_split(n, g.nseg) : (bool)g.wave_split);
+    if (fin) NB_TRY(ensure_arrived(c));
     hipEvent_t e0 = nullptr;
     if (allow_timing) NB_TRY(record_start(c, &e0));
     if (c->is_double) {
@@ -295,6 +325,7 @@ int run_force(nb_ctx *c, bool with_pot, bool allow_timing, bool allow_sort = tru
         a.G = c->G;
         a.ax = c->ax; a.ay = c->ay; a.az = c->az; a.pot = c->pot;
         a.part = c->part;
+        a.arrived = fin ? c->arrived : nullptr;
         a.skip_src = (c->mode == NB_MODE_SPLIT_CENTRAL && c->ncentral > 0) ? c->central : nullptr;
         a.accumulate = 0;
         if (!f64 && (!with_pot || pot_only) && far_path_weighted(c->tun.far_path)) {
@@ -321,9 +352,9 @@ int run_force(nb_ctx *c, bool with_pot, bool allow_timing, bool allow_sort = tru
         a.G = c->G;
         a.ax = c->ax; a.ay = c->ay; a.az = c->az; a.pot = c->pot;
         a.part = c->part;
+        a.arrived = fin ? c->arrived : nullptr;
         a.skip_src = nullptr;
         a.accumulate = 0;
-        const bool acc_out = !(with_pot && pot_only);
         if ((!with_pot || !acc_out) && c->tun.far_path == FAR_MFMA_BF16) {
             NB_TRY(ensure_source_weights(c));
             a.sw = c->wsrc;
@@ -331,17 +362,13 @@ int run_force(nb_ctx *c, bool with_pot, bool allow_timing, bool allow_sort = tru
         NB_TRY(launch_force_f32(a, tpt, with_pot, s, acc_out, c->tun.far_path));
     }
     if (allow_timing) NB_TRY(record_stop(c, e0));
-    // the step's kick takes the segments' sums (and the central bodies' terms)
-    // when nothing else adds to the accelerations
-    if (fuse && !with_pot && g.nseg > 1 && c->bg.empty() && !(c->mond_acc0 > 0.0)) {
+    if (leave) {
         fuse->left = true;
         fuse->nseg = g.nseg;
         return NB_OK;
     }
-    if (g.nseg > 1) {
-        NB_TRY(launch_finalize(c->part, g.nseg, n, c->G, c->ax, c->ay, c->az, c->pot, with_pot, s,
-                               !(with_pot && pot_only) || f64));
-    }
+    if (g.nseg > 1 && !fin)
+        NB_TRY(launch_finalize(c->part, g.nseg, n, c->G, c->ax, c->ay, c->az, c->pot, with_pot, s, acc_out));
     // FP64 central-body terms: every target, sources = the central particles.
     if (c->mode == NB_MODE_SPLIT_CENTRAL && c->ncentral > 0) {
         const int64_t k = c->ncentral;
@@ -936,23 +963,11 @@ static bool one_launch_steps(const nb_ctx *c) {
     return g.wave_split && (g.nseg > 1 || c->ncentral == 0);
 }
 
-// Their second set of positions and boxes, and the counters (zeros between
-// launches); before any capture.
+// Their second set of positions and boxes; before any capture.
 static int ensure_step2(nb_ctx *c) {
-    if (c->arrived) return NB_OK;
-    const size_t nn = (size_t)c->n, groups = (nn + 63) / 64;
-    dfree(c->xyz2); dfree(c->sub2);
-    NB_TRY(dalloc(&c->xyz2, (c->is_double ? sizeof(double) : sizeof(float)) * 3 * nn));
-    NB_TRY(dalloc(&c->sub2, sizeof(double) * 8 * NQ * ((nn + BS - 1) / BS)));
-    unsigned *arrived = nullptr;
-    NB_TRY(dalloc(&arrived, sizeof(unsigned) * groups));
-    const hipError_t e = hipMemsetAsync(arrived, 0, sizeof(unsigned) * groups, c->stream);
-    if (e != hipSuccess) {
-        dfree(arrived);
-        set_error("hipMemsetAsync failed: %s", hipGetErrorString(e));
-        return NB_ERR_HIP;
-    }
-    c->arrived = arrived;
+    const size_t nn = (size_t)c->n;
+    if (!c->xyz2) NB_TRY(dalloc(&c->xyz2, (c->is_double ? sizeof(double) : sizeof(float)) * 3 * nn));
+    if (!c->sub2) NB_TRY(dalloc(&c->sub2, sizeof(double) * 8 * NQ * ((nn + BS - 1) / BS)));
     return NB_OK;
 }
 
@@ -1026,6 +1041,7 @@ int nb_kdk_steps(nb_ctx *c, int64_t nsteps, double dt, double t_begin, int32_t u
             NB_TRY(ensure_tbg(c, g));
             if (weighted) NB_TRY(ensure_source_weights(c));
             const bool one = one_launch_steps(c);
+            NB_TRY(ensure_arrived(c));
             if (one) NB_TRY(ensure_step2(c));
             NB_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
             const int rc = !one ? enqueue_steps(c, 0, chunk, dt, false, false)

@@ -78,7 +78,7 @@ struct nb_ctx {
     size_t nflag_cap = 0;
     void *xyz2 = nullptr;         // 3n: the other positions of a run of k_force_step launches
     double *sub2 = nullptr;       // their quarter boxes
-    unsigned *arrived = nullptr;  // [64-target groups] workgroups counted in (k_force_step)
+    unsigned *arrived = nullptr;  // [64-target groups] workgroups counted in (last_arrival)
     double *part = nullptr;
     int part_cap = 0;             // segments the partial buffer holds
     double *stage = nullptr;      // 3n doubles

@@ -71,6 +71,84 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(MF == 4 ? 4 
     }
 }
 
+// Segments g, g + NW, ... of target i's partial sums (part: [nseg][4][n], from
+// the first of the NV values on), in order.
+// SHARED: other workgroups of this launch wrote them.
+template <bool SHARED, int NV>
+__device__ __forceinline__ void group_sums(const double *part, int64_t n, int nseg, int64_t i, int grp,
+                                           double (&s)[NV]) {
+    const double *p = part + i;
+    constexpr int U = 4;   // segments in flight; past the end: the last one's, not added
+    for (int g = grp; g < nseg; g += U * NW) {
+        double t[U][NV];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int gu = g + u * NW < nseg ? g + u * NW : nseg - 1;
+#pragma unroll
+            for (int q = 0; q < NV; ++q) {
+                const double *e = p + ((int64_t)gu * 4 + q) * n;
+                t[u][q] = SHARED ? __hip_atomic_load(e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *e;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (g + u * NW < nseg) {
+#pragma unroll
+                for (int q = 0; q < NV; ++q) s[q] += t[u][q];
+            }
+    }
+}
+
+// The waves' values, added in order in wave 0.
+template <int NV>
+__device__ __forceinline__ void add_waves(double (&s)[NV], double (&red)[NW - 1][NV][64]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (wave > 0) {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) red[wave - 1][q][lane] = s[q];
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int w = 0; w < NW - 1; ++w)
+#pragma unroll
+        for (int q = 0; q < NV; ++q) s[q] += red[w][q][lane];
+}
+
+// The sums over all segments of target i (v: it exists), s being segment seg's
+// in wave 0: true in wave 0 of the workgroup that is the last of its 64 targets'
+// to arrive, whose s they then are (added as k_finalize adds them).
+// The segments' sums cross XCDs: they are written and read as agent-scope
+// atomics, which pass the XCDs' L2s by, and a workgroup counts itself in
+// (arrived) once its own are written; the last one leaves the count at zero.
+// (Plain stores between agent-scope fences write back and invalidate an L2 per
+// workgroup: k_force_step on 4096 particles took 175 us.)
+template <int NV>
+__device__ __forceinline__ bool last_arrival(double (&s)[NV], double *part, int64_t n, int nseg, int seg, int64_t i,
+                                             bool v, unsigned *arrived, double (&red)[NW - 1][NV][64], int &last) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if (wave == 0) {
+        if (v) {
+            double *p = part + (int64_t)seg * 4 * n + i;
+#pragma unroll
+            for (int q = 0; q < NV; ++q) __hip_atomic_store(p + q * n, s[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's sums are written
+        if (lane == 0) {
+            last = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                   (unsigned)nseg - 1;
+            if (last) *arrived = 0;
+        }
+    }
+    __syncthreads();
+    if (!last) return false;
+#pragma unroll
+    for (int q = 0; q < NV; ++q) s[q] = 0.0;
+    if (v) group_sums<true>(part, n, nseg, i, wave, s);
+    add_waves(s, red);
+    return wave == 0;
+}
+
 // Far path 0 with one target per lane (wave_force).
 // split = 0: wave w of workgroup ib owns the targets 64 (NW ib + w).. and walks
 // the whole segment; the waves share the scalar cache's lines of its sources,
@@ -79,18 +157,21 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(MF == 4 ? 4 
 // of the segment each, down to 16 sources, and their sums meet in LDS in a
 // fixed order: the same waves on a quarter of the segments, so a quarter of the
 // partial sums to write and to add up.
+// FIN (split, several segments): the last workgroup of its 64 targets to arrive
+// adds the segments' sums (last_arrival), which spares the launch of k_finalize.
 // Held to 6 waves per SIMD (two values spilled outside the pair loops;
 // 5 without): 60000 particles in FP32 986 -> 929 us a force, 30011 in split
 // precision 312 -> 308 us.  Against the block-wide kernel that it replaced (one
 // force call with its boxes and segment sums, split precision, Plummer): 1000
 // particles 32 -> 12.5 us, 4096 35 -> 22, 16384 130 -> 106, 30011 333 -> 301;
 // FP32 60000 1030 -> 929.
-template <typename T, bool ACC, bool POT>
+template <typename T, bool ACC, bool POT, bool FIN>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(ACC &&POT && sizeof(T) == 8 ? 5 : 6)))
 void k_force_wave(ForceArgs<T> a, int split) {
     constexpr int NV = (ACC ? 3 : 0) + (POT ? 1 : 0);
     __shared__ WaveStage<T> st[NW];
     __shared__ double red[NW - 1][NV][64];
+    __shared__ int last;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int logical = xcd_remap(blockIdx.x, gridDim.x);
@@ -107,36 +188,35 @@ void k_force_wave(ForceArgs<T> a, int split) {
         j0 = j0 + part * wave < j1 ? j0 + part * wave : j1;
         j1 = j0 + part < j1 ? j0 + part : j1;
     }
+    constexpr int V0 = ACC ? 0 : 3;
     double v[4];   // ax, ay, az, pot
     wave_force<T, ACC, POT>(st[wave], a.tx[ic], a.ty[ic], a.tz[ic], a.th ? a.th[ic] : a.th_const,
                             a.tbox ? a.tbox + (i0 / 64) * 8 : nullptr, a.sx, a.sy, a.sz, a.sm, a.skip_src,
                             a.sub_box ? a.sub_box + (j0 / SB) * 8 : nullptr,
                             a.sub_box ? nullptr : a.tile_box + (j0 / BS) * 8, j0, j1, v[0], v[1], v[2], v[3]);
-    constexpr int V0 = ACC ? 0 : 3;
+    double s[NV];
+#pragma unroll
+    for (int q = 0; q < NV; ++q) s[q] = v[V0 + q];
     if (split) {
-        if (wave > 0) {
-#pragma unroll
-            for (int q = 0; q < NV; ++q) red[wave - 1][q][lane] = v[V0 + q];
+        add_waves(s, red);
+        if constexpr (FIN) {
+            if (!last_arrival(s, a.part + V0 * a.nt, a.nt, a.nseg, seg, i, i < a.nt, a.arrived + ib, red, last)) return;
+        } else {
+            if (wave > 0) return;
         }
-        __syncthreads();
-        if (wave > 0) return;
-#pragma unroll
-        for (int w = 0; w < NW - 1; ++w)
-#pragma unroll
-            for (int q = 0; q < NV; ++q) v[V0 + q] += red[w][q][lane];
     }
     if (i >= a.nt) return;
-    if (a.nseg == 1) {
+    if (FIN || a.nseg == 1) {
         if (ACC) {
-            a.ax[i] = a.G * v[0];
-            a.ay[i] = a.G * v[1];
-            a.az[i] = a.G * v[2];
+            a.ax[i] = a.G * s[0];
+            a.ay[i] = a.G * s[1];
+            a.az[i] = a.G * s[2];
         }
-        if (POT) a.pot[i] = -a.G * v[3];
+        if (POT) a.pot[i] = -a.G * s[NV - 1];
     } else {
         double *p = a.part + (int64_t)seg * 4 * a.nt;
 #pragma unroll
-        for (int q = 0; q < NV; ++q) p[(V0 + q) * a.nt + i] = v[V0 + q];
+        for (int q = 0; q < NV; ++q) p[(V0 + q) * a.nt + i] = s[q];
     }
 }
 
@@ -145,9 +225,16 @@ static void launch_wave(ForceArgs<T> a, bool pot, bool acc, hipStream_t s) {
     const int split = a.wave_split;
     if (split) a.nblk_i = (int)((a.nt + 63) / 64);
     const unsigned nb = (unsigned)((int64_t)a.nblk_i * a.nseg);
-    if (pot && acc) k_force_wave<T, true, true><<<nb, BS, 0, s>>>(a, split);
-    else if (pot) k_force_wave<T, false, true><<<nb, BS, 0, s>>>(a, split);
-    else k_force_wave<T, true, false><<<nb, BS, 0, s>>>(a, split);
+    const bool fin = split && a.nseg > 1 && a.arrived;
+#define NB_W(A_, P_)                                                       \
+    do {                                                                   \
+        if (fin) k_force_wave<T, A_, P_, true><<<nb, BS, 0, s>>>(a, split); \
+        else k_force_wave<T, A_, P_, false><<<nb, BS, 0, s>>>(a, split);    \
+    } while (0)
+    if (pot && acc) NB_W(true, true);
+    else if (pot) NB_W(false, true);
+    else NB_W(true, false);
+#undef NB_W
 }
 
 // Near pass of a split bf16 launch (forces only): one wavefront per
@@ -291,9 +378,12 @@ __device__ __forceinline__ void sources_f64(const double *__restrict__ sx, const
     for (; j < j1; ++j) pair_f64<POT>(sx[j], sy[j], sz[j], sm[j], xi, yi, zi, h, hinv, hinv3, Ax, Ay, Az, Aq);
 }
 
-template <bool POT>
+// FIN (split, several segments): as in k_force_wave.
+template <bool POT, bool FIN>
 __global__ __launch_bounds__(BS) void k_force_f64(ForceArgs<double> a, int split) {
-    __shared__ double red[NW - 1][POT ? 4 : 3][64];
+    constexpr int NV = POT ? 4 : 3;
+    __shared__ double red[NW - 1][NV][64];
+    __shared__ int last;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int logical = xcd_remap(blockIdx.x, gridDim.x);
@@ -313,25 +403,22 @@ __global__ __launch_bounds__(BS) void k_force_f64(ForceArgs<double> a, int split
     }
     sources_f64<POT>(a.sx, a.sy, a.sz, a.sm, j0, j1, xi, yi, zi, h, Ax, Ay, Az, Aq);
     if (split) {   // (uniform over the launch)
-        if (wave > 0) {
-            red[wave - 1][0][lane] = Ax;
-            red[wave - 1][1][lane] = Ay;
-            red[wave - 1][2][lane] = Az;
-            if (POT) red[wave - 1][POT ? 3 : 0][lane] = Aq;
+        double v[NV] = {Ax, Ay, Az};
+        if (POT) v[NV - 1] = Aq;
+        add_waves(v, red);
+        if constexpr (FIN) {
+            if (!last_arrival(v, a.part, a.nt, a.nseg, seg, i, valid, a.arrived + ib, red, last)) return;
+        } else {
+            if (wave > 0) return;
         }
-        __syncthreads();
-        if (wave > 0) return;
-#pragma unroll
-        for (int w = 0; w < NW - 1; ++w) {
-            Ax += red[w][0][lane];
-            Ay += red[w][1][lane];
-            Az += red[w][2][lane];
-            if (POT) Aq += red[w][POT ? 3 : 0][lane];
-        }
+        Ax = v[0];
+        Ay = v[1];
+        Az = v[2];
+        if (POT) Aq = v[NV - 1];
     }
     if (!valid) return;
-    if (a.nseg == 1) {
-        if (a.accumulate) {
+    if (FIN || a.nseg == 1) {
+        if (!FIN && a.accumulate) {
             a.ax[i] += Ax * a.G;
             a.ay[i] += Ay * a.G;
             a.az[i] += Az * a.G;
@@ -537,34 +624,6 @@ __device__ __forceinline__ void drift_particle(const StepArgs &a, int64_t j, boo
     }
 }
 
-// Segments g, g + STEP_GROUPS, ... of target i's partial sums, in order.
-// SHARED: other workgroups of this launch wrote them.
-constexpr int STEP_GROUPS = 4;
-template <bool SHARED>
-__device__ __forceinline__ void group_sums(const double *part, int64_t n, int nseg, int64_t i, int grp,
-                                           double (&s)[3]) {
-    const double *p = part + i;
-    constexpr int U = 4;   // segments in flight; past the end: the last one's, not added
-    for (int g = grp; g < nseg; g += U * STEP_GROUPS) {
-        double t[U][3];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int gu = g + u * STEP_GROUPS < nseg ? g + u * STEP_GROUPS : nseg - 1;
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                const double *e = p + ((int64_t)gu * 4 + q) * n;
-                t[u][q] = SHARED ? __hip_atomic_load(e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *e;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (g + u * STEP_GROUPS < nseg) {
-#pragma unroll
-                for (int q = 0; q < 3; ++q) s[q] += t[u][q];
-            }
-    }
-}
-
 // The per-particle part of a KDK step, between one force launch and the next
 // (one workgroup per 256 particles): the sums of the force's segments, the
 // central bodies' FP64 terms and the kick (a.kick), then the next step's drift
@@ -581,6 +640,7 @@ __device__ __forceinline__ void group_sums(const double *part, int64_t n, int ns
 //          to time[wr] (rd != wr)
 // The central bodies' terms read their positions from c_in, and the drift
 // leaves the new ones in c_out: other workgroups still read the old ones.
+constexpr int STEP_GROUPS = NW;   // (the groups of group_sums)
 template <typename T, bool GEO, bool ROWS>
 __global__ __launch_bounds__(BS * STEP_GROUPS) void k_step(StepArgs a) {
     __shared__ double sums[STEP_GROUPS - 1][3][BS];
@@ -599,7 +659,7 @@ __global__ __launch_bounds__(BS * STEP_GROUPS) void k_step(StepArgs a) {
     }
     if (a.kick) {
         double s[3] = {0.0, 0.0, 0.0};
-        if (v) group_sums<false>(a.part, a.n, a.nseg, j, grp, s);
+        if (v) group_sums<false, 3>(a.part, a.n, a.nseg, j, grp, s);
         if (grp > 0) {
 #pragma unroll
             for (int q = 0; q < 3; ++q) sums[grp - 1][q][tid] = s[q];
@@ -638,24 +698,20 @@ __global__ __launch_bounds__(BS * STEP_GROUPS) void k_step(StepArgs a) {
 // A whole step of a small system in one launch: k_force_wave's forces on targets
 // that share waves, then, in the workgroup that is the last of its 64 targets'
 // segments to arrive, k_step's sums, kick and drift of those targets.
-// The segments' sums cross XCDs: they are written and read as agent-scope
-// atomics, which pass the XCDs' L2s by, and a workgroup counts itself in
-// (arrived) once its own are written; the last one leaves the count at zero.
-// (Plain stores between agent-scope fences write back and invalidate an L2 per
-// workgroup: 4096 particles 175 us a step.)  Small systems are bound by the
-// chain of memory latencies from the targets' load to the new boxes.
+// Positions are double-buffered: other workgroups still read the old ones.
+// Small systems are bound by the chain of memory latencies from the targets'
+// load to the new boxes.
 // A step in split precision, two launches -> one: 300 particles 13.8 -> 12.3 us,
 // 1000 14.4 -> 13.3, 2000 18.5 -> 15.5, 4096 26.5 -> 23.9, 8000 44.8 -> 43.0,
 // 30000 308 -> 304; FP32: 1000 13.3 -> 12.8, 4096 22.7 -> 19.4, 16001 87.1 ->
-// 86.5.  Five waves per SIMD: nothing spills.  Positions are double-buffered: other workgroups
-// still read the old ones.
+// 86.5 (with re-sorts that have become shorter since: 9.9, 11.5, 12.8, 20.8 and
+// 40.1 us at 300 to 8000).
 template <typename T>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(5))) void k_force_step(ForceArgs<T> a,
                                                                                            StepArgs st) {
     __shared__ WaveStage<T> stage[NW];
     __shared__ double red[NW - 1][3][64];
     __shared__ int last;
-    static_assert(NW == STEP_GROUPS, "one wave per group of segments");
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int logical = xcd_remap(blockIdx.x, gridDim.x);
@@ -672,19 +728,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(5))) void k_
     double s[3], q;
     wave_force<T, true, false, false, true>(stage[wave], xt, yt, zt, ph, a.tbox + (i0 / 64) * 8, a.sx, a.sy, a.sz, a.sm,
                                a.skip_src, a.sub_box + (j0 / SB) * 8, a.tile_box, j0, j1, s[0], s[1], s[2], q);
-    auto add_waves = [&]() {   // the waves' sums, in order, in wave 0
-        if (wave > 0) {
-#pragma unroll
-            for (int d = 0; d < 3; ++d) red[wave - 1][d][lane] = s[d];
-        }
-        __syncthreads();
-        if (wave > 0) return;
-#pragma unroll
-        for (int w = 0; w < NW - 1; ++w)
-#pragma unroll
-            for (int d = 0; d < 3; ++d) s[d] += red[w][d][lane];
-    };
-    add_waves();
+    add_waves(s, red);
     const bool v = i < a.nt;
     T ux = 0, uy = 0, uz = 0;
     if (wave == 0 && v) {   // (requested before the wait for the sums' stores)
@@ -692,28 +736,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(5))) void k_
         uy = ((const T *)st.vy)[i];
         uz = ((const T *)st.vz)[i];
     }
-    if (a.nseg > 1) {
-        if (wave == 0 && v) {
-            double *p = a.part + (int64_t)seg * 4 * a.nt + i;
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-                __hip_atomic_store(p + d * a.nt, s[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (wave == 0) {
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's sums are written
-            if (lane == 0) {
-                last = __hip_atomic_fetch_add(st.arrived + ib, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                       (unsigned)a.nseg - 1;
-                if (last) st.arrived[ib] = 0;
-            }
-        }
-        __syncthreads();
-        if (!last) return;
-        s[0] = s[1] = s[2] = 0.0;
-        if (i < a.nt) group_sums<true>(a.part, a.nt, a.nseg, i, wave, s);
-        add_waves();
-    }
-    if (wave > 0) return;
+    if (a.nseg == 1 ? wave > 0 : !last_arrival(s, a.part, a.nt, a.nseg, seg, i, v, st.arrived + ib, red, last)) return;
     T px = xt, py = yt, pz = zt;
     if (v) kick_particle<T>(st, i, s, px, py, pz, ph, ux, uy, uz);
     if (!st.drift) return;
@@ -884,13 +907,14 @@ int launch_source_weights(const void *m, bool is_double, int64_t n, float *w, hi
 int launch_force_f64(const ForceArgs<double> &a_in, bool pot, hipStream_t s) {
     ForceArgs<double> a = a_in;
     if (a.nt <= 0 || a.nseg <= 0) return NB_OK;
-    // 64 targets per workgroup while the launch stays under 2^22 workgroups
-    const int64_t n64 = (a.nt + 63) / 64;
-    const int split = n64 * a.nseg <= (1 << 22);
-    a.nblk_i = (int)(split ? n64 : (a.nt + BS - 1) / BS);
-    const int64_t nb = (int64_t)a.nblk_i * a.nseg;
-    if (pot) k_force_f64<true><<<(unsigned)nb, BS, 0, s>>>(a, split);
-    else k_force_f64<false><<<(unsigned)nb, BS, 0, s>>>(a, split);
+    const int split = f64_split(a.nt, a.nseg);
+    a.nblk_i = (int)(split ? (a.nt + 63) / 64 : (a.nt + BS - 1) / BS);
+    const unsigned nb = (unsigned)((int64_t)a.nblk_i * a.nseg);
+    const bool fin = split && a.nseg > 1 && a.arrived;
+    if (pot && fin) k_force_f64<true, true><<<nb, BS, 0, s>>>(a, split);
+    else if (pot) k_force_f64<true, false><<<nb, BS, 0, s>>>(a, split);
+    else if (fin) k_force_f64<false, true><<<nb, BS, 0, s>>>(a, split);
+    else k_force_f64<false, false><<<nb, BS, 0, s>>>(a, split);
     return check_launch("k_force_f64");
 }
 

@@ -67,6 +67,8 @@ struct ForceArgs {
     double G;
     double *ax, *ay, *az, *pot;  // final outputs (nseg == 1)
     double *part;                // partials [nseg][4][nt] (nseg > 1)
+    unsigned *arrived;           // [64-target groups], zeros between launches: where the waves of a workgroup
+                                 // share targets, the launch adds the segments' sums itself; or nullptr
     const uint8_t *skip_src;     // sources excluded from the FP32 sum (central bodies) or nullptr
     int accumulate;              // 1: add G*sum to the outputs instead of storing (nseg == 1)
     const float *sw;             // source weights m^(-2/3) (far paths 3 and 4) or nullptr
@@ -134,6 +136,10 @@ inline Geometry wave_launch_geometry(int64_t nt, int64_t ns, int64_t want_seg, i
     return g;
 }
 
+// Whether the waves of k_force_f64's workgroups share 64 targets: while the
+// launch stays under 2^22 workgroups.
+inline bool f64_split(int64_t nt, int nseg) { return (nt + 63) / 64 * nseg <= (1 << 22); }
+
 // Passes of the force kernel (force_block): every tile, or the far tiles
 // only (the split bf16 matrix-core launch, whose near tiles k_force_near adds).
 constexpr int PASS_ALL = 0;
@@ -185,7 +191,7 @@ struct StepArgs {
     double *box, *sub, *tgeo;    // box may be nullptr
     unsigned *tbg;
     int use_origin;
-    unsigned *arrived;           // k_force_step: [target groups], zeros between launches
+    unsigned *arrived;           // k_force_step: as in ForceArgs
 };
 int launch_step(const StepArgs &a, bool is_double, hipStream_t s);
 // The forces of far path 0 on targets that share waves (wave_split) and the

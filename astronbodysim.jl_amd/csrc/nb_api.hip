@@ -157,7 +157,7 @@ int ensure_arrived(nb_ctx *c) {
 
 // The launch of the context's own forces or potentials.
 Geometry force_geometry(const nb_ctx *c, bool pot, bool acc) {
-    if (c->mode == NB_MODE_FP64) return geometry(c->n, c->n, 1, c->tun.j_segments);
+    if (c->mode == NB_MODE_FP64) return f64_launch_geometry(c->n, c->n, c->tun.j_segments);
     if (wave_path(c->tun.far_path, c->tun.targets_per_thread, pot, acc))
         return wave_launch_geometry(c->n, c->n, c->tun.j_segments, pot ? WAVE_SEGMENTS : STEP_SEGMENTS);
     return geometry(c->n, c->n, c->tun.targets_per_thread, c->tun.j_segments);

@@ -136,6 +136,23 @@ inline Geometry wave_launch_geometry(int64_t nt, int64_t ns, int64_t want_seg, i
     return g;
 }
 
+// A k_force_f64 launch: segments of whole tiles, or, for few targets, of quarters
+// until the chip has about WAVE_FILL workgroups (at 1000 particles four tiles
+// gave 64 workgroups of four waves with 62 sources each).  A force call with its
+// download: 300 to 1000 particles 40.5 -> 34 us, 3000 47.9 -> 43.7; on device
+// arrays: 700 21.8 -> 18.8, 3000 28.5 -> 23.3; alike from 5000 on.
+inline Geometry f64_launch_geometry(int64_t nt, int64_t ns, int64_t want_seg, int64_t max_seg = WAVE_SEGMENTS) {
+    Geometry g = geometry(nt, ns, 1, want_seg);
+    const int64_t groups = std::max<int64_t>((nt + 63) / 64, 1), nq = std::max<int64_t>((ns + SB - 1) / SB, 1);
+    const int64_t fill = std::min<int64_t>(std::min<int64_t>((WAVE_FILL + groups - 1) / groups, max_seg), nq);
+    if (fill > g.nseg) {
+        const int64_t qs = (nq + fill - 1) / fill;
+        g.seg_len = qs * SB;
+        g.nseg = (int)((nq + qs - 1) / qs);
+    }
+    return g;
+}
+
 // Whether the waves of k_force_f64's workgroups share 64 targets: while the
 // launch stays under 2^22 workgroups.
 inline bool f64_split(int64_t nt, int nseg) { return (nt + 63) / 64 * nseg <= (1 << 22); }

@@ -101,6 +101,7 @@ extern "C" int nb_compute_force_noalloc(int32_t precision_mode, int64_t n, const
     const int64_t fit = (int64_t)((SCRATCH_BYTES - box_bytes) / seg_bytes);
     const int64_t want = std::min<int64_t>(std::min<int64_t>(std::max<int64_t>((8192 + nblk - 1) / nblk, 1), 64), fit);
     const Geometry g = quarters ? wave_launch_geometry(n, n, 1, std::max<int64_t>(std::min<int64_t>(want, fit), 1))
+                       : f64    ? f64_launch_geometry(n, n, want, std::min<int64_t>(fit, WAVE_SEGMENTS))
                                 : geometry(n, n, 1, want);
     double *box = (double *)base;
     double *part = g.nseg > 1 ? (double *)((unsigned char *)base + box_bytes) : nullptr;

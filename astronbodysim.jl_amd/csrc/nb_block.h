@@ -26,17 +26,37 @@ __device__ __forceinline__ V wave_sum(V v) {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     return v;
 }
-template <typename V>
-__device__ __forceinline__ V wave_min(V v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_xor(v, off, 64));
-    return v;
+// The smallest and largest FP64 value of a wavefront, in every lane: six DPP
+// steps (within rows of 16, then across them; a lane without a source keeps its
+// own value) and a read of lane 63.  Through __shfl_xor each step was two LDS
+// permutes and their latency: the seven reductions of 64 particles' box took
+// about 0.3 us at the end of a step, and in k_rank_gather the LDS was the bound.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_f64(double v) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const int lo = (int)(unsigned)b, hi = (int)(unsigned)(b >> 32);
+    const unsigned l = (unsigned)__builtin_amdgcn_update_dpp(lo, lo, CTRL, ROWS, 0xf, false);
+    const unsigned h = (unsigned)__builtin_amdgcn_update_dpp(hi, hi, CTRL, ROWS, 0xf, false);
+    return __builtin_bit_cast(double, (unsigned long long)h << 32 | l);
 }
-template <typename V>
-__device__ __forceinline__ V wave_max(V v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-    return v;
+template <typename F>
+__device__ __forceinline__ double wave_reduce_f64(double v, F op) {
+    v = op(v, dpp_f64<0x111, 0xf>(v));   // row_shr:1
+    v = op(v, dpp_f64<0x112, 0xf>(v));   // row_shr:2
+    v = op(v, dpp_f64<0x114, 0xf>(v));   // row_shr:4
+    v = op(v, dpp_f64<0x118, 0xf>(v));   // row_shr:8
+    v = op(v, dpp_f64<0x142, 0xa>(v));   // row_bcast:15, to rows 1 and 3
+    v = op(v, dpp_f64<0x143, 0xc>(v));   // row_bcast:31, to rows 2 and 3
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, 63);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), 63);
+    return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+}
+__device__ __forceinline__ double wave_min(double v) {
+    return wave_reduce_f64(v, [](double p, double q) { return fmin(p, q); });
+}
+__device__ __forceinline__ double wave_max(double v) {
+    return wave_reduce_f64(v, [](double p, double q) { return fmax(p, q); });
 }
 
 // Block statistics of the targets: centroid, bounding box, largest h.

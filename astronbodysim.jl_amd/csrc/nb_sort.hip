@@ -171,12 +171,9 @@ __global__ __launch_bounds__(64 * RANK_WAVES) void k_rank_gather(GatherSet g, co
     }
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < RANK_WAVES; ++u) {
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            v[d] = fmin(v[d], red[u][d]);
-            v[3 + d] = fmax(v[3 + d], red[u][3 + d]);
-        }
+    for (int d = 0; d < 3; ++d) {   // (one wave's result per lane, repeated)
+        v[d] = wave_min(red[lane % RANK_WAVES][d]);
+        v[3 + d] = wave_max(red[lane % RANK_WAVES][3 + d]);
     }
 #pragma unroll
     for (int u = 0; u < PER; ++u) {

@@ -704,8 +704,8 @@ __global__ __launch_bounds__(BS * STEP_GROUPS) void k_step(StepArgs a) {
 // A step in split precision, two launches -> one: 300 particles 13.8 -> 12.3 us,
 // 1000 14.4 -> 13.3, 2000 18.5 -> 15.5, 4096 26.5 -> 23.9, 8000 44.8 -> 43.0,
 // 30000 308 -> 304; FP32: 1000 13.3 -> 12.8, 4096 22.7 -> 19.4, 16001 87.1 ->
-// 86.5 (with re-sorts that have become shorter since: 9.9, 11.5, 12.8, 20.8 and
-// 40.1 us at 300 to 8000).
+// 86.5 (with shorter re-sorts and DPP reductions since then: 9.3, 10.9, 12.4,
+// 20.3 and 39.9 us at 300 to 8000).
 template <typename T>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(5))) void k_force_step(ForceArgs<T> a,
                                                                                            StepArgs st) {

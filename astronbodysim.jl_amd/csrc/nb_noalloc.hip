@@ -2,8 +2,8 @@
 // arrays the caller already holds in device memory, with no device allocation.
 //
 // The kernels are the ones nb_compute_force launches (k_tile_boxes,
-// k_force_f32 / k_force_f64, k_finalize).  Their scratch -- the bounding box
-// of every 256-source tile and, with several source segments, the
+// k_force_wave / k_force_f64, k_finalize).  Their scratch -- the bounding boxes
+// of the 64-source quarters (or 256-source tiles) and, with several source segments, the
 // per-segment partial sums -- lives in one file-scope device array instead of
 // context buffers.  Each GPU holds its own copy of that array for the life of
 // the process; its address is looked up once per device with

@@ -1,6 +1,6 @@
 // nb_wave.h -- the wavefront-level all-pairs routine of far path 0 with one
 // target per lane, shared by the one-system kernel (nb_force.hip) and the
-// ragged ensemble kernel (nb_batch.hip).
+// ragged ensemble kernel (nb_batch_wave.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <float.h>

@@ -9,10 +9,12 @@
 namespace nb {
 
 // Far path 0 with one target per lane (wave_force): one workgroup per quarter
-// (64 targets) of an item, whose W waves take a part of the system's sources
-// each, by whole tiles; their sums meet in LDS in a fixed order.  The origins,
-// classes and FP32 sums of a tile are force_block's, so the results are too (but
-// for the order of the FP64 sums).  Bound by FP32 VALU issue on large
+// (64 targets) of an item.  The system's source tiles are cut into PARTS parts,
+// of which each of the W waves takes PARTS / W, one after the other; a part's FP64
+// sums are its own and the parts' are added in order, so a system's bits depend
+// on the system alone, not on W, which follows from the size of the whole
+// ensemble.  The origins, classes and FP32 sums of a tile are force_block's, so
+// the results are too (but for the order of the FP64 sums).  Bound by FP32 VALU issue on large
 // ensembles (2.85e12 pairs/s on the 512 clusters below); the block-wide
 // persistent kernel that it replaced held a workgroup at its barriers for the
 // slowest of four waves, and a small ensemble gave it few waves with long
@@ -28,13 +30,14 @@ namespace nb {
 // log-uniform): 512 clusters 6.05 -> 5.76 ms, 200 2.16 -> 1.85, 64 1.21 -> 0.74,
 // 32 1.05 -> 0.48, 8 0.98 -> 0.30, one of 3271 0.223 -> 0.055 ms.
 constexpr unsigned ITEM_RUN = 16, XCDS = 8;
+constexpr int PARTS = 8;   // (of one tile at least: a system of few tiles has empty ones)
 template <bool ACC, bool POT, int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(ACC &&POT ? 5 : 6)))
 void k_batch_wave(BatchArgs a) {
     constexpr int NV = (ACC ? 3 : 0) + (POT ? 1 : 0);
     constexpr int V0 = ACC ? 0 : 3;
     __shared__ WaveStage<double> st[W];
-    __shared__ double red[W - 1][NV][64];
+    __shared__ double red[PARTS][NV][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     unsigned b = blockIdx.x;
@@ -50,25 +53,31 @@ void k_batch_wave(BatchArgs a) {
     if (i0 >= o1) return;   // (the whole workgroup)
     const int64_t i = i0 + lane;
     const int64_t ic = i < o1 ? i : o1 - 1;
-    const int64_t part = ((o1 - o0 + BS - 1) / BS + W - 1) / W * BS;
-    const int64_t j0 = o0 + part * wave < o1 ? o0 + part * wave : o1;
-    const int64_t j1 = j0 + part < o1 ? j0 + part : o1;
-    const int64_t tb = a.tile_base[s];
+    const int64_t tb = a.tile_base[s], nt = (o1 - o0 + BS - 1) / BS;
+    const auto part = [&](int g) { return o0 + nt * g / PARTS * BS; };   // its first source
+    constexpr int MINE = PARTS / W;
+    static_assert(MINE == 1 || MINE == 2, "a wave takes one part or two");
+    const int g0 = wave * MINE;
+    const int64_t j0 = part(g0), j1 = g0 + MINE < PARTS ? part(g0 + MINE) : o1;
     double v[4];   // ax, ay, az, pot
+    if (MINE == 2) {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) red[g0][q][lane] = 0.0;   // (an empty first part)
+    }
     wave_force<double, ACC, POT, true>(st[wave], a.x[ic], a.y[ic], a.z[ic], a.h[ic], nullptr, a.x, a.y, a.z, a.m,
                                        a.skip_src, a.sub_box + (tb * NQ + (j0 - o0) / SB) * 8, a.tile_box, j0, j1,
-                                       v[0], v[1], v[2], v[3], a.tgeo + (tb + qt / NQ) * TG_STRIDE,
-                                       (int)(qt % NQ));
-    if (wave > 0) {
+                                       v[0], v[1], v[2], v[3], a.tgeo + (tb + qt / NQ) * TG_STRIDE, (int)(qt % NQ),
+                                       MINE == 2 ? (int)((part(g0 + 1) - j0) / SB) - 1 : -1, red[g0]);
 #pragma unroll
-        for (int q = 0; q < NV; ++q) red[wave - 1][q][lane] = v[V0 + q];
-    }
+    for (int q = 0; q < NV; ++q) red[g0 + MINE - 1][q][lane] = v[V0 + q];
     __syncthreads();
     if (wave > 0) return;
 #pragma unroll
-    for (int w = 0; w < W - 1; ++w)
+    for (int q = 0; q < NV; ++q) v[V0 + q] = red[0][q][lane];
 #pragma unroll
-        for (int q = 0; q < NV; ++q) v[V0 + q] += red[w][q][lane];
+    for (int g = 1; g < PARTS; ++g)
+#pragma unroll
+        for (int q = 0; q < NV; ++q) v[V0 + q] += red[g][q][lane];
     if (i >= o1) return;
     const double G = a.Gs[s];
     if (ACC) {

@@ -144,7 +144,8 @@ __device__ __forceinline__ void near_sources(scalar_ptr<T> sx, scalar_ptr<T> sy,
 // on, or, when null, tile_box: the boxes of the BS-source tiles from j0 on.
 // TILES: the origin, box and classes are those of the targets' block (tgeo, its
 // stored record, and the wave's place gw in it) and the FP32 sums run over a
-// whole tile (j0 starts one), as in force_block, whose sums these then are.
+// whole tile (j0 starts one), as in force_block, whose sums these then are.  After
+// quarter qm, the last of a tile, the sums so far go to mid and start again.
 // EARLY (with sub_box): the first quarter's sources and the boxes of the first 64 quarters (one
 // per lane) are requested before anything waits for the targets, in 15 more
 // registers (4096 particles 24.5 -> 23.9 us a step of k_force_step; at six
@@ -158,7 +159,8 @@ __device__ __forceinline__ void wave_force(WaveStage<T> &st, T xt, T yt, T zt, d
                                            const double *__restrict__ sub_box,
                                            const double *__restrict__ tile_box, int64_t j0, int64_t j1,
                                            double &Ax, double &Ay, double &Az, double &Aq,
-                                           const double *__restrict__ tgeo = nullptr, int gw = 0) {
+                                           const double *__restrict__ tgeo = nullptr, int gw = 0, int qm = -1,
+                                           double (*mid)[64] = nullptr) {
     constexpr bool D = WaveStage<T>::D;
     const int lane = threadIdx.x & 63;
     // the next quarter's sources are loaded while the current one is computed
@@ -280,6 +282,11 @@ __device__ __forceinline__ void wave_force(WaveStage<T> &st, T xt, T yt, T zt, d
         if (ACC) { Ax += (double)ax; Ay += (double)ay; Az += (double)az; }
         if (POT) Aq += (double)aq;
         ax = ay = az = aq = 0.0f;
+        if (TILES && q == qm) {
+            if (ACC) { mid[0][lane] = Ax; mid[1][lane] = Ay; mid[2][lane] = Az; }
+            if (POT) mid[ACC ? 3 : 0][lane] = Aq;
+            Ax = Ay = Az = Aq = 0.0;
+        }
     }
 }
 

@@ -100,7 +100,7 @@ struct BatchArgs {
 };
 
 // nb_batch_wave.hip: the FP32-pair sums of every item on far path 0 with one
-// target per lane.
-int launch_batch_wave(const BatchArgs &a, bool pot, bool acc, hipStream_t s);
+// target per lane; blocks > 0: by at most that many workgroups.
+int launch_batch_wave(const BatchArgs &a, int blocks, bool pot, bool acc, hipStream_t s);
 
 }  // namespace nb

@@ -1119,7 +1119,7 @@ static int bforce(nb_batch *b, bool with_pot, bool allow_timing, bool pot_only =
             a.w = b->wsrc;
         }
         if (wave) {
-            NB_TRY(launch_batch_wave(a, with_pot, !pot_only, s));
+            NB_TRY(launch_batch_wave(a, b->tun.blocks, with_pot, !pot_only, s));
         } else {
             int nblk = b->tun.blocks > 0 ? b->tun.blocks : 8 * b->cu_count;
             nblk = (int)std::max<int64_t>(1, std::min<int64_t>(nblk, b->nitems));
@@ -1992,10 +1992,12 @@ int nb_batch_autotune(nb_batch *b) {
     // (targets per thread, far path) as in the one-system autotuner
     const int cand[9][2] = {{1, 0}, {2, 0}, {4, 0}, {1, 3}, {2, 3}, {4, 3}, {1, 4}, {1, 1}, {1, 2}};
     for (int ti = 0; ti < 9 && rc == NB_OK; ++ti) {
-        for (int mi = 0; mi < 4 && rc == NB_OK; ++mi) {
+        // (k_batch_wave wants a workgroup per 64 targets: fewer only bound it)
+        const bool wave = wave_path(cand[ti][1], cand[ti][0], false, true);
+        for (int mi = 0; mi < (wave ? 1 : 4) && rc == NB_OK; ++mi) {
             b->tun.targets_per_thread = cand[ti][0];
             b->tun.far_path = cand[ti][1];
-            b->tun.blocks = mult[mi] * b->cu_count;
+            b->tun.blocks = wave ? 0 : mult[mi] * b->cu_count;
             rc = bforce(b, false, false);
             if (rc) break;
             (void)hipEventRecord(e0, b->stream);

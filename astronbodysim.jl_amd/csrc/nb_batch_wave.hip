@@ -31,20 +31,17 @@ namespace nb {
 // 32 1.05 -> 0.48, 8 0.98 -> 0.30, one of 3271 0.223 -> 0.055 ms.
 constexpr unsigned ITEM_RUN = 16, XCDS = 8;
 constexpr int PARTS = 8;   // (of one tile at least: a system of few tiles has empty ones)
+template <bool ACC, bool POT>
+constexpr int NVALUES = (ACC ? 3 : 0) + (POT ? 1 : 0);
+
+// The sums of quarter b of the items, by a whole workgroup.
 template <bool ACC, bool POT, int W>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(ACC &&POT ? 5 : 6)))
-void k_batch_wave(BatchArgs a) {
-    constexpr int NV = (ACC ? 3 : 0) + (POT ? 1 : 0);
+__device__ __forceinline__ void item_quarter(const BatchArgs &a, unsigned b, WaveStage<double> (&st)[W],
+                                             double (&red)[PARTS][NVALUES<ACC, POT>][64]) {
+    constexpr int NV = NVALUES<ACC, POT>;
     constexpr int V0 = ACC ? 0 : 3;
-    __shared__ WaveStage<double> st[W];
-    __shared__ double red[PARTS][NV][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    unsigned b = blockIdx.x;
-    if (b < gridDim.x / (ITEM_RUN * XCDS) * (ITEM_RUN * XCDS)) {
-        const unsigned slot = b / XCDS;
-        b = (slot / ITEM_RUN * XCDS + b % XCDS) * ITEM_RUN + slot % ITEM_RUN;
-    }
     const int64_t item = a.items[b / NQ];
     const int s = (int)(item >> 32);
     const int64_t o0 = a.off[s], o1 = a.off[s + 1];
@@ -88,12 +85,36 @@ void k_batch_wave(BatchArgs a) {
     if (POT) a.pot[i] = -G * v[3];
 }
 
-template <int W>
-static void launch(const BatchArgs &a, bool pot, bool acc, hipStream_t s) {
-    const unsigned nb = (unsigned)(a.nitems * NQ), bs = 64 * W;
-    if (pot && acc) k_batch_wave<true, true, W><<<nb, bs, 0, s>>>(a);
-    else if (pot) k_batch_wave<false, true, W><<<nb, bs, 0, s>>>(a);
-    else k_batch_wave<true, false, W><<<nb, bs, 0, s>>>(a);
+// PERSISTENT: nb_batch_tuning.blocks workgroups go through the quarters, of eight
+// waves each (64 clusters of 200 to 3000 bodies on 8 / 64 / 512 workgroups:
+// 3.72 / 0.50 / 0.115 ms a force, by four waves 4.88 / 0.66 / 0.137).
+template <bool ACC, bool POT, int W, bool PERSISTENT>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(ACC &&POT ? 5 : 6)))
+void k_batch_wave(BatchArgs a) {
+    __shared__ WaveStage<double> st[W];
+    __shared__ double red[PARTS][NVALUES<ACC, POT>][64];
+    if constexpr (PERSISTENT) {
+        const unsigned total = (unsigned)(a.nitems * NQ);
+        for (unsigned b = blockIdx.x; b < total; b += gridDim.x) {
+            item_quarter<ACC, POT, W>(a, b, st, red);
+            __syncthreads();   // red is read before the next quarter's sums
+        }
+    } else {
+        unsigned b = blockIdx.x;
+        if (b < gridDim.x / (ITEM_RUN * XCDS) * (ITEM_RUN * XCDS)) {
+            const unsigned slot = b / XCDS;
+            b = (slot / ITEM_RUN * XCDS + b % XCDS) * ITEM_RUN + slot % ITEM_RUN;
+        }
+        item_quarter<ACC, POT, W>(a, b, st, red);
+    }
+}
+
+template <int W, bool PERSISTENT>
+static void launch(const BatchArgs &a, bool pot, bool acc, unsigned nb, hipStream_t s) {
+    const unsigned bs = 64 * W;
+    if (pot && acc) k_batch_wave<true, true, W, PERSISTENT><<<nb, bs, 0, s>>>(a);
+    else if (pot) k_batch_wave<false, true, W, PERSISTENT><<<nb, bs, 0, s>>>(a);
+    else k_batch_wave<true, false, W, PERSISTENT><<<nb, bs, 0, s>>>(a);
 }
 
 // Four waves per 64 targets, or eight while the launch has fewer workgroups
@@ -103,14 +124,16 @@ static void launch(const BatchArgs &a, bool pot, bool acc, hipStream_t s) {
 // quarters instead of tiles).
 constexpr int64_t EIGHT_WAVES_BELOW = 3072;
 
-int launch_batch_wave(const BatchArgs &a, bool pot, bool acc, hipStream_t s) {
+int launch_batch_wave(const BatchArgs &a, int blocks, bool pot, bool acc, hipStream_t s) {
     if (a.nitems <= 0) return NB_OK;
     if (a.nitems * NQ > INT32_MAX) {
         set_error("ensemble force grid too large (%lld items)", (long long)a.nitems);
         return NB_ERR_INVALID;
     }
-    if (a.nitems * NQ < EIGHT_WAVES_BELOW) launch<2 * NW>(a, pot, acc, s);
-    else launch<NW>(a, pot, acc, s);
+    const unsigned nb = (unsigned)(a.nitems * NQ);
+    if (blocks > 0 && (unsigned)blocks < nb) launch<2 * NW, true>(a, pot, acc, (unsigned)blocks, s);
+    else if (nb < EIGHT_WAVES_BELOW) launch<2 * NW, false>(a, pot, acc, nb, s);
+    else launch<NW, false>(a, pot, acc, nb, s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         set_error("launch of k_batch_wave failed: %s", hipGetErrorString(e));

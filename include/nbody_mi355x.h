@@ -288,8 +288,8 @@ NB_API int nb_adaptive_set_steps(nb_ctx *ctx, const int64_t *endstep, const int6
 
 typedef struct nb_batch_tuning {
     int32_t targets_per_thread; /* 1, 2 or 4 (targets of a work item = 256 x this)   */
-    int32_t blocks;             /* persistent blocks of the ragged kernel (0 = 8 per CU; not used by
-                                   far_path 0 with one target per thread) */
+    int32_t blocks;             /* persistent blocks of the ragged kernel (0 = 8 per CU, or, on
+                                   far_path 0 with one target per thread, one per 64 targets) */
     int32_t steps_per_graph;    /* KDK steps per captured HIP graph (even, >= 2)     */
     int32_t sort_interval;      /* re-sort every system into Morton order every k force calls (0 = never) */
     int32_t resident;           /* 1: multi-step resident kernel when every system fits it: its

@@ -21,7 +21,6 @@
 #include <atomic>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 
 #include "nb_download.h"
@@ -136,9 +135,9 @@ int copy_direct(const DownField *f, int nf, hipStream_t s) {
 }
 
 int copy_pieces(const DownField *f, int nf, Block *b, size_t npieces, hipStream_t s) {
-    // worker t empties the pieces t, t + T, ... once `ready` has passed them
-    // (T = 1: the calling thread does)
-    const int T = npieces >= DL_SLOTS ? DL_THREADS : 1;
+    // Worker t empties the pieces t, t + DL_THREADS, ... once `ready` has passed
+    // them.  The workers start with the first piece's arrival, not before: they
+    // wait in a loop, and the device may still have a whole run ahead of it.
     std::atomic<size_t> ready{0};
     std::atomic<size_t> emptied[DL_SLOTS];   // pieces emptied from each slot
     for (auto &e : emptied) e.store(0, std::memory_order_relaxed);
@@ -151,7 +150,7 @@ int copy_pieces(const DownField *f, int nf, Block *b, size_t npieces, hipStream_
         Pieces it{f, nf};
         Piece p;
         for (size_t k = 0; it.next(p); ++k) {
-            if ((int)(k % T) != t) continue;
+            if ((int)(k % DL_THREADS) != t) continue;
             while (ready.load(std::memory_order_acquire) <= k) {
                 if (stop.load(std::memory_order_relaxed)) return;
                 std::this_thread::yield();
@@ -160,17 +159,17 @@ int copy_pieces(const DownField *f, int nf, Block *b, size_t npieces, hipStream_
         }
     };
     std::thread threads[DL_THREADS];
-    int started = 0;
-    if (T > 1) {
+    int started = 0;   // (none: the calling thread empties the pieces)
+    auto start_workers = [&] {
         try {
-            for (; started < T; ++started) threads[started] = std::thread(worker, started);
-        } catch (const std::system_error &) {
+            for (; started < DL_THREADS; ++started) threads[started] = std::thread(worker, started);
+        } catch (...) {   // no thread or no memory for one
             stop.store(true);
             for (int t = 0; t < started; ++t) threads[t].join();
-            started = -1;
+            started = 0;
+            stop.store(false);
         }
-        if (started < 0) return copy_direct(f, nf, s);
-    }
+    };
     int rc = NB_OK;
     Pieces sent{f, nf}, got{f, nf};
     Piece p;
@@ -205,7 +204,8 @@ int copy_pieces(const DownField *f, int nf, Block *b, size_t npieces, hipStream_
             rc = NB_ERR_HIP;
             break;
         }
-        if (T > 1) {
+        if (k == 0 && npieces >= DL_SLOTS) start_workers();
+        if (started > 0) {
             ready.store(k + 1, std::memory_order_release);
         } else if (got.next(p)) {
             empty(p, k);

@@ -19,11 +19,11 @@
 
 #include <algorithm>
 #include <atomic>
-#include <mutex>
 #include <new>
 #include <thread>
 
 #include "nb_download.h"
+#include "nb_idle_pool.h"
 #include "nb_internal.h"
 
 namespace nb {
@@ -38,14 +38,11 @@ struct Block {
     int dev = 0;
     char *mem = nullptr;
     hipEvent_t ev[DL_SLOTS] = {};
+    Block *next = nullptr;
 };
 
-// Idle blocks, at most DL_IDLE of them, while any context or ensemble lives.
-constexpr int DL_IDLE = 4;
-std::mutex g_mutex;
-Block *g_idle[DL_IDLE];
-int g_nidle = 0;
-int64_t g_live = 0;
+// Idle blocks while any context or ensemble lives.
+IdlePool<Block, 4> g_pool;
 
 void free_block(Block *b) {
     if (!b) return;
@@ -57,15 +54,7 @@ void free_block(Block *b) {
 
 // nullptr when the host has no pinned memory left.
 Block *take_block(int dev) {
-    {
-        std::lock_guard<std::mutex> lock(g_mutex);
-        for (int k = 0; k < g_nidle; ++k)
-            if (g_idle[k]->dev == dev) {
-                Block *b = g_idle[k];
-                g_idle[k] = g_idle[--g_nidle];
-                return b;
-            }
-    }
+    if (Block *idle = g_pool.take(dev)) return idle;
     Block *b = new (std::nothrow) Block;
     if (!b) return nullptr;
     b->dev = dev;
@@ -80,17 +69,6 @@ Block *take_block(int dev) {
         return nullptr;
     }
     return b;
-}
-
-void give_block(Block *b) {
-    {
-        std::lock_guard<std::mutex> lock(g_mutex);
-        if (g_live > 0 && g_nidle < DL_IDLE) {
-            g_idle[g_nidle++] = b;
-            return;
-        }
-    }
-    free_block(b);
 }
 
 // Coalesced stores to pinned host memory: one launch instead of a copy command.
@@ -249,27 +227,19 @@ int download_fields(const DownField *f, int nf, int dev, hipStream_t s) {
         return NB_OK;
     }
     const int rc = copy_pieces(f, nf, todo, b, npieces, s);
-    give_block(b);
+    if (!g_pool.give(b)) free_block(b);
     return rc;
 }
 
-DownloadUse::DownloadUse() {
-    std::lock_guard<std::mutex> lock(g_mutex);
-    ++g_live;
-}
+DownloadUse::DownloadUse() { g_pool.hold(); }
 
 DownloadUse::~DownloadUse() {
-    Block *idle[DL_IDLE];
-    int n = 0;
-    {
-        std::lock_guard<std::mutex> lock(g_mutex);
-        if (--g_live == 0) {
-            n = g_nidle;
-            std::copy(g_idle, g_idle + n, idle);
-            g_nidle = 0;
-        }
+    Block *b = g_pool.release();
+    while (b) {
+        Block *next = b->next;
+        free_block(b);
+        b = next;
     }
-    for (int k = 0; k < n; ++k) free_block(idle[k]);
 }
 
 }  // namespace nb

@@ -270,6 +270,17 @@ static int ensure_source_weights(nb_ctx *c) {
     return NB_OK;
 }
 
+// The central bodies' terms whose sums may be left to the step's kick: there one
+// lane per target walks them with the general FP64 pair on a quarter of the
+// waves, where k_force_f64 has the fast pair and shares a target's sources
+// between four waves, but is a launch of its own.  A step of 4097 / 16001
+// particles takes 32.7 / 126 us with 16 of them in the kick, 39.4 / 136 with 32
+// there and 36.9 / 128 with 32 apart; with 1024 372 / 505 and 80 / 168.
+constexpr int64_t CENTRAL_IN_STEP = 16;
+int64_t central_in_step(const nb_ctx *c) {
+    return c->mode == NB_MODE_SPLIT_CENTRAL && c->ncentral <= CENTRAL_IN_STEP ? c->ncentral : 0;
+}
+
 // A KDK step around run_force: the drift has written the tile boxes already
 // (boxes_ready), and the sums of the force's segments may be left to the step's
 // k_step (left reports whether they were, with nseg segments).
@@ -301,7 +312,8 @@ int run_force(nb_ctx *c, bool with_pot, bool allow_timing, bool allow_sort = tru
     const bool acc_out = !(with_pot && pot_only) || f64;
     // the step's kick takes the segments' sums (and the central bodies' terms)
     // when nothing else adds to the accelerations
-    const bool leave = fuse && !with_pot && g.nseg > 1 && c->bg.empty() && !(c->mond_acc0 > 0.0);
+    const bool leave = fuse && !with_pot && g.nseg > 1 && c->bg.empty() && !(c->mond_acc0 > 0.0) &&
+                       c->ncentral <= CENTRAL_IN_STEP;
     // few targets: the launch adds its segments' sums itself
     const bool fin = !leave && n <= OWN_SUMS_UPTO && g.nseg > 1 && (f64 ? f64_split(n, g.nseg) : (bool)g.wave_split);
     if (fin) NB_TRY(ensure_arrived(c));
@@ -878,7 +890,7 @@ static int step_args(nb_ctx *c, int64_t k, double dt, StepArgs &a, int *geo_read
     a.vx = c->vx; a.vy = c->vy; a.vz = c->vz; a.m = c->m; a.h = c->h;
     a.ax = c->ax; a.ay = c->ay; a.az = c->az;
     a.time = c->time; a.box = c->tile_box; a.sub = c->sub_box;
-    if (c->mode == NB_MODE_SPLIT_CENTRAL && c->ncentral > 0) {
+    if (central_in_step(c) > 0) {
         a.ncentral = c->ncentral; a.cidx = c->cidx; a.central = c->central;
         a.c_in = c->cstep + (k & 1) * 4 * c->ncentral;
     }
@@ -955,7 +967,7 @@ static int enqueue_steps(nb_ctx *c, int64_t k, int64_t count, double dt, bool al
 // a launch gap at every size), with nothing else that adds to the accelerations.
 static bool one_launch_steps(const nb_ctx *c) {
     if (c->n <= 0 || c->mode == NB_MODE_FP64 || !wave_path(c->tun.far_path, c->tun.targets_per_thread, false, true) ||
-        !c->bg.empty() || c->mond_acc0 > 0.0)
+        !c->bg.empty() || c->mond_acc0 > 0.0 || c->ncentral > CENTRAL_IN_STEP)
         return false;
     // (with one segment the uncaptured steps take the central bodies' terms from
     // the FP64 force kernel, whose last bits differ from the kick's)
@@ -1133,7 +1145,7 @@ int nb_set_central(nb_ctx *c, int64_t count) {
         NB_TRY(dalloc(&c->cz, sizeof(double) * count));
         NB_TRY(dalloc(&c->cm, sizeof(double) * count));
         NB_TRY(dalloc(&c->cidx, sizeof(int64_t) * count));
-        NB_TRY(dalloc(&c->cstep, sizeof(double) * 8 * count));
+        NB_TRY(dalloc(&c->cstep, sizeof(double) * 8 * std::min<int64_t>(count, CENTRAL_IN_STEP)));
     }
     NB_HIP(hipMemsetAsync(c->central, 0, (size_t)c->n, c->stream));
     NB_TRY(rebuild_central(c));

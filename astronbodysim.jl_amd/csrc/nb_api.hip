@@ -587,7 +587,7 @@ int nb_destroy(nb_ctx *c) {
     dfree(c->time); dfree(c->flag); dfree(c->central);
     dfree(c->cx); dfree(c->cy); dfree(c->cz); dfree(c->cm); dfree(c->cidx); dfree(c->cstep);
     dfree(c->ti_end); dfree(c->ti_beg);
-    dfree(c->ad.mask); dfree(c->ad.count); dfree(c->ad.idx); dfree(c->ad.cnt); dfree(c->ad.buf);
+    dfree(c->ad.mask); dfree(c->ad.count); dfree(c->ad.before); dfree(c->ad.idx); dfree(c->ad.cnt); dfree(c->ad.buf);
     if (c->ad.red) (void)hipHostFree(c->ad.red);
     sort_free(c);
     snapshot_free(c);

@@ -31,6 +31,7 @@ struct AdaptState {
     double err_tol = 0.0, min_step = 0.0, max_step = 0.0;
     uint64_t *mask = nullptr;  // active particles: one ballot per 64
     int *count = nullptr;      // and their number per 256
+    int64_t *before = nullptr; // and in the blocks before each, in large systems
     int64_t *idx = nullptr;    // compacted active indices
     int64_t *cnt = nullptr;    // [0] active count
     int64_t *red = nullptr;    // pinned host: (min, count, error flags) of each reduction block

@@ -100,7 +100,8 @@ struct BatchArgs {
 };
 
 // nb_batch_wave.hip: the FP32-pair sums of every item on far path 0 with one
-// target per lane; blocks > 0: by at most that many workgroups.
-int launch_batch_wave(const BatchArgs &a, int blocks, bool pot, bool acc, hipStream_t s);
+// target per lane; max_n: the particles of the largest system; blocks > 0: by at
+// most that many workgroups.
+int launch_batch_wave(const BatchArgs &a, int64_t max_n, int blocks, bool pot, bool acc, hipStream_t s);
 
 }  // namespace nb

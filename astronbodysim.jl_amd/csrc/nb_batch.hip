@@ -1119,7 +1119,7 @@ static int bforce(nb_batch *b, bool with_pot, bool allow_timing, bool pot_only =
             a.w = b->wsrc;
         }
         if (wave) {
-            NB_TRY(launch_batch_wave(a, b->tun.blocks, with_pot, !pot_only, s));
+            NB_TRY(launch_batch_wave(a, b->max_ns, b->tun.blocks, with_pot, !pot_only, s));
         } else {
             int nblk = b->tun.blocks > 0 ? b->tun.blocks : 8 * b->cu_count;
             nblk = (int)std::max<int64_t>(1, std::min<int64_t>(nblk, b->nitems));

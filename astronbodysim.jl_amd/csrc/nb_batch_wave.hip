@@ -9,12 +9,15 @@
 namespace nb {
 
 // Far path 0 with one target per lane (wave_force): one workgroup per quarter
-// (64 targets) of an item.  The system's source tiles are cut into PARTS parts,
-// of which each of the W waves takes PARTS / W, one after the other; a part's FP64
-// sums are its own and the parts' are added in order, so a system's bits depend
-// on the system alone, not on W, which follows from the size of the whole
-// ensemble.  The origins, classes and FP32 sums of a tile are force_block's, so
-// the results are too (but for the order of the FP64 sums).  Bound by FP32 VALU issue on large
+// (64 targets) of an item.  The system's source tiles are cut into PARTS parts, of
+// which each of the W waves takes one, or two one after the other.  A part's FP64
+// sums are its own, and the parts' are added pair by pair in order, so a system's
+// bits depend on the system alone, not on W, which follows from the size of the
+// whole ensemble.  A wave without a tile leaves at once: with one to four waves
+// of eight at work on systems of one to four tiles, the others held the places of
+// the next workgroups until the barrier (700 systems of 256 bodies 113 us a force).
+// The origins, classes and FP32 sums of a tile are force_block's, so the results
+// are too (but for the order of the FP64 sums).  Bound by FP32 VALU issue on large
 // ensembles (2.85e12 pairs/s on the 512 clusters below); the block-wide
 // persistent kernel that it replaced held a workgroup at its barriers for the
 // slowest of four waves, and a small ensemble gave it few waves with long
@@ -34,10 +37,11 @@ constexpr int PARTS = 8;   // (of one tile at least: a system of few tiles has e
 template <bool ACC, bool POT>
 constexpr int NVALUES = (ACC ? 3 : 0) + (POT ? 1 : 0);
 
-// The sums of quarter b of the items, by a whole workgroup.
-template <bool ACC, bool POT, int W>
+// The sums of quarter b of the items, by a whole workgroup.  LEAVE: its waves
+// without a part end here; else every wave returns, by way of the same barriers.
+template <bool ACC, bool POT, int W, bool LEAVE>
 __device__ __forceinline__ void item_quarter(const BatchArgs &a, unsigned b, WaveStage<double> (&st)[W],
-                                             double (&red)[PARTS][NVALUES<ACC, POT>][64]) {
+                                             double (&red)[W][NVALUES<ACC, POT>][64]) {
     constexpr int NV = NVALUES<ACC, POT>;
     constexpr int V0 = ACC ? 0 : 3;
     const int lane = threadIdx.x & 63;
@@ -55,26 +59,38 @@ __device__ __forceinline__ void item_quarter(const BatchArgs &a, unsigned b, Wav
     constexpr int MINE = PARTS / W;
     static_assert(MINE == 1 || MINE == 2, "a wave takes one part or two");
     const int g0 = wave * MINE;
-    const int64_t j0 = part(g0), j1 = g0 + MINE < PARTS ? part(g0 + MINE) : o1;
+    const int64_t j0 = part(g0), jm = part(g0 + 1), j1 = g0 + MINE < PARTS ? part(g0 + MINE) : o1;
+    unsigned busy = 0;   // the waves with a part
+#pragma unroll
+    for (int w = 0; w < W; ++w) busy |= (unsigned)(nt * w / W < nt * (w + 1) / W) << w;
     double v[4];   // ax, ay, az, pot
-    if (MINE == 2) {
+    if (LEAVE && j0 >= j1) return;   // (never the last wave, which adds up; a barrier waits for the waves that remain)
+    if (j0 < j1) {
+        wave_force<double, ACC, POT, true>(st[wave], a.x[ic], a.y[ic], a.z[ic], a.h[ic], nullptr, a.x, a.y, a.z, a.m,
+                                           a.skip_src, a.sub_box + (tb * NQ + (j0 - o0) / SB) * 8, a.tile_box, j0,
+                                           j1, v[0], v[1], v[2], v[3], a.tgeo + (tb + qt / NQ) * TG_STRIDE,
+                                           (int)(qt % NQ), MINE == 2 ? (int)((jm - j0) / SB) - 1 : -1, red[wave]);
+        if (MINE == 2 && jm > j0) {   // the pair's sum
 #pragma unroll
-        for (int q = 0; q < NV; ++q) red[g0][q][lane] = 0.0;   // (an empty first part)
+            for (int q = 0; q < NV; ++q) v[V0 + q] = red[wave][q][lane] + v[V0 + q];
+        }
+#pragma unroll
+        for (int q = 0; q < NV; ++q) red[wave][q][lane] = v[V0 + q];
     }
-    wave_force<double, ACC, POT, true>(st[wave], a.x[ic], a.y[ic], a.z[ic], a.h[ic], nullptr, a.x, a.y, a.z, a.m,
-                                       a.skip_src, a.sub_box + (tb * NQ + (j0 - o0) / SB) * 8, a.tile_box, j0, j1,
-                                       v[0], v[1], v[2], v[3], a.tgeo + (tb + qt / NQ) * TG_STRIDE, (int)(qt % NQ),
-                                       MINE == 2 ? (int)((part(g0 + 1) - j0) / SB) - 1 : -1, red[g0]);
-#pragma unroll
-    for (int q = 0; q < NV; ++q) red[g0 + MINE - 1][q][lane] = v[V0 + q];
     __syncthreads();
-    if (wave > 0) return;
+    if (wave < W - 1) return;
 #pragma unroll
-    for (int q = 0; q < NV; ++q) v[V0 + q] = red[0][q][lane];
+    for (int q = 0; q < NV; ++q) v[V0 + q] = 0.0;
 #pragma unroll
-    for (int g = 1; g < PARTS; ++g)
+    for (int g = 0; g < PARTS; g += 2) {
+        const int w = g / MINE;
 #pragma unroll
-        for (int q = 0; q < NV; ++q) v[V0 + q] += red[g][q][lane];
+        for (int q = 0; q < NV; ++q) {
+            double p = busy >> w & 1 ? red[w][q][lane] : 0.0;
+            if (MINE == 1) p += busy >> (w + 1) & 1 ? red[w + 1][q][lane] : 0.0;
+            v[V0 + q] += p;
+        }
+    }
     if (i >= o1) return;
     const double G = a.Gs[s];
     if (ACC) {
@@ -92,11 +108,11 @@ template <bool ACC, bool POT, int W, bool PERSISTENT>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(ACC &&POT ? 5 : 6)))
 void k_batch_wave(BatchArgs a) {
     __shared__ WaveStage<double> st[W];
-    __shared__ double red[PARTS][NVALUES<ACC, POT>][64];
+    __shared__ double red[W][NVALUES<ACC, POT>][64];
     if constexpr (PERSISTENT) {
         const unsigned total = (unsigned)(a.nitems * NQ);
         for (unsigned b = blockIdx.x; b < total; b += gridDim.x) {
-            item_quarter<ACC, POT, W>(a, b, st, red);
+            item_quarter<ACC, POT, W, false>(a, b, st, red);
             __syncthreads();   // red is read before the next quarter's sums
         }
     } else {
@@ -105,7 +121,7 @@ void k_batch_wave(BatchArgs a) {
             const unsigned slot = b / XCDS;
             b = (slot / ITEM_RUN * XCDS + b % XCDS) * ITEM_RUN + slot % ITEM_RUN;
         }
-        item_quarter<ACC, POT, W>(a, b, st, red);
+        item_quarter<ACC, POT, W, true>(a, b, st, red);
     }
 }
 
@@ -121,10 +137,11 @@ static void launch(const BatchArgs &a, bool pot, bool acc, unsigned nb, hipStrea
 // than this: eight / four waves took 48 / 62 us a force at 52 workgroups, 273 /
 // 302 at 776 and 459 / 479 at 2100, but 713 / 710 at 3600 and 5.66 / 5.57 ms at
 // 33000; sixteen were slower from 776 on (timed with the sources split by
-// quarters instead of tiles).
+// quarters instead of tiles).  Four also where no system has more than four tiles
+// (1 to 399 bodies in 399 systems: 38 us by four waves, 41 by eight).
 constexpr int64_t EIGHT_WAVES_BELOW = 3072;
 
-int launch_batch_wave(const BatchArgs &a, int blocks, bool pot, bool acc, hipStream_t s) {
+int launch_batch_wave(const BatchArgs &a, int64_t max_n, int blocks, bool pot, bool acc, hipStream_t s) {
     if (a.nitems <= 0) return NB_OK;
     if (a.nitems * NQ > INT32_MAX) {
         set_error("ensemble force grid too large (%lld items)", (long long)a.nitems);
@@ -132,7 +149,7 @@ int launch_batch_wave(const BatchArgs &a, int blocks, bool pot, bool acc, hipStr
     }
     const unsigned nb = (unsigned)(a.nitems * NQ);
     if (blocks > 0 && (unsigned)blocks < nb) launch<2 * NW, true>(a, pot, acc, (unsigned)blocks, s);
-    else if (nb < EIGHT_WAVES_BELOW) launch<2 * NW, false>(a, pot, acc, nb, s);
+    else if (nb < EIGHT_WAVES_BELOW && max_n > NW * BS) launch<2 * NW, false>(a, pot, acc, nb, s);
     else launch<NW, false>(a, pot, acc, nb, s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {

@@ -91,7 +91,7 @@ __device__ __forceinline__ void near_sources(scalar_ptr<T> sx, scalar_ptr<T> sy,
             x = load_four<T>(sx + jn);
             y = load_four<T>(sy + jn);
             z = load_four<T>(sz + jn);
-            m4 = *reinterpret_cast<const float4 *>(sm + jn);
+            if (CHECKED) m4 = *reinterpret_cast<const float4 *>(sm + jn);
 #pragma unroll
             for (int g = 0; g < GR; ++g) {
                 r2[g] = __builtin_fmaf(dx[g], dx[g], __builtin_fmaf(dy[g], dy[g], dz[g] * dz[g]));
@@ -99,6 +99,9 @@ __device__ __forceinline__ void near_sources(scalar_ptr<T> sx, scalar_ptr<T> sy,
                 q[g] = m[g] * ri;
                 fac[g] = q[g] * (ri * ri);
             }
+            // (requested after the last use of m where that comes first: else the compiler
+            // may copy the four to other registers on every trip, 2.5 % of 512 clusters)
+            if (!CHECKED) m4 = *reinterpret_cast<const float4 *>(sm + jn);
             if (CHECKED) {
                 const float rmin = fminf(fminf(r2[0], r2[1]), fminf(r2[2], r2[3]));
                 if (__builtin_expect(rmin < t.h2c, 0)) {

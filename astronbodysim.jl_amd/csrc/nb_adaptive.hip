@@ -526,13 +526,15 @@ int nb_adaptive_compute_force(nb_ctx *c, int64_t t_int, int64_t *nactive) {
     // path gives way to the wavefront kernel, whose segments go down to one
     // quarter: 20 targets among 60000 took 52 us in 59 blocks, 8.7 us here.
     // Above, about 16384 blocks even out the last round (4180 blocks on the 1024
-    // that fit: five rounds for four), with the target geometry stored once.
-    const int64_t nblk = (na + BS - 1) / BS;
+    // that fit: five rounds for four), with the target geometry stored once; the
+    // wavefront kernel takes them too once its waves walk whole segments (49500 /
+    // 64900 targets 0.94 / 1.47 ms in 2048 blocks, 0.83 / 1.34 in 12500 and more).
+    const int64_t nblk = (na + BS - 1) / BS, rounds = std::min<int64_t>((16384 + nblk - 1) / nblk, 64);
     int far = c->is_double || c->tun.far_path == FAR_MFMA_BF16 ? c->tun.far_path : FAR_VALU;
     if (far == FAR_MFMA_BF16 && na < (1 << 14)) far = FAR_VALU;
     const Geometry g = c->mode != NB_MODE_FP64 && wave_path(far, 1, false, true)
-                           ? wave_launch_geometry(na, n, 1, 256)
-                           : geometry(na, n, 1, std::min<int64_t>((16384 + nblk - 1) / nblk, 64));
+                           ? wave_launch_geometry(na, n, na < WAVE_SPLIT_BELOW ? 1 : rounds, 256)
+                           : geometry(na, n, 1, rounds);
     const int nseg = g.nseg;
     // (the buffer holds part_cap segments of n targets)
     NB_TRY(ctx_ensure_part(c, (int)std::max<int64_t>((na * nseg + n - 1) / n, 2)));

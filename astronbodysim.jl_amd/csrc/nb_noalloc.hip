@@ -98,9 +98,12 @@ extern "C" int nb_compute_force_noalloc(int32_t precision_mode, int64_t n, const
     const size_t seg_bytes = sizeof(double) * 4 * (size_t)n;
     const int64_t nblk = (n + BS - 1) / BS;
     // about 8k blocks to fill the 256 CUs, as many segments as the scratch holds
+    // (k_force_wave: from WAVE_SPLIT_BELOW on; in its own 2048 blocks 100000 / 200000
+    // unsorted particles took 4.43 / 17.9 ms, in these 3.82 / 15.0)
     const int64_t fit = (int64_t)((SCRATCH_BYTES - box_bytes) / seg_bytes);
     const int64_t want = std::min<int64_t>(std::min<int64_t>(std::max<int64_t>((8192 + nblk - 1) / nblk, 1), 64), fit);
-    const Geometry g = quarters ? wave_launch_geometry(n, n, 1, std::max<int64_t>(std::min<int64_t>(want, fit), 1))
+    const Geometry g = quarters ? wave_launch_geometry(n, n, n < WAVE_SPLIT_BELOW ? 1 : want,
+                                                       std::max<int64_t>(std::min<int64_t>(want, fit), 1))
                        : f64    ? f64_launch_geometry(n, n, want, std::min<int64_t>(fit, WAVE_SEGMENTS))
                                 : geometry(n, n, 1, want);
     double *box = (double *)base;

@@ -67,7 +67,10 @@ __device__ __forceinline__ typename Four<T>::vec load_four(scalar_ptr<T> p) {
 // left the scalar registers, so that their latency runs beside the rest (scalar
 // and LDS loads share a counter, hence the masses too), and one test per
 // group finds a pair inside some target's h.
-template <typename T, bool CHECKED, bool ACC, bool POT>
+// LATE: the masses are requested after their last use in the group: requested
+// earlier, they were copied to other registers on every trip of k_batch_wave's
+// unchecked loop (2.5 % of 512 clusters).
+template <typename T, bool CHECKED, bool ACC, bool POT, bool LATE>
 __device__ __forceinline__ void near_sources(scalar_ptr<T> sx, scalar_ptr<T> sy, scalar_ptr<T> sz,
                                              const float *__restrict__ sm, int cnt, T xt, T yt, T zt,
                                              const SoftF32 &t, float &ax, float &ay, float &az, float &aq) {
@@ -91,7 +94,7 @@ __device__ __forceinline__ void near_sources(scalar_ptr<T> sx, scalar_ptr<T> sy,
             x = load_four<T>(sx + jn);
             y = load_four<T>(sy + jn);
             z = load_four<T>(sz + jn);
-            if (CHECKED) m4 = *reinterpret_cast<const float4 *>(sm + jn);
+            if (!LATE) m4 = *reinterpret_cast<const float4 *>(sm + jn);
 #pragma unroll
             for (int g = 0; g < GR; ++g) {
                 r2[g] = __builtin_fmaf(dx[g], dx[g], __builtin_fmaf(dy[g], dy[g], dz[g] * dz[g]));
@@ -99,9 +102,7 @@ __device__ __forceinline__ void near_sources(scalar_ptr<T> sx, scalar_ptr<T> sy,
                 q[g] = m[g] * ri;
                 fac[g] = q[g] * (ri * ri);
             }
-            // (requested after the last use of m where that comes first: else the compiler
-            // may copy the four to other registers on every trip, 2.5 % of 512 clusters)
-            if (!CHECKED) m4 = *reinterpret_cast<const float4 *>(sm + jn);
+            if (LATE) m4 = *reinterpret_cast<const float4 *>(sm + jn);
             if (CHECKED) {
                 const float rmin = fminf(fminf(r2[0], r2[1]), fminf(r2[2], r2[3]));
                 if (__builtin_expect(rmin < t.h2c, 0)) {
@@ -264,11 +265,11 @@ __device__ __forceinline__ void wave_force(WaveStage<T> &st, T xt, T yt, T zt, d
         const uint64_t bit = 1ull << (q & 63);
         const int cnt = j1 - base < SB ? (int)(j1 - base) : SB;
         if (m_soft & bit) {
-            near_sources<T, true, ACC, POT>(as_scalar(sx + base), as_scalar(sy + base), as_scalar(sz + base), st.m,
-                                            cnt, xt, yt, zt, t, ax, ay, az, aq);
+            near_sources<T, true, ACC, POT, false>(as_scalar(sx + base), as_scalar(sy + base), as_scalar(sz + base),
+                                                   st.m, cnt, xt, yt, zt, t, ax, ay, az, aq);
         } else if (!D || (m_close & bit)) {
-            near_sources<T, false, ACC, POT>(as_scalar(sx + base), as_scalar(sy + base), as_scalar(sz + base),
-                                             st.m, cnt, xt, yt, zt, t, ax, ay, az, aq);
+            near_sources<T, false, ACC, POT, TILES>(as_scalar(sx + base), as_scalar(sy + base), as_scalar(sz + base),
+                                                    st.m, cnt, xt, yt, zt, t, ax, ay, az, aq);
         } else if constexpr (D) {
 #pragma unroll 1
             for (int j = 0; j < cnt; j += 4) {   // (past cnt: padding)

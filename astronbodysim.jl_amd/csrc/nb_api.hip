@@ -125,11 +125,12 @@ int ensure_tbg(nb_ctx *c, const Geometry &g) {
     return dalloc(&c->tbg, sizeof(unsigned) * 16 * (size_t)BS * (size_t)((c->n + BS - 1) / BS + 1));
 }
 
-// At most STEP_SEGMENTS source segments for the forces of few targets: in
-// k_force_step each is one more arrival before the last one's sums (2000
-// particles in 32 / 16 segments 17.4 / 15.3 us a step, 4096 in FP32 23.5 / 19.1,
-// from 8000 on alike), and every other launch of the same forces cuts the
-// sources alike, so that its sums have the same bits.
+// The forces of few targets are spread over at most STEP_SEGMENTS source segments
+// to fill the chip (j_segments above 4 STEP_SEGMENTS asks for more, a quarter of
+// its number): in k_force_step each is one more arrival before the last one's
+// sums (2000 particles in 32 / 16 segments 17.4 / 15.3 us a step, 4096 in FP32
+// 23.5 / 19.1, from 8000 on alike), and every other launch of the same forces
+// cuts the sources alike, so that its sums have the same bits.
 constexpr int STEP_SEGMENTS = 16;
 
 // Up to this many particles a launch adds its segments' sums itself instead of
@@ -742,10 +743,12 @@ int nb_compute_potential(nb_ctx *c, int32_t add_self_term) {
 constexpr size_t PROBE_KEEP_BYTES = (size_t)64 << 20;
 
 // Source segments of a probe launch: few points are few target blocks (1009
-// points: four), so the sources are cut until the launch has about 4096
-// blocks.  One segment left 252 of the 256 CUs idle: 1009 points in 200003
-// particles took 12.2 ms a call, 0.19 ms in 782 segments.
-// (The FP32-pair kernels: at most PROBE_SEGMENTS.)
+// points: four), so the sources are cut.  One segment left 252 of the 256 CUs
+// idle.  FP64 pairs: until the launch has about 4096 blocks of 256 points (four
+// times as many workgroups where the waves of k_force_f64 share 64): 1009 points
+// in 200003 particles 37.6 -> 0.25 ms a call, in 782 segments.  FP32 pairs: as
+// k_force_wave is filled, up to PROBE_SEGMENTS: 12.1 -> 0.14 ms in split
+// precision, 8.5 -> 0.13 in FP32.
 constexpr int PROBE_SEGMENTS = 512;
 static int probe_segments(int64_t npts, int64_t n) {
     const int64_t nblk = (npts + BS - 1) / BS;

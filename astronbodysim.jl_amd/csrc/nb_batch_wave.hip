@@ -26,12 +26,12 @@ namespace nb {
 // The items come in order of cost, so the last workgroups are the shortest, and
 // ITEM_RUN consecutive ones (quarters of one system, or of a few) run on the
 // same XCD, whose L2 then holds their sources.  Runs of 8, 16 and 32 are alike
-// (512 clusters 5.75 / 5.76 / 5.79 ms a force); 256 leave the XCDs unequal work
-// (5 % slower).
+// (within 0.7 % on 512 clusters); 256 leave the XCDs unequal work (5 % slower).
 //
-// Measured per force with its tile boxes (clusters of 256 to 16384 bodies,
-// log-uniform): 512 clusters 6.05 -> 5.76 ms, 200 2.16 -> 1.85, 64 1.21 -> 0.74,
-// 32 1.05 -> 0.48, 8 0.98 -> 0.30, one of 3271 0.223 -> 0.055 ms.
+// A force call with its tile boxes against that kernel (clusters of 256 to 16384
+// bodies, log-uniform): 512 clusters 5.47 -> 5.13 ms, 200 2.30 -> 1.96, 64
+// 1.16 -> 0.80, 32 1.05 -> 0.52, 8 0.48 -> 0.10; 700 systems of 256 bodies
+// 56 -> 42 us, 6000 of 100 239 -> 147, 399 of 1 to 399 57 -> 37.
 constexpr unsigned ITEM_RUN = 16, XCDS = 8;
 constexpr int PARTS = 8;   // (of one tile at least: a system of few tiles has empty ones)
 template <bool ACC, bool POT>
@@ -136,8 +136,8 @@ static void launch(const BatchArgs &a, bool pot, bool acc, unsigned nb, hipStrea
 // Four waves per 64 targets, or eight while the launch has fewer workgroups
 // than this: eight / four waves took 48 / 62 us a force at 52 workgroups, 273 /
 // 302 at 776 and 459 / 479 at 2100, but 713 / 710 at 3600 and 5.66 / 5.57 ms at
-// 33000; sixteen were slower from 776 on (timed with the sources split by
-// quarters instead of tiles).  Four also where no system has more than four tiles
+// 33000; sixteen were slower from 776 on (all timed in a form that split the
+// sources by quarters instead of tiles).  Four also where no system has more than four tiles
 // (1 to 399 bodies in 399 systems: 38 us by four waves, 41 by eight).
 constexpr int64_t EIGHT_WAVES_BELOW = 3072;
 

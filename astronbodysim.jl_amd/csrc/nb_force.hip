@@ -123,6 +123,10 @@ __device__ __forceinline__ void add_waves(double (&s)[NV], double (&red)[NW - 1]
 // (arrived) once its own are written; the last one leaves the count at zero.
 // (Plain stores between agent-scope fences write back and invalidate an L2 per
 // workgroup: k_force_step on 4096 particles took 175 us.)
+// The atomics are relaxed, so the language's memory model does not order the sums
+// before the count: that rests on gfx950, where an agent-scope store is
+// acknowledged (vmcnt) once it is past the L2, and an agent-scope load reads past
+// it.  The wait below is the acknowledgement of every store of the wave.
 template <int NV>
 __device__ __forceinline__ bool last_arrival(double (&s)[NV], double *part, int64_t n, int nseg, int seg, int64_t i,
                                              bool v, unsigned *arrived, double (&red)[NW - 1][NV][64], int &last) {
@@ -332,8 +336,8 @@ __global__ __launch_bounds__(BS) void k_target_geom(ForceArgs<T> a, bool hilo) {
 // test per pair (newton_f64), where the former kernel spent about 60 on sqrt
 // and divide.  A workgroup's four waves share 64 targets and take a quarter
 // of the segment's sources each (their sums meet in LDS in a fixed order), so
-// a small system still gives every SIMD a wave: 2048 particles in 8 segments
-// are 256 workgroups instead of 64.  The source index is wave-uniform, so the
+// a small system still gives every SIMD waves: 2048 particles are 32 groups of
+// targets and, in 32 segments, 1024 workgroups.  The source index is wave-uniform, so the
 // sources come through scalar loads and sit in SGPRs: no LDS staging and no
 // barrier in the loop.  Measured: 10007 particles 199 -> 92 us a launch, 2048
 // (forces and potentials) 56 -> 14 us.  Where 64-target workgroups would be too many for one

@@ -61,7 +61,10 @@ struct ForceArgs {
     uint8_t *nflag;          // [nblk_i * nseg * NW]: waves with near tiles (split passes), or nullptr
     int use_origin;          // 1: per-block FP64 origin (SPLIT), 0: absolute FP32 coordinates
     int nseg;                // source segments (grid = nblk_i * nseg)
-    int64_t seg_len;         // sources per segment (multiple of BS)
+    int64_t seg_len;         // sources per segment: a multiple of BS for the block-wide kernels, of SB (a
+                             // quarter) for k_force_wave and k_force_f64; below BS, and wherever wave_split
+                             // cuts a segment into the waves' parts, these do not start on tiles, so
+                             // k_force_wave needs sub_box there
     int nblk_i;              // target blocks
     int wave_split;          // k_force_wave: the waves of a workgroup share 64 targets and split the segment
     double G;
